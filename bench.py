@@ -161,7 +161,7 @@ def main():
     s1 = pt.stats()
     n = pt.num_tris()
     nodes4 = reachable_bvh4_nodes(pt)
-    bvh_bytes = 128 * nodes4 + 48 * n   # reachable BVH4 nodes + leaf intersection records
+    bvh_bytes = 64 * nodes4 + 64 * n   # reachable traversal nodes + leaf intersection records
     cam_rays = s1["rays_camera"] - s0["rays_camera"]
     ext_rays = s1["rays_extension"] - s0["rays_extension"]
     launches = s1["launches_trace_closest"]

@@ -1064,8 +1064,14 @@ bi_pt_status bi_pt_debug_get_bvh4(bi_pt_ctx* ctx, int32_t* child4, float* box4) 
     const uint32_t n = ctx->num_tris;
     if (n == 0) return BI_PT_OK;
     const size_t ni = n > 1 ? n - 1 : 1;
+    // the children of the traversal's nodes with their exact boxes, made from the BVH2
+    DevBuf<Bvh4Node> exact;
+    BI_TRY(dalloc(ctx, exact, ni));
+    launch_collapse_exact(ctx->nodes.p, n, exact.p, nullptr);
     std::vector<Bvh4Node> nodes(ni);
-    BI_HIP_TRY(ctx, hipMemcpy(nodes.data(), ctx->nodes4.p, ni * sizeof(Bvh4Node), hipMemcpyDeviceToHost));
+    const hipError_t e = hipMemcpy(nodes.data(), exact.p, ni * sizeof(Bvh4Node), hipMemcpyDeviceToHost);
+    dfree(ctx, exact);
+    BI_HIP_TRY(ctx, e);
     for (size_t i = 0; i < ni; ++i) {
         if (child4) std::memcpy(&child4[4 * i], nodes[i].child, 16);
         if (box4) std::memcpy(&box4[24 * i], nodes[i].lox, 96);
@@ -1165,6 +1171,8 @@ bi_pt_status bi_pt_debug_trace(bi_pt_ctx* ctx, uint32_t n, const float* rays, in
             ta.parts = kWorkParts;
             ta.refill = 32;
             ta.any_hit = ctx->non_opaque ? 1u : 0u;
+    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
+    ta.step_bound = trace_step_bound(ctx->num_tris);
             ta.hits = HitBuf{hrec.p};
             ta.error = &ctx->eng.counters.p[kCntError];
             if (status == BI_PT_OK) launch_trace_closest(ta, n, false, 16, 256, nullptr);
@@ -1226,6 +1234,8 @@ bi_pt_status bi_pt_trace_closest(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* r
     ta.parts = kWorkParts;
     ta.refill = 32;
     ta.any_hit = ctx->non_opaque ? 1u : 0u;
+    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
+    ta.step_bound = trace_step_bound(ctx->num_tris);
     ta.hits = HitBuf{ctx->rq_hits.p};
     ta.error = &ctx->eng.counters.p[kCntError];
     launch_trace_closest(ta, n, false, 16, 256, s);
@@ -1332,6 +1342,8 @@ bi_pt_status bi_pt_trace_closest_noalloc(bi_pt_ctx* ctx, uint32_t n, const bi_pt
     ta.parts = kWorkParts;
     ta.refill = 32;
     ta.any_hit = ctx->non_opaque ? 1u : 0u;
+    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
+    ta.step_bound = trace_step_bound(ctx->num_tris);
     ta.hits = HitBuf{hits};
     ta.error = &ctx->eng.counters.p[kCntError];
     launch_trace_closest(ta, n, false, 16, 256, s);

@@ -35,12 +35,7 @@ bi_pt_status engine_init(Owner* own, Engine& eng) {
     BI_TRY(dalloc(own, eng.counters, kCntSlots));
     BI_HIP_TRY(own, hipMemset(eng.counters.p, 0, kCntSlots * sizeof(uint32_t)));
     BI_TRY(dalloc(own, eng.empty_tree, 1));
-    Bvh4Node e{};
-    for (int j = 0; j < 4; ++j) {
-        e.lox[j] = e.loy[j] = e.loz[j] = e.hix[j] = e.hiy[j] = e.hiz[j] = INFINITY;
-        e.child[j] = 0;
-        e.pad[j] = 0;
-    }
+    const TravNode e{};   // every link 0: no child
     BI_HIP_TRY(own, hipMemcpy(eng.empty_tree.p, &e, sizeof e, hipMemcpyHostToDevice));
     for (auto& ev : eng.ev) BI_HIP_TRY(own, hipEventCreate(&ev));
     BI_HIP_TRY(own, hipEventCreate(&eng.plan_ev));
@@ -634,10 +629,13 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
 
         for (size_t w = 0; w < waves.size(); ++w) {
             const WaveJobs& J = wj[w];
-            uint32_t D = 0, max_nl = 0;
+            uint32_t D = 0, max_nl = 0, max_tris = 0;
+            const uint32_t one =
+                J.num_jobs == 1u && prep[waves[w][0].job].scene->num_tris <= kSmallTreeTris ? 1u : 0u;
             bool wave_cached = false, wave_rect = false;
             for (const Item& it : waves[w]) {
                 D = std::max(D, prep[it.job].D);
+                max_tris = std::max(max_tris, prep[it.job].scene->num_tris);
                 max_nl = std::max(max_nl, prep[it.job].nl);
                 wave_rect |= prep[it.job].nrect > 0;
                 wave_cached |= prep[it.job].role == kRoleCached;
@@ -670,6 +668,8 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 ta.parts = parts;
                 ta.refill = refill;
                 ta.any_hit = any_hit ? 1u : 0u;
+                ta.one = one;
+                ta.step_bound = trace_step_bound(max_tris);
                 ta.error = &cnt[kCntError];
                 BI_TRY(mark(0));
                 launch_trace_closest(ta, J.num_paths, primary, lds_stack, block, s);
@@ -733,6 +733,8 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 sha.parts = parts;
                 sha.refill = refill;
                 sha.any_hit = (any_hit || any_point) ? 1u : 0u;
+                sha.one = one;
+                sha.step_bound = ta.step_bound;
                 sha.error = &cnt[kCntError];
                 if (overlap) {   // fork: the shadow rays trace beside the next closest-hit launch
                     BI_HIP_TRY(own, hipEventRecord(eng.ev_shade, s));

@@ -354,8 +354,6 @@ __global__ __launch_bounds__(256) void k_leaves(const uint32_t* __restrict__ ord
     // alpha-tested and translucent triangles are marked for the traversal's any-hit test
     // (the instance flags force_opaque / force_non_opaque of accel.cpp:108-116, per material)
     g.v[9] = __uint_as_float(mats[tri_mat[t]].blend_mode != kBlendOpaque ? kLeafNonOpaque : 0u);
-    g.v[10] = g.v[11] = 0.0f;
-    geo[k] = g;
     LeafShade sh;
     for (int a = 0; a < 9; ++a) sh.n[a] = tri_n[9 * (size_t)t + a];
     sh.material = tri_mat[t];
@@ -366,6 +364,8 @@ __global__ __launch_bounds__(256) void k_leaves(const uint32_t* __restrict__ ord
         box[a] = sel_min(sel_min(v[a], v[3 + a]), v[6 + a]) + 0.0f;
         box[3 + a] = sel_max(sel_max(v[a], v[3 + a]), v[6 + a]) + 0.0f;
     }
+    for (int a = 0; a < 6; ++a) g.v[10 + a] = box[a];
+    geo[k] = g;
     if (n == 1) {
         for (int a = 0; a < 6; ++a) { nodes[0].box[a] = box[a]; nodes[0].box[6 + a] = box[a]; }
         return;
@@ -953,12 +953,8 @@ __global__ __launch_bounds__(64) void k_tl_climb(TreeletArgs a) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_collapse4(const BvhNode* __restrict__ nodes, int ni,
-                                                   Bvh4Node* __restrict__ out) {
-    const int k = (int)(blockIdx.x * 256u + threadIdx.x);
-    if (k >= ni) return;
-    int id[4];
-    float box[4][6];
+// The children of BVH4 node k: links id and boxes (lo xyz, hi xyz); returns how many.
+__device__ __forceinline__ int collapse4(const BvhNode* __restrict__ nodes, int k, int (&id)[4], float (&box)[4][6]) {
     int cnt = 2;
     for (int c = 0; c < 2; ++c) {
         id[c] = nodes[k].child[c];
@@ -980,6 +976,28 @@ __global__ __launch_bounds__(256) void k_collapse4(const BvhNode* __restrict__ n
         for (int a = 0; a < 6; ++a) box[pick][a] = m.box[a];
         ++cnt;
     }
+    return cnt;
+}
+
+// The traversal's nodes.
+__global__ __launch_bounds__(256) void k_collapse4(const BvhNode* __restrict__ nodes, int ni,
+                                                   TravNode* __restrict__ out) {
+    const int k = (int)(blockIdx.x * 256u + threadIdx.x);
+    if (k >= ni) return;
+    int id[4];
+    float box[4][6];
+    const int cnt = collapse4(nodes, k, id, box);
+    out[k] = trav_pack(box, id, cnt);
+}
+
+// The same nodes with exact boxes (inspection).
+__global__ __launch_bounds__(256) void k_collapse4_exact(const BvhNode* __restrict__ nodes, int ni,
+                                                         Bvh4Node* __restrict__ out) {
+    const int k = (int)(blockIdx.x * 256u + threadIdx.x);
+    if (k >= ni) return;
+    int id[4];
+    float box[4][6];
+    const int cnt = collapse4(nodes, k, id, box);
     Bvh4Node r;
     const float inf = __builtin_inff();
     for (int j = 0; j < 4; ++j) {
@@ -1039,6 +1057,11 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
         }
     }
     hipLaunchKernelGGL(k_collapse4, dim3((ni + 255) / 256), dim3(256), 0, s, a.nodes, ni, a.nodes4);
+}
+
+void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s) {
+    const int ni = n > 1 ? (int)n - 1 : 1;
+    hipLaunchKernelGGL(k_collapse4_exact, dim3((ni + 255) / 256), dim3(256), 0, s, nodes, ni, out);
 }
 
 uint32_t treelet_start_cap(uint32_t n) { return n / 6u + 1u; }

@@ -22,7 +22,6 @@
 
 namespace bipt {
 
-#define PT_HD __host__ __device__ __forceinline__
 
 struct V3 { float x, y, z; };
 PT_HD V3 v3(float x, float y, float z) { return V3{x, y, z}; }

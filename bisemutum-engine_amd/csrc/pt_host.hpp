@@ -102,7 +102,7 @@ struct Engine {
     unsigned char* plan_host = nullptr;    // pinned staging of the plan (copied asynchronously)
     size_t plan_host_n = 0;
     bool plan_pending = false;             // plan_ev marks the end of the last plan copy
-    DevBuf<Bvh4Node> empty_tree;           // one node of empty slots (jobs without triangles)
+    DevBuf<TravNode> empty_tree;           // one node of empty slots (jobs without triangles)
     hipEvent_t ev[3] = {};
     hipEvent_t plan_ev = nullptr;
     // A segment's shadow launch runs on aux_s, forked after its shading (ev_shade) and
@@ -197,7 +197,7 @@ struct bi_pt_ctx : bipt::Owner {
     bipt::DevBuf<float> tri_v, tri_n, cb_out;
     bipt::DevBuf<uint32_t> tri_mat, cb_ord, keys0, keys1, vals0, vals1, hist, refit_cnt;
     bipt::DevBuf<bipt::BvhNode> nodes;
-    bipt::DevBuf<bipt::Bvh4Node> nodes4;
+    bipt::DevBuf<bipt::TravNode> nodes4;
     bipt::DevBuf<int32_t> parent;
     bipt::DevBuf<bipt::LeafGeo> leaf_geo;
     bipt::DevBuf<bipt::LeafShade> leaf_shade;

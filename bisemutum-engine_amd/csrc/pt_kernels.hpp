@@ -37,7 +37,7 @@ struct BuildArgs {
     uint32_t* vals[2];
     uint32_t* hist;
     BvhNode* nodes;
-    Bvh4Node* nodes4;
+    TravNode* nodes4;
     int32_t* parent;
     uint32_t* refit_cnt;
     LeafGeo* leaf_geo;
@@ -58,6 +58,8 @@ struct BuildArgs {
     uint32_t* tl_starts; // 1 + treelet_start_cap(num_tris) entries
 };
 void launch_build_lbvh(const BuildArgs& a, hipStream_t s);
+// BVH4 nodes with exact boxes of a built BVH2 (inspection): n triangles, max(n - 1, 1) nodes.
+void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s);
 uint32_t sort_hist_entries(uint32_t n);
 uint32_t treelet_start_cap(uint32_t n);
 
@@ -109,8 +111,13 @@ struct TraceArgs {
     uint32_t parts;             // queue parts (1..kWorkPartsMax)
     uint32_t refill;            // idle lanes before a refill (1..64)
     uint32_t any_hit;           // nonzero: some scene of the call has non-opaque triangles
+    uint32_t one;               // nonzero: one job whose scene has at most kSmallTreeTris triangles
+    uint32_t step_bound;        // steps without a finished ray that only corrupt links can reach (trace_step_bound)
     uint32_t* error;
 };
+// A ray enters each node of its tree at most once and then waits for its leaves' tests:
+// tris is the most triangles of a scene of the launch.
+PT_HD uint32_t trace_step_bound(uint32_t tris) { return tris + 4u; }
 // block: threads per workgroup of the persistent grid (128, 256 or 512; else 256).
 void launch_trace_closest(const TraceArgs& a, uint32_t capacity, bool primary, uint32_t lds_stack, uint32_t block,
                           hipStream_t s);
@@ -128,6 +135,8 @@ struct ShadowArgs {
     uint32_t parts;             // queue parts (1..kWorkPartsMax)
     uint32_t refill;            // idle lanes before a refill (1..64)
     uint32_t any_hit;           // nonzero: some scene of the call has non-opaque triangles or point lights
+    uint32_t one;               // nonzero: one job whose scene has at most kSmallTreeTris triangles
+    uint32_t step_bound;        // steps without a finished ray that only corrupt links can reach (trace_step_bound)
     uint32_t* error;
 };
 void launch_trace_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds_stack, uint32_t block, hipStream_t s);

@@ -7,21 +7,23 @@
 //              table, sky texels (equirect or six cube faces) + importance and guide tables
 //   per frame  world triangles (36 B) + normals (36 B) in instance order, Morton keys,
 //              sorted order, BVH2 nodes (64 B: both child boxes + child links; the build
-//              structure), BVH4 nodes (128 B, one 128-B line: four child boxes as six
-//              4-wide planes + four child links; the traversal structure, stored at the
-//              index of the BVH2 node it collapses), leaf intersection records (48 B:
-//              v0, e1, e2, a non-opaque mark), leaf shading records (48 B: n0, n1, n2,
+//              structure), BVH4 traversal nodes (64 B: four child boxes as 8-bit planes in
+//              the node's frame + four child links, pt_trav.hpp; stored at the index of the
+//              BVH2 node they collapse), leaf intersection records (64 B: v0, e1, e2, a
+//              non-opaque mark, the triangle's box), leaf shading records (48 B: n0, n1, n2,
 //              material) and, where needed, leaf texture coordinates (32 B) and tangents
 //              (48 B) in sorted leaf order
 //   per wave   SoA ray queues (o.xyz, d.xyz, path id), 16-B hit records (t, leaf, u, v),
 //              SoA path state (throughput, last BSDF pdf), per-kind radiance accumulators,
 //              SoA shadow queue (o.xyz, d.xyz, contribution.xyz, path<<3|kind)
-// Nodes are read whole by one lane (7 x 16-B loads); rays, hits and path state are
+// Nodes are read whole by one lane (4 x 16-B loads); rays, hits and path state are
 // read by consecutive lanes at consecutive addresses (coalesced).
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include "pt_trav.hpp"
 
 namespace bipt {
 
@@ -32,6 +34,8 @@ constexpr int kMaxKinds = kMaxDirLights + 3;   // miss, lights..., sky, rect lig
 // at most 3 siblings.
 constexpr int kStackMax = 192;
 constexpr uint32_t kLeafMiss = 0xffffffffu;
+// Scenes whose traversal nodes (one slot per internal node) lie within 4 GB.
+constexpr uint32_t kSmallTreeTris = 1u << 26;
 constexpr uint32_t kKindSky = 7u;
 
 struct alignas(16) BvhNode {
@@ -41,7 +45,8 @@ struct alignas(16) BvhNode {
 };
 static_assert(sizeof(BvhNode) == 64, "node record is 64 bytes");
 
-// BVH4 node: child k's box is (lox[k], loy[k], loz[k]) - (hix[k], hiy[k], hiz[k]);
+// BVH4 node with exact boxes (inspection; the traversal reads the TravNode made from the
+// same children): child k's box is (lox[k], loy[k], loz[k]) - (hix[k], hiy[k], hiz[k]);
 // child k is internal (BVH4 node index >= 0) or leaf j (stored as ~j).  An empty slot
 // has the box (+inf,+inf,+inf)-(+inf,+inf,+inf), which every slab test rejects.
 struct alignas(128) Bvh4Node {
@@ -51,8 +56,8 @@ struct alignas(128) Bvh4Node {
 };
 static_assert(sizeof(Bvh4Node) == 128, "BVH4 node record is 128 bytes");
 
-struct alignas(16) LeafGeo {
-    float v[12];       // v0.xyz, e1.xyz, e2.xyz; v[9]: flag bits (kLeafNonOpaque), then unused
+struct alignas(64) LeafGeo {
+    float v[16];       // v0.xyz, e1.xyz, e2.xyz; v[9]: flag bits (kLeafNonOpaque); box lo.xyz, hi.xyz
 };
 constexpr uint32_t kLeafNonOpaque = 1u;   // the triangle's material is alpha-tested or translucent
 struct alignas(16) LeafShade {
@@ -60,7 +65,7 @@ struct alignas(16) LeafShade {
     uint32_t material;
     uint32_t pad[2];
 };
-static_assert(sizeof(LeafGeo) == 48 && sizeof(LeafShade) == 48, "leaf records are 48 bytes");
+static_assert(sizeof(LeafGeo) == 64 && sizeof(LeafShade) == 48, "leaf records are 64 and 48 bytes");
 
 struct MaterialRec {   // = bi_pt_material
     float base_color[3];
@@ -221,7 +226,7 @@ struct SkyParams {
 };
 
 struct BvhView {
-    const Bvh4Node* nodes;
+    const TravNode* nodes;
     const LeafGeo* leaf_geo;
     uint32_t num_tris;
     // any-hit inputs of non-opaque leaves
@@ -259,7 +264,7 @@ static_assert(sizeof(NrcRecord) == 64, "cache record is 64 bytes");
 // path_base[j+1]) and the pixel slots [pix_base, pix_base + npix) of the resolve pass.
 // Kernels find a path's job by a binary search over the wave's path bases.
 struct JobRec {
-    const Bvh4Node* nodes;
+    const TravNode* nodes;
     const LeafGeo* leaf_geo;
     const LeafShade* leaf_shade;
     const MaterialRec* materials;

@@ -3,25 +3,36 @@
 // Replaces TraceRay of rt_gbuffer.hlsl:25 (closest hit, TMin 0.001, TMax
 // ray_length) and the shadow-map lookups of lights.hlsl:69-101 (exact any-hit
 // shadow rays).  Rays come from SoA queues (coalesced); the traversal structure is
-// the BVH4 collapsed from the LBVH, one 128-B node per step (7 x 16-B loads).  Short
-// stack: the top `L` entries live in LDS ([slot][lane], bank conflict free for equal
-// depths), deeper entries spill to a per-lane private array; the total depth bound
-// kStackMax covers any tree the build can produce.
+// the BVH4 collapsed from the LBVH, one 64-B node per step (4 x 16-B loads, child boxes
+// as 8-bit planes: pt_trav.hpp).  Node boxes only steer the traversal; a hit counts if the
+// exact FP32 tests of its triangle and of its triangle's own box pass.  Short stack: the
+// bottom `L` entries live in LDS ([slot][lane], bank conflict free for equal depths), deeper
+// entries in a per-lane private array; the total depth bound kStackMax covers any tree
+// the build can produce.
 //
 // Persistent lanes with dynamic ray fetch: a workgroup-resident grid of wavefronts
 // keeps lanes busy -- lanes whose rays have finished take the next ray indices from
 // per-XCD counters (one atomic per wavefront and refill, lanes ranked by a ballot), so
 // secondary rays of very different lengths do not idle the SIMD.  Each step is
-// node-centric: the four child boxes of one node are tested, hit leaves intersected,
-// the nearest hit internal child entered and the other hit internal children pushed
-// (ascending slot order).  Each lane's visiting order is a function of its own ray
-// only, the order of the CPU restatement, so hits and error flags agree bit for bit.
+// node-centric: the four child boxes of one node are tested, hit leaves queued, the
+// nearest hit internal child entered and the other hit internal children pushed
+// (ascending slot order).
+//
+// What bounds it (atrium, 16 spp at 1080p, depth 8, SQ and TCP counters): extension rays
+// issue 1.05 VALU instructions per clock and CU and look up 0.83 cache lines per clock and
+// CU in the vector cache, whose limit is one; with 128-B nodes of FP32 planes it was the
+// lookups alone (seven 16-B loads a node).  Closest hit 24.4 -> 17.5 ms, shadow 16.5 ->
+// 12.9 ms per frame from 64-B nodes (4 loads), near and far planes by the ray's signs and
+// fused multiply-adds, winners' barycentrics kept in LDS instead of a second triangle test,
+// and a step whose masks stay in scalar registers (215 -> 150 VALU instructions).
 #include "pt_kernels.hpp"
 
 namespace bipt {
 namespace {
 
-constexpr int kDone = (int)0x80000000;
+// What a lane does, in one register: the node it visits next (>= 0), or
+constexpr int kParked = -1;   // no node left: waits for its queued leaves to be tested
+constexpr int kIdle = -2;     // no ray
 constexpr uint32_t kNoRay = 0xffffffffu;
 
 __device__ __forceinline__ V3 safe_inv(V3 d) {
@@ -33,66 +44,76 @@ __device__ __forceinline__ V3 safe_inv(V3 d) {
     return v3(one(d.x), one(d.y), one(d.z));
 }
 
-struct Node4 {
-    float4 lx, ly, lz, hx, hy, hz;   // child k's box in component k
-    int4 ch;
-};
 // Node and leaf records are read through global-address-space pointers (the integer
 // round trip keeps the compiler from folding the cast away): global loads, not flat ones,
-// so the seven 16-B loads of a node issue back to back and the waits count only vector
+// so the 16-B loads of a node issue back to back and the waits count only vector
 // memory (flat loads, which might address LDS, made the compiler wait between them).
 typedef float VF4 __attribute__((ext_vector_type(4)));
-typedef float VF2 __attribute__((ext_vector_type(2)));
+typedef int VI4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const VF4 GlobalF4;
-typedef __attribute__((address_space(1))) const VF2 GlobalF2;
-__device__ __forceinline__ float4 f4(VF4 v) { return make_float4(v.x, v.y, v.z, v.w); }
-__device__ __forceinline__ Node4 load_node(const Bvh4Node* nodes, int i) {
-    const GlobalF4* p = (const GlobalF4*)(uintptr_t)(nodes + i);
-    Node4 n;
-    n.lx = f4(p[0]);
-    n.ly = f4(p[1]);
-    n.lz = f4(p[2]);
-    n.hx = f4(p[3]);
-    n.hy = f4(p[4]);
-    n.hz = f4(p[5]);
-    const VF4 c = p[6];
-    n.ch = make_int4(__float_as_int(c.x), __float_as_int(c.y), __float_as_int(c.z), __float_as_int(c.w));
-    return n;
-}
+typedef __attribute__((address_space(1))) const char GlobalChar;
 
-__device__ __forceinline__ float comp(float4 v, int k) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; }
-__device__ __forceinline__ int comp(int4 v, int k) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; }
-
-// Slab test of child k (k a compile-time constant after unrolling).  No operand can
-// be NaN ((b - o) is finite or +inf and inv is finite and nonzero), so fminf/fmaxf
-// select exactly what the CPU's comparisons select, up to the sign of zero, which
-// only ever reaches comparisons.
-__device__ __forceinline__ bool box_k(const Node4& n, int k, V3 o, V3 inv, float tmin, float tmax, float* tn_out) {
-    const float x0 = (comp(n.lx, k) - o.x) * inv.x, x1 = (comp(n.hx, k) - o.x) * inv.x;
-    const float y0 = (comp(n.ly, k) - o.y) * inv.y, y1 = (comp(n.hy, k) - o.y) * inv.y;
-    const float z0 = (comp(n.lz, k) - o.z) * inv.z, z1 = (comp(n.hz, k) - o.z) * inv.z;
-    const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), tmin));
-    const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tmax));
-    *tn_out = tn;
-    return tn <= tf * kRobust;
-}
-
-// Leaf intersection record held in registers: v0, e1, e2 and the flag word.
-struct LeafRegs {
-    float4 g0, g1;
-    float2 g2;
-};
-__device__ __forceinline__ LeafRegs load_leaf(const LeafGeo* geo, uint32_t leaf) {
-    const GlobalF4* p = (const GlobalF4*)(uintptr_t)(geo + leaf);
-    LeafRegs r;
-    r.g0 = f4(p[0]);
-    r.g1 = f4(p[1]);
-    const VF2 g2 = ((const GlobalF2*)(p + 2))[0];
-    r.g2 = make_float2(g2.x, g2.y);
+__device__ __forceinline__ TravRay trav_ray(V3 o, V3 d) {
+    const V3 inv = safe_inv(d);
+    TravRay r;
+    trav_ray_axis(r, 0, o.x, inv.x);
+    trav_ray_axis(r, 1, o.y, inv.y);
+    trav_ray_axis(r, 2, o.z, inv.z);
     return r;
 }
+__device__ __forceinline__ V3 trav_inv(const TravRay& r) { return v3(r.inv[0], r.inv[1], r.inv[2]); }
+
+// A node's record in registers.
+struct NodeRegs {
+    VF4 n0, n1, n2;
+    VI4 ch;
+};
+// SMALL: the nodes lie within 4 GB of `nodes`, which is the same for every lane (scalar
+// base, 32-bit offset).
+template <bool SMALL>
+__device__ __forceinline__ void load_node(NodeRegs& r, const TravNode* nodes, int i) {
+    GlobalChar* at = (GlobalChar*)(uintptr_t)nodes;
+    if constexpr (SMALL) at += (uint32_t)i << 6;
+    else at += (size_t)(uint32_t)i * sizeof(TravNode);
+    GlobalF4* p = (GlobalF4*)at;
+    r.n0 = p[0];
+    r.n1 = p[1];
+    r.n2 = p[2];
+    r.ch = __builtin_bit_cast(VI4, p[3]);
+}
+__device__ __forceinline__ TravPlanes node_planes(const NodeRegs& n, const TravRay& r) {
+    TravPlanes p;
+    trav_planes_axis(p, 0, r, n.n0[0], n.n0[3], __float_as_uint(n.n1[2]), __float_as_uint(n.n1[3]));
+    trav_planes_axis(p, 1, r, n.n0[1], n.n1[0], __float_as_uint(n.n2[0]), __float_as_uint(n.n2[1]));
+    trav_planes_axis(p, 2, r, n.n0[2], n.n1[1], __float_as_uint(n.n2[2]), __float_as_uint(n.n2[3]));
+    return p;
+}
+
+// Leaf intersection record held in registers: v0, e1, e2, the flag word, the low corner of
+// the box (x, y); the rest of the box is read only where the triangle is hit.
+struct LeafRegs {
+    VF4 g0, g1, g2;
+};
+__device__ __forceinline__ LeafRegs load_leaf(const LeafGeo* geo, uint32_t leaf) {
+    GlobalF4* p = (GlobalF4*)(uintptr_t)(geo + leaf);
+    return LeafRegs{p[0], p[1], p[2]};
+}
+// The exact slab test of the leaf's own box for a ray extent up to tmax, as the CPU
+// restatement computes it.  No operand can be NaN for a finite ray ((b - o) and inv are
+// finite, inv nonzero), so fminf/fmaxf select what its comparisons select, up to the sign
+// of zero, which only ever reaches comparisons.
+__device__ __forceinline__ bool box_exact(const LeafRegs& g, const LeafGeo* geo, uint32_t leaf, V3 o, V3 inv,
+                                          float tmin, float tmax) {
+    const VF4 g3 = ((GlobalF4*)(uintptr_t)(geo + leaf))[3];
+    const float x0 = (g.g2[2] - o.x) * inv.x, x1 = (g3[1] - o.x) * inv.x;
+    const float y0 = (g.g2[3] - o.y) * inv.y, y1 = (g3[2] - o.y) * inv.y;
+    const float z0 = (g3[0] - o.z) * inv.z, z1 = (g3[3] - o.z) * inv.z;
+    const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), tmin));
+    const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tmax));
+    return tn <= tf * kRobust;
+}
 __device__ __forceinline__ bool leaf_non_opaque(const LeafRegs& r) {
-    return (__float_as_uint(r.g2.y) & kLeafNonOpaque) != 0u;
+    return (__float_as_uint(r.g2[1]) & kLeafNonOpaque) != 0u;
 }
 // Any-hit test of a non-opaque leaf hit at barycentric numerators (un, vn) / det by the
 // ray (o, d) of a job: whether its surface is present for that ray.
@@ -105,9 +126,9 @@ __device__ __forceinline__ bool leaf_present(const JobRec& J, uint32_t leaf, flo
 // Moller-Trumbore with division-free barycentric acceptance; t = tn / det.
 __device__ __forceinline__ bool tri_test(const LeafRegs& g, V3 o, V3 d, float* t_out, float* un_out, float* vn_out,
                                          float* det_out) {
-    V3 v0 = v3(g.g0.x, g.g0.y, g.g0.z);
-    V3 e1 = v3(g.g0.w, g.g1.x, g.g1.y);
-    V3 e2 = v3(g.g1.z, g.g1.w, g.g2.x);
+    V3 v0 = v3(g.g0[0], g.g0[1], g.g0[2]);
+    V3 e1 = v3(g.g0[3], g.g1[0], g.g1[1]);
+    V3 e2 = v3(g.g1[2], g.g1[3], g.g2[0]);
     V3 pv = cross(d, e2);
     float det = dot(e1, pv);
     if (det == 0.0f) return false;
@@ -127,40 +148,32 @@ __device__ __forceinline__ bool tri_test(const LeafRegs& g, V3 o, V3 d, float* t
     *det_out = det;
     return true;
 }
-__device__ __forceinline__ bool tri_test(const LeafGeo* geo, uint32_t leaf, V3 o, V3 d, float* t_out, float* un_out,
-                                         float* vn_out, float* det_out) {
-    return tri_test(load_leaf(geo, leaf), o, d, t_out, un_out, vn_out, det_out);
-}
-
-// The stack depth lives in a register of the caller (`sp`), apart from the spill
-// array: an array indexed at run time is placed in private memory, and a counter
-// stored next to it would follow it there.  The spill array is touched only inside
-// branches taken when some lane of the wavefront is that deep, and its loaded value is
-// consumed inside the branch: the common path is then pure LDS, with no generic
-// (flat) access and no wait on the vector-memory counter, which would also wait for
-// the node load issued ahead of it.
+// A lane's traversal stack: the bottom L entries in its LDS column (B ints apart), deeper
+// ones in a private array.  A node step pushes at most three entries and pops one; while
+// every lane of the wavefront keeps them within the LDS part (`shallow`, one ballot per
+// step), a push is one LDS write and one addition, with no check of its own and no
+// private-memory access (whose wait would also wait for the node loads).  `top` is the
+// lane's next free entry, kept by the caller in a register, apart from the spill array (an
+// array indexed at run time is placed in private memory, and a counter beside it would
+// follow it there).
+typedef __attribute__((address_space(3))) int LdsInt;
 template <int L, int B = 256>
 struct ShortStack {
     int spill[kStackMax - L];
-    __device__ __forceinline__ bool push(int (*lds)[B], int& sp, int x) {
-        const int s = sp;
-        if (s >= kStackMax) return false;
-        if (s < L) lds[s][threadIdx.x] = x;
-        if (__ballot(s >= L) != 0ull) {
-            if (s >= L) spill[s - L] = x;
-        }
-        sp = s + 1;
+    LdsInt* bottom;
+    __device__ __forceinline__ bool shallow(LdsInt* top) const { return __ballot(top > bottom + (L - 3) * B) == 0ull; }
+    __device__ __forceinline__ bool push(LdsInt*& top, int x) {   // any depth
+        const int sp = (int)(top - bottom) / B;
+        if (sp >= kStackMax) return false;
+        if (sp < L) *top = x;
+        else spill[sp - L] = x;
+        top += B;
         return true;
     }
-    __device__ __forceinline__ int pop(int (*lds)[B], int& sp) {
-        const int s = sp - 1;
-        sp = s;
-        int v = lds[s < L ? s : L - 1][threadIdx.x];
-        if (__ballot(s >= L) != 0ull) {
-            const int w = spill[s >= L ? s - L : 0];
-            v = s >= L ? w : v;
-        }
-        return v;
+    __device__ __forceinline__ int pop(LdsInt*& top) {   // any depth
+        top -= B;
+        const int sp = (int)(top - bottom) / B;
+        return sp < L ? *top : spill[sp - L];
     }
 };
 
@@ -170,7 +183,7 @@ struct ShortStack {
 // line; a wavefront starts on the part of its workgroup's XCD (workgroups go to the
 // XCDs round-robin) and moves on to the following parts when its part runs dry, so
 // no single counter sees every refill.  Returns the new ray index for a lane that
-// asked and got one, kNoRay otherwise; sets *exhausted when every part is drained.
+// asked and got one, kNoRay otherwise; every part is drained once `left` is 0.
 struct WorkCursor {
     uint32_t part;    // part the wavefront draws from
     uint32_t left;    // parts not yet found empty
@@ -180,33 +193,26 @@ struct WorkCursor {
 __device__ __forceinline__ WorkCursor work_cursor(uint32_t count, uint32_t parts) {
     return WorkCursor{blockIdx.x % parts, parts, parts, (count + parts - 1u) / parts};
 }
-__device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bool want, bool* exhausted,
-                                              WorkCursor& wc) {
+__device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bool want, WorkCursor& wc) {
     const uint64_t m = __ballot(want);
     if (m == 0ull) return kNoRay;
-    if (wc.left == 0) {
-        if (want) *exhausted = true;
-        return kNoRay;
-    }
     const uint32_t lane = __lane_id();
     const uint32_t leader = (uint32_t)__builtin_ctzll(m);
     const uint32_t rank = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    for (;;) {
+    while (wc.left != 0u) {
         const uint32_t lo = min(wc.part * wc.chunk, count);
         const uint32_t hi = min(lo + wc.chunk, count);
         uint32_t base = 0;
         if (lane == leader) base = atomicAdd(work + wc.part * kWorkStride, (uint32_t)__popcll(m));
-        base = __shfl(base, (int)leader);
+        base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
         if (base < hi - lo) {
             const uint32_t idx = base + rank;
             return (want && idx < hi - lo) ? lo + idx : kNoRay;
         }
         wc.part = wc.part + 1u == wc.parts ? 0u : wc.part + 1u;
-        if (--wc.left == 0) {
-            if (want) *exhausted = true;
-            return kNoRay;
-        }
+        --wc.left;
     }
+    return kNoRay;
 }
 
 // Deferred leaf tests.  A box step does not intersect the leaves it reaches: it appends
@@ -225,10 +231,6 @@ __device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bo
 // prunes later box tests a little later.
 constexpr uint32_t kLeafQueue = 64u + 4u * 64u;   // < 64 before a step, which adds <= 4 per lane
 
-__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
 // Pointer held by another lane.
 template <class T>
 __device__ __forceinline__ T* shfl_ptr(T* p, int src) {
@@ -237,37 +239,97 @@ __device__ __forceinline__ T* shfl_ptr(T* p, int src) {
     return reinterpret_cast<T*>(((uint64_t)hi << 32) | lo);
 }
 
-// Appends the hit leaf children (mask lm over the slots of ch) of every lane, with their
-// box entry distances when qtn is given; returns the new queue length (uniform).
-__device__ __forceinline__ uint32_t append_leaves(uint32_t* qleaf, uint8_t* qown, float* qtn, uint32_t qn,
-                                                  uint32_t lm, int4 ch, float4 tn, uint32_t lane) {
+// Appends the leaf child `link` of the lanes marked in m, with its owner, to the
+// wavefront's queue of length qn (uniform).
+__device__ __forceinline__ void append_leaf(uint2* queue, uint32_t& qn, bool bit, int link, uint32_t lane) {
+    const uint64_t m = __ballot(bit);
+    if (bit) {
+        const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, qn));
+        queue[at] = make_uint2((uint32_t)link, lane);
+    }
+    qn += (uint32_t)__popcll(m);
+}
+
+// One step of every lane that visits a node (cur >= 0): the four child boxes are tested,
+// the hit leaves queued, the hit internal child entered nearest (NEAREST) or farthest
+// along the ray becomes the next node and the others are pushed in slot order; with none,
+// the next node comes from the stack (none left: kParked).
+//
+// The arithmetic runs for the whole wavefront (idle lanes on whatever their node registers
+// hold, their results masked), so that the masks stay in scalar registers and nothing is
+// merged at the end of a divergent region; only the loads are under the lanes' mask.
+template <bool NEAREST, bool SMALL, int L, int B>
+__device__ __forceinline__ void node_step(const TravNode* nodes, int& cur, const TravRay& ray, float tmax,
+                                          ShortStack<L, B>& st, LdsInt*& top, uint2* queue, uint32_t& qn, uint32_t lane,
+                                          uint32_t* error) {
+    const bool busy = cur >= 0;
+    NodeRegs n;
+    asm volatile("" : "=v"(n.n0), "=v"(n.n1), "=v"(n.n2), "=v"(n.ch));   // any value: masked below
+    if (busy) load_node<SMALL>(n, nodes, cur);
+    const TravPlanes p = node_planes(n, ray);
+    bool in[4], leaf[4];
+    float tn[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const bool bit = (lm >> k) & 1u;
-        const uint64_t m = __ballot(bit);
-        if (m == 0ull) continue;
-        if (bit) {
-            const uint32_t idx = qn + lanes_below(m);
-            qleaf[idx] = (uint32_t)~comp(ch, k);
-            qown[idx] = (uint8_t)lane;
-            if (qtn) qtn[idx] = comp(tn, k);
-        }
-        qn += (uint32_t)__popcll(m);
+        const bool h = busy & trav_visit(p, k, tmax, &tn[k]);
+        in[k] = h & (n.ch[k] > 0);     // an empty slot's link is 0, the root, no node's child
+        leaf[k] = h & (n.ch[k] < 0);
     }
-    return qn;
+    // the entered child: the first of the best; upd[k]: child k was the best so far
+    float tb = NEAREST ? (in[0] ? tn[0] : __builtin_inff()) : (in[0] ? tn[0] : -1.0f);
+    int next = n.ch[0];
+    bool upd[4];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+        upd[k] = in[k] & (NEAREST ? tn[k] < tb : tn[k] > tb);
+        if (k < 3) tb = upd[k] ? tn[k] : tb;
+        next = upd[k] ? n.ch[k] : next;
+    }
+    const bool none = busy & !(in[0] | in[1] | in[2] | in[3]);
+    const bool push[4] = {bool(in[0] & (upd[1] | upd[2] | upd[3])), bool(in[1] & !(upd[1] & !upd[2] & !upd[3])),
+                          bool(in[2] & !(upd[2] & !upd[3])), bool(in[3] & !upd[3])};
+    if (st.shallow(top)) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (push[k]) {
+                *top = n.ch[k];
+                top += B;
+            }
+        }
+        if (none) {
+            next = kParked;
+            if (top > st.bottom) {
+                top -= B;
+                next = *top;
+            }
+        }
+    } else {
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (ok && push[k]) ok = st.push(top, n.ch[k]);
+        if (!ok) {
+            atomicOr(error, 1u);
+            next = kParked;
+        } else if (none) {
+            next = top > st.bottom ? st.pop(top) : kParked;
+        }
+    }
+    cur = busy ? next : cur;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) append_leaf(queue, qn, leaf[k], n.ch[k], lane);
 }
 
 // AH: the call's scenes hold non-opaque (alpha-tested or translucent) triangles, whose
 // hits pass the any-hit test; without them the test and its registers are compiled out.
-// ONE: every ray of the launch belongs to job 0, so the scene pointers are uniform
-// (scalar registers) instead of per lane.
+// ONE: every ray of the launch belongs to job 0 and its nodes lie within 4 GB, so the
+// scene pointers are uniform (scalar registers) instead of per lane.
 template <bool PRIMARY, bool AH, int L, int B, bool ONE>
 __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
     __shared__ int lds[L][B];
-    __shared__ uint32_t s_qleaf[B / 64][kLeafQueue];
-    __shared__ uint8_t s_qown[B / 64][kLeafQueue];
-    __shared__ float s_qtn[B / 64][kLeafQueue];
+    __shared__ uint2 s_queue[B / 64][kLeafQueue];
     __shared__ unsigned long long s_key[B / 64][64];
+    __shared__ float2 s_uv[B / 64][64];
     const uint32_t count = PRIMARY ? a.jobs.num_paths : *a.count_in;
     const float tmin = kTMin;
     // Each lane keeps its ray's scene (BVH nodes, leaf records, triangle count): a wave
@@ -278,87 +340,49 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
     // nearest (a lane with nothing left is parked until its queued leaves are tested);
     // (2) the leaf queue is flushed when full, before a refill, or when no lane is busy,
     // and parked lanes with no queued leaves write their hit; (3) idle lanes take new
-    // rays (starting at the root) once enough of them are idle.  The node a lane visits
-    // is loaded where its boxes are tested: its 28 registers are then free during the
-    // leaf flush, which keeps the kernel at 79 VGPRs (6 wavefronts per SIMD when the LDS
-    // stack is 12 deep or less).
+    // rays (starting at the root) once enough of them are idle.  The best hit of a lane's
+    // ray sits in LDS: key (t bits, leaf), the smaller the better, and the barycentrics,
+    // written by the lane that tested the winning leaf.
     const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
-    uint32_t* qleaf = s_qleaf[w];
-    uint8_t* qown = s_qown[w];
-    float* qtn = s_qtn[w];
+    uint2* queue = s_queue[w];
     unsigned long long* key = s_key[w];
-    key[lane] = ~0ull;
+    float2* uv = s_uv[w];
     uint32_t qn = 0;
     uint32_t ray = kNoRay;
-    bool parked = false, exhausted = false;
     WorkCursor wc = work_cursor(count, a.parts);
-    V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f), inv = v3(0.f, 0.f, 0.f);
+    V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f);
+    TravRay rb = trav_ray(o, d);
     float tbest = 0.0f;
-    uint32_t best = kLeafMiss;
-    const Bvh4Node* nodes = a.jobs.rec[0].nodes;
+    const TravNode* nodes = a.jobs.rec[0].nodes;
     const LeafGeo* geo = a.jobs.rec[0].leaf_geo;
     const JobRec* jr = a.jobs.rec;   // the lane's job (materials for any-hit tests)
     ShortStack<L, B> st;
-    int sp = 0;
-    uint32_t steps_left = 0;   // node visits left before the ray is taken to loop
-    int cur_i = 0;             // the node the lane visits next
+    st.bottom = (LdsInt*)&lds[0][threadIdx.x];
+    LdsInt* top = st.bottom;
+    int cur = kIdle;
+    uint32_t dry = 0;   // steps since a ray of the wavefront finished
     for (;;) {
-        int next = kDone;
-        uint32_t lm = 0;
-        int4 ch = make_int4(0, 0, 0, 0);
-        float4 tnv = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (ray != kNoRay && !parked) {
-            const Node4 nb = load_node(nodes, cur_i);
-            ch = nb.ch;
-            float tn[4];
-            bool h[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) h[k] = box_k(nb, k, o, inv, tmin, tbest, &tn[k]);
-            tnv = make_float4(tn[0], tn[1], tn[2], tn[3]);
-            int nearest = -1, nearc = kDone;
-            float tnear = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int c = comp(ch, k);
-                if (h[k] && c < 0) lm |= 1u << k;
-                if (h[k] && c >= 0 && (nearest < 0 || tn[k] < tnear)) {
-                    nearest = k;
-                    nearc = c;
-                    tnear = tn[k];
-                }
-            }
-            bool ok = true;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int c = comp(ch, k);
-                if (ok && k != nearest && h[k] && c >= 0) ok = st.push(lds, sp, c);
-            }
-            if (!ok) atomicOr(a.error, 1u);
-            else if (nearest >= 0) next = nearc;
-            else if (sp > 0) next = st.pop(lds, sp);
-            // a ray enters each node at most once: more steps than nodes means corrupt
-            // links, and the ray is ended instead of looping
-            if (steps_left-- == 0u) {
-                atomicOr(a.error, 8u);
-                next = kDone;
-            }
-            parked = next == kDone;
+        node_step<true, ONE, L, B>(nodes, cur, rb, tbest, st, top, queue, qn, lane, a.error);
+        // a ray enters each node at most once: more steps than nodes with no ray finished
+        // means corrupt links, and the rays are ended instead of looping
+        if (++dry > a.step_bound) {
+            if (lane == 0) atomicOr(a.error, 8u);
+            if (cur >= 0) cur = kParked;
         }
-        qn = append_leaves(qleaf, qown, qtn, qn, lm, ch, tnv, lane);
-        const bool busy = ray != kNoRay && !parked;
-        const uint64_t wm = __ballot((ray == kNoRay || parked) && !exhausted);
-        const bool any_busy = __ballot(busy) != 0ull;
-        const bool refill_now = wm != 0ull && (!any_busy || (uint32_t)__popcll(wm) >= a.refill);
-        if (qn != 0u && (qn >= 64u || refill_now || !any_busy)) {
+        const uint64_t busy = __ballot(cur >= 0);
+        const bool refill_now =
+            wc.left != 0u && (busy == 0ull || 64u - (uint32_t)__popcll(busy) >= a.refill);
+        if (qn != 0u && (qn >= 64u || refill_now || busy == 0ull)) {
             __builtin_amdgcn_wave_barrier();
             for (uint32_t b = 0; b < qn; b += 64u) {
                 const uint32_t e = b + lane;
                 const bool valid = e < qn;
-                const uint32_t leaf = valid ? qleaf[e] : 0u;
-                const float tnl = valid ? qtn[e] : 0.0f;
-                const int owner = valid ? (int)qown[e] : (int)lane;
+                const uint2 q = valid ? queue[e] : make_uint2(~0u, lane);
+                const uint32_t leaf = ~q.x;
+                const int owner = (int)q.y;
                 const V3 oo = v3(__shfl(o.x, owner), __shfl(o.y, owner), __shfl(o.z, owner));
                 const V3 dd = v3(__shfl(d.x, owner), __shfl(d.y, owner), __shfl(d.z, owner));
+                const V3 oi = v3(__shfl(rb.inv[0], owner), __shfl(rb.inv[1], owner), __shfl(rb.inv[2], owner));
                 const float tb = __shfl(tbest, owner);
                 const LeafGeo* og = ONE ? geo : shfl_ptr(geo, owner);
                 // a hit counts only where the leaf's own box passes the slab test up to the
@@ -366,9 +390,10 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
                 // of the order leaves are found in), and, for a non-opaque leaf, where its
                 // surface is present for the ray (a function of the ray and the leaf alone)
                 float t = 0.0f, un = 0.0f, vn = 0.0f, det = 1.0f;
-                const LeafRegs lr = valid ? load_leaf(og, leaf) : LeafRegs{};
+                LeafRegs lr{};
+                if (valid) lr = load_leaf(og, leaf);
                 bool cand = valid && tri_test(lr, oo, dd, &t, &un, &vn, &det) && t >= tmin && t <= tb &&
-                            tnl <= t * kRobust;
+                            box_exact(lr, og, leaf, oo, oi, tmin, t);
                 if constexpr (AH) {
                     const bool nop = cand && leaf_non_opaque(lr);
                     if (__ballot(nop) != 0ull) {
@@ -376,51 +401,36 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
                         if (nop) cand = leaf_present(*oj, leaf, un, vn, det, oo, dd);
                     }
                 }
-                if (cand) atomicMin(&key[owner], ((unsigned long long)__float_as_uint(t) << 32) | leaf);
+                const unsigned long long mine = ((unsigned long long)__float_as_uint(t) << 32) | leaf;
+                if (cand) atomicMin(&key[owner], mine);
+                __builtin_amdgcn_wave_barrier();
+                if (cand && key[owner] == mine) uv[owner] = make_float2(un / det, vn / det);
             }
             __builtin_amdgcn_wave_barrier();
             qn = 0;
-            const unsigned long long kb = key[lane];
-            if (kb != ~0ull) {
-                key[lane] = ~0ull;
-                const float t = __uint_as_float((uint32_t)(kb >> 32));
-                const uint32_t leaf = (uint32_t)kb;
-                if (t < tbest || (t == tbest && leaf < best)) {
-                    tbest = t;
-                    best = leaf;
-                }
-            }
+            tbest = __uint_as_float((uint32_t)(key[lane] >> 32));
         }
-        if (parked && qn == 0u) {
-            // every leaf of the ray is tested: write the hit; u, v come from repeating
-            // the winning test
-            float u = 0.0f, v = 0.0f;
-            if (best != kLeafMiss) {
-                float t, un, vn, det;
-                tri_test(geo, best, o, d, &t, &un, &vn, &det);
-                u = un / det;
-                v = vn / det;
+        if (qn == 0u && __ballot(cur == kParked) != 0ull) {   // rays whose leaves are all tested: write the hits
+            dry = 0;
+            if (cur == kParked) {
+                const float2 buv = uv[lane];
+                a.hits.rec[ray] = HitRec{tbest, (uint32_t)key[lane], buv.x, buv.y};
+                cur = kIdle;
             }
-            a.hits.rec[ray] = HitRec{tbest, best, u, v};
-            ray = kNoRay;
-            parked = false;
         }
         uint32_t got = kNoRay;
-        if (refill_now) got = fetch_ray(a.work, count, ray == kNoRay && !exhausted, &exhausted, wc);
+        if (refill_now) got = fetch_ray(a.work, count, cur == kIdle, wc);
         const bool fresh = got != kNoRay;
-        V3 no = o, nd = d;
-        float tmax = 0.0f;
-        uint32_t setup_steps = 0;
         if (fresh) {
             // one job: its record sits at a uniform address (scalar loads); several: the
             // path's job is looked up per lane
+            float tmax = 0.0f;
             auto setup = [&](const JobRec& J, uint32_t local) {
                 if constexpr (!ONE) {
                     nodes = J.nodes;
                     geo = J.leaf_geo;
                     jr = &J;
                 }
-                setup_steps = J.num_tris > 1u ? J.num_tris : 1u;
                 tmax = J.ray_length;
                 if (PRIMARY) {
                     const PathKey k = path_key(J, local);
@@ -430,7 +440,7 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
                         jx = pcg_float(jr);
                         jy = pcg_float(jr);
                     }
-                    camera_ray(J.cam, k.pixel % J.cam.width, k.pixel / J.cam.width, jx, jy, &no, &nd);
+                    camera_ray(J.cam, k.pixel % J.cam.width, k.pixel / J.cam.width, jx, jy, &o, &d);
                 }
             };
             if (ONE || a.jobs.num_jobs == 1u) {
@@ -441,23 +451,18 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
                 setup(a.jobs.rec[jid], path - a.jobs.path_base[jid]);
             }
             if (!PRIMARY) {
-                no = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
-                nd = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
+                o = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
+                d = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
             }
-            next = 0;
-        }
-        cur_i = next != kDone ? next : 0;
-        if (fresh) {
             ray = got;
-            o = no;
-            d = nd;
-            inv = safe_inv(nd);
+            rb = trav_ray(o, d);
             tbest = tmax;
-            best = kLeafMiss;
-            sp = 0;
-            steps_left = setup_steps;
+            key[lane] = ((unsigned long long)__float_as_uint(tmax) << 32) | kLeafMiss;
+            uv[lane] = make_float2(0.0f, 0.0f);
+            top = st.bottom;
+            cur = 0;
         }
-        if (__ballot(ray != kNoRay) == 0ull && __ballot(!exhausted) == 0ull) break;
+        if (wc.left == 0u && __ballot(cur != kIdle) == 0ull) break;
     }
 }
 
@@ -480,56 +485,56 @@ template <int L>
 __device__ __forceinline__ bool occluded(const BvhView& bvh, int (*lds)[256], V3 o, V3 d, float tmin, float tmax,
                                          uint32_t* error) {
     if (bvh.num_tris == 0) return false;
-    const V3 inv = safe_inv(d);
+    const TravRay rb = trav_ray(o, d);
     ShortStack<L> st;
-    int sp = 0;
+    st.bottom = (LdsInt*)&lds[0][threadIdx.x];
+    LdsInt* top = st.bottom;
     int node = 0;
     for (uint32_t steps = 1;; ++steps) {
         if (steps > bvh.num_tris) {   // corrupt links: end the ray instead of looping
             atomicOr(error, 8u);
             return false;
         }
-        const Node4 nb = load_node(bvh.nodes, node);
-        int next = kDone;
-        bool ok = true;
-        bool h[4];
-        int far = -1;   // the shadow kernel's order: the farthest-entered hit internal child first
-        float tfar = 0.0f;
+        NodeRegs n;
+        load_node<false>(n, bvh.nodes, node);
+        const TravPlanes p = node_planes(n, rb);
+        int next = kParked;
+        bool in[4], lf[4];
+        float tfar = -1.0f;   // the shadow kernel's order: the farthest-entered hit internal child first
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             float tn;
-            h[k] = box_k(nb, k, o, inv, tmin, tmax, &tn);
-            if (h[k] && comp(nb.ch, k) >= 0 && (far < 0 || tn > tfar)) {
-                far = k;
+            const bool h = trav_visit(p, k, tmax, &tn);
+            in[k] = h && n.ch[k] > 0;
+            lf[k] = h && n.ch[k] < 0;
+            if (in[k] && tn > tfar) {
                 tfar = tn;
+                next = n.ch[k];
             }
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if (!h[k]) continue;
-            const int c = comp(nb.ch, k);
-            if (c < 0) {
-                float t, un, vn, det;
-                const uint32_t leaf = (uint32_t)~c;
-                const LeafRegs lr = load_leaf(bvh.leaf_geo, leaf);
-                if (tri_test(lr, o, d, &t, &un, &vn, &det) && t >= tmin && t <= tmax &&
-                    (!leaf_non_opaque(lr) ||
-                     surface_present(bvh.materials[bvh.leaf_shade[leaf].material], bvh.tex, bvh.leaf_uv, leaf,
-                                     un / det, vn / det, opacity_random(bvh.seed, o, d))))
-                    return true;
-            } else if (k == far) {
-                next = c;
-            } else if (ok) {
-                ok = st.push(lds, sp, c);
+            if (!lf[k]) continue;
+            float t, un, vn, det;
+            const uint32_t leaf = (uint32_t)~n.ch[k];
+            const LeafRegs lr = load_leaf(bvh.leaf_geo, leaf);
+            if (tri_test(lr, o, d, &t, &un, &vn, &det) && t >= tmin && t <= tmax &&
+                box_exact(lr, bvh.leaf_geo, leaf, o, trav_inv(rb), tmin, tmax) &&
+                (!leaf_non_opaque(lr) ||
+                 surface_present(bvh.materials[bvh.leaf_shade[leaf].material], bvh.tex, bvh.leaf_uv, leaf, un / det,
+                                 vn / det, opacity_random(bvh.seed, o, d))))
+                return true;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (in[k] && n.ch[k] != next && !st.push(top, n.ch[k])) {
+                atomicOr(error, 1u);
+                return false;
             }
         }
-        if (!ok) {
-            atomicOr(error, 1u);
-            return false;
-        }
-        if (next == kDone) {
-            if (sp == 0) return false;
-            next = st.pop(lds, sp);
+        if (next == kParked) {
+            if (top == st.bottom) return false;
+            next = st.pop(top);
         }
         node = next;
     }
@@ -566,11 +571,10 @@ __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bo
 
 // AH (the general variant): any-hit tests of non-opaque leaves and rays that end at a
 // point light; launched when a scene of the call has either.
-template <bool AH, int L, int B>
-__global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
+template <bool AH, int L, int B, bool ONE>
+__device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
     __shared__ int lds[L][B];
-    __shared__ uint32_t s_qleaf[B / 64][kLeafQueue];
-    __shared__ uint8_t s_qown[B / 64][kLeafQueue];
+    __shared__ uint2 s_queue[B / 64][kLeafQueue];
     __shared__ uint32_t s_occ[B / 64][64];
     const uint32_t count = *a.count_in;
     const float tmin = kTMin;
@@ -585,87 +589,55 @@ __global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
     // pushed in slot order (the answer is order-independent).  A flush that finds a ray
     // occluded ends it at once, busy or parked.
     const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
-    uint32_t* qleaf = s_qleaf[w];
-    uint8_t* qown = s_qown[w];
+    uint2* queue = s_queue[w];
     uint32_t* occf = s_occ[w];
     occf[lane] = 0u;
     uint32_t qn = 0;
     uint32_t ray = kNoRay;
-    bool parked = false, exhausted = false;
     WorkCursor wc = work_cursor(count, a.parts);
-    V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f), inv = v3(0.f, 0.f, 0.f);
-    const Bvh4Node* nodes = a.jobs.rec[0].nodes;   // the lane's ray's scene (see k_trace_closest)
+    V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f);
+    TravRay rb = trav_ray(o, d);
+    const TravNode* nodes = a.jobs.rec[0].nodes;   // the lane's ray's scene (see k_trace_closest)
     const LeafGeo* geo = a.jobs.rec[0].leaf_geo;
     const JobRec* jr = a.jobs.rec;
     ShortStack<L, B> st;
-    int sp = 0;
-    uint32_t steps_left = 0;   // node visits left before the ray is taken to loop
+    st.bottom = (LdsInt*)&lds[0][threadIdx.x];
+    LdsInt* top = st.bottom;
+    int cur = kIdle;
+    uint32_t dry = 0;   // steps since a ray of the wavefront finished
     uint32_t sky_rays = 0;   // ray statistics: sky shadow rays this lane finished
-    int cur_i = 0;             // the node the lane visits next
     for (;;) {
-        int next = kDone;
-        uint32_t lm = 0;
-        int4 ch = make_int4(0, 0, 0, 0);
-        if (ray != kNoRay && !parked) {
-            const Node4 nb = load_node(nodes, cur_i);
-            ch = nb.ch;
-            bool h[4];
-            int far = -1;   // the hit internal child entered farthest along the ray
-            float tfar = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float tn;
-                h[k] = box_k(nb, k, o, inv, tmin, tmax, &tn);
-                if (h[k] && comp(ch, k) >= 0 && (far < 0 || tn > tfar)) {
-                    far = k;
-                    tfar = tn;
-                }
-            }
-            bool ok = true;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int c = comp(ch, k);
-                if (!h[k]) continue;
-                if (c < 0) lm |= 1u << k;
-                else if (k == far) next = c;
-                else if (ok) ok = st.push(lds, sp, c);
-            }
-            if (!ok) {
-                atomicOr(a.error, 1u);
-                next = kDone;
-            } else if (next == kDone && sp > 0) {
-                next = st.pop(lds, sp);
-            }
-            if (steps_left-- == 0u) {   // corrupt links: end the ray instead of looping
-                atomicOr(a.error, 8u);
-                next = kDone;
-            }
-            parked = next == kDone;
+        node_step<false, ONE, L, B>(nodes, cur, rb, tmax, st, top, queue, qn, lane, a.error);
+        if (++dry > a.step_bound) {   // corrupt links (see k_trace_closest)
+            if (lane == 0) atomicOr(a.error, 8u);
+            if (cur >= 0) cur = kParked;
         }
-        qn = append_leaves(qleaf, qown, nullptr, qn, lm, ch, make_float4(0.f, 0.f, 0.f, 0.f), lane);
-        const bool busy = ray != kNoRay && !parked;
-        const uint64_t wm = __ballot((ray == kNoRay || parked) && !exhausted);
-        const bool any_busy = __ballot(busy) != 0ull;
-        const bool refill_now = wm != 0ull && (!any_busy || (uint32_t)__popcll(wm) >= a.refill);
+        const uint64_t busy = __ballot(cur >= 0);
+        const bool refill_now =
+            wc.left != 0u && (busy == 0ull || 64u - (uint32_t)__popcll(busy) >= a.refill);
         bool occ = false;
-        if (qn != 0u && (qn >= 64u || refill_now || !any_busy)) {
+        if (qn != 0u && (qn >= 64u || refill_now || busy == 0ull)) {
             __builtin_amdgcn_wave_barrier();
             for (uint32_t b = 0; b < qn; b += 64u) {
                 const uint32_t e = b + lane;
                 const bool valid = e < qn;
-                const uint32_t leaf = valid ? qleaf[e] : 0u;
-                const int owner = valid ? (int)qown[e] : (int)lane;
+                const uint2 q = valid ? queue[e] : make_uint2(~0u, lane);
+                const uint32_t leaf = ~q.x;
+                const int owner = (int)q.y;
                 const V3 oo = v3(__shfl(o.x, owner), __shfl(o.y, owner), __shfl(o.z, owner));
                 const V3 dd = v3(__shfl(d.x, owner), __shfl(d.y, owner), __shfl(d.z, owner));
-                const LeafGeo* og = shfl_ptr(geo, owner);
+                const V3 oi = v3(__shfl(rb.inv[0], owner), __shfl(rb.inv[1], owner), __shfl(rb.inv[2], owner));
+                const LeafGeo* og = ONE ? geo : shfl_ptr(geo, owner);
                 float t = 0.0f, un = 0.0f, vn = 0.0f, det = 1.0f;
-                const LeafRegs lr = valid ? load_leaf(og, leaf) : LeafRegs{};
+                LeafRegs lr{};
+                if (valid) lr = load_leaf(og, leaf);
                 const float tm = AH ? __shfl(tmax, owner) : kShadowTMax;
-                bool cand = valid && tri_test(lr, oo, dd, &t, &un, &vn, &det) && t >= tmin && t <= tm;
+                bool cand = valid && tri_test(lr, oo, dd, &t, &un, &vn, &det) && t >= tmin && t <= tm &&
+                            box_exact(lr, og, leaf, oo, oi, tmin, tm);
                 if constexpr (AH) {
                     const bool nop = cand && leaf_non_opaque(lr);
                     if (__ballot(nop) != 0ull) {
-                        const JobRec* oj = shfl_ptr(jr, owner);
+                        const JobRec* oj = ONE ? jr : shfl_ptr(jr, owner);
                         if (nop) cand = leaf_present(*oj, leaf, un, vn, det, oo, dd);
                     }
                 }
@@ -676,53 +648,49 @@ __global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
             occ = occf[lane] != 0u;
             if (occ) occf[lane] = 0u;
         }
-        if (ray != kNoRay && (occ || (parked && qn == 0u))) {
-            sky_rays += apply_shadow(a, ray, occ) ? 1u : 0u;
-            ray = kNoRay;
-            parked = false;
+        const bool done = cur != kIdle && (occ || (cur == kParked && qn == 0u));
+        if (__ballot(done) != 0ull) {
+            dry = 0;
+            if (done) {
+                sky_rays += apply_shadow(a, ray, occ) ? 1u : 0u;
+                cur = kIdle;
+            }
         }
         uint32_t got = kNoRay;
-        if (refill_now) got = fetch_ray(a.work, count, ray == kNoRay && !exhausted, &exhausted, wc);
+        if (refill_now) got = fetch_ray(a.work, count, cur == kIdle, wc);
         const bool fresh = got != kNoRay;
-        V3 no = o, nd = d;
-        uint32_t setup_steps = 0;
         if (fresh) {
             auto setup = [&](const JobRec& J) {
-                nodes = J.nodes;
-                geo = J.leaf_geo;
-                jr = &J;
-                setup_steps = J.num_tris > 1u ? J.num_tris : 1u;
+                if constexpr (!ONE) {
+                    nodes = J.nodes;
+                    geo = J.leaf_geo;
+                    jr = &J;
+                }
             };
             const uint32_t pk = a.q.pk[got];
-            const JobRec& J = a.jobs.num_jobs == 1u ? a.jobs.rec[0]
+            const JobRec& J = ONE || a.jobs.num_jobs == 1u ? a.jobs.rec[0]
                                                     : a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, pk >> 3)];
             setup(J);
-            no = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
+            o = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
             // a sky ray's direction is in the queue; a light's ray is rebuilt from the
             // light as the shading built it (without point lights, every light is
             // directional and every extent unbounded)
             const uint32_t kind = pk & 7u;
             if (kind == kKindSky) {
-                nd = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
+                d = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
                 if constexpr (AH) tmax = kShadowTMax;
             } else if constexpr (AH) {
-                light_shadow_ray(J.lights[kind], no, &nd, &tmax);
+                light_shadow_ray(J.lights[kind], o, &d, &tmax);
             } else {
                 const LightRec& Lk = J.lights[kind];
-                nd = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
+                d = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
             }
-            next = 0;
-        }
-        cur_i = next != kDone ? next : 0;
-        if (fresh) {
             ray = got;
-            o = no;
-            d = nd;
-            inv = safe_inv(nd);
-            sp = 0;
-            steps_left = setup_steps;
+            rb = trav_ray(o, d);
+            top = st.bottom;
+            cur = 0;
         }
-        if (__ballot(ray != kNoRay) == 0ull && __ballot(!exhausted) == 0ull) break;
+        if (wc.left == 0u && __ballot(cur != kIdle) == 0ull) break;
     }
     // the shade launch counted every shadow ray as a light shadow ray: move the sky
     // rays over, one atomic pair per workgroup
@@ -739,6 +707,13 @@ __global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
         }
     }
 }
+
+template <bool AH, int L, int B>
+__global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
+    trace_shadow_body<AH, L, B, false>(a);
+}
+// One job, opaque scene, the default stack and block (as k_trace_closest_one).
+__global__ __launch_bounds__(256) void k_trace_shadow_one(ShadowArgs a) { trace_shadow_body<false, 12, 256, true>(a); }
 
 template <int L>
 __global__ __launch_bounds__(256) void k_debug_anyhit(BvhView bvh, RayQueue q, uint32_t n, float tmax,
@@ -784,6 +759,15 @@ void closest_one(const TraceArgs& a, uint32_t capacity, hipStream_t s) {
     if (groups > resident) groups = resident;
     if (groups == 0) groups = 1;
     hipLaunchKernelGGL((k_trace_closest_one<P>), dim3(groups), dim3(256), 0, s, a);
+}
+
+void shadow_one(const ShadowArgs& a, uint32_t capacity, hipStream_t s) {
+    uint32_t groups = (capacity + 255u) / 256u;
+    static uint32_t resident = 0;
+    if (resident == 0) resident = resident_groups(k_trace_shadow_one, 256);
+    if (groups > resident) groups = resident;
+    if (groups == 0) groups = 1;
+    hipLaunchKernelGGL(k_trace_shadow_one, dim3(groups), dim3(256), 0, s, a);
 }
 
 template <bool AH, int L, int B>
@@ -834,7 +818,7 @@ void dispatch_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds, uint3
 void launch_trace_closest(const TraceArgs& a, uint32_t capacity, bool primary, uint32_t lds_stack, uint32_t block,
                           hipStream_t s) {
     if (capacity == 0) return;
-    if (a.jobs.num_jobs == 1u && !a.any_hit && block == 256 && lds_stack > 8 && lds_stack <= 12) {
+    if (a.one && !a.any_hit && block == 256 && lds_stack > 8 && lds_stack <= 12) {
         if (primary) closest_one<true>(a, capacity, s);
         else closest_one<false>(a, capacity, s);
         return;
@@ -856,6 +840,10 @@ void launch_debug_anyhit(const BvhView& bvh, const RayQueue& q, uint32_t n, floa
 
 void launch_trace_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds, uint32_t block, hipStream_t s) {
     if (capacity == 0) return;
+    if (a.one && !a.any_hit && block == 256 && lds > 8 && lds <= 12) {
+        shadow_one(a, capacity, s);
+        return;
+    }
     if (a.any_hit) dispatch_shadow<true>(a, capacity, lds, block, s);
     else dispatch_shadow<false>(a, capacity, lds, block, s);
 }
