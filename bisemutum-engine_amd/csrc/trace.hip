@@ -218,8 +218,8 @@ __device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bo
 // Deferred leaf tests.  A box step does not intersect the leaves it reaches: it appends
 // (leaf, owner lane) to its wavefront's queue in LDS, and the queue is flushed -- 64
 // tests at a time, one per lane, each lane testing a leaf of any owner with the
-// owner's ray fetched by a cross-lane read -- once it holds a wavefront's worth of
-// tests, before lanes take new rays, or when no lane has a node left to visit.  So the
+// owner's ray fetched by a cross-lane read -- once it holds a test for every busy lane,
+// before lanes take new rays, or when no lane has a node left to visit.  So the
 // triangle tests run with full wavefronts instead of the few lanes that reach a leaf
 // in a given step.  A closest-hit candidate is accepted only where its leaf's own box
 // passes the slab test up to the candidate's distance t.  Boxes nest and the slab
@@ -230,6 +230,15 @@ __device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bo
 // occlusion is an OR over leaves tested against a fixed extent.  A deferred hit only
 // prunes later box tests a little later.
 constexpr uint32_t kLeafQueue = 64u + 4u * 64u;   // < 64 before a step, which adds <= 4 per lane
+
+// Queue length at which a wavefront with the lanes `busy` visiting nodes tests its queued
+// leaves: one leaf per busy lane, at least 8.  A full wavefront waits for 64 tests, so that
+// they fill it; a wavefront whose rays are running out (the tail of every launch, and small
+// launches throughout) would never gather 64 and its lanes would walk on without the hits
+// that end them or shorten them.  Atrium at 1080p, 1 spp: closest hit 2.24 -> 1.95 ms and
+// shadow rays 2.15 -> 1.76 ms per frame against waiting for 64; at 16 spp 17.5 -> 17.2 and
+// 12.9 -> 12.6 ms.  1.5 or 2 leaves per busy lane: 0.5% slower; half a leaf: 3% slower.
+__device__ __forceinline__ uint32_t flush_at(uint64_t busy) { return min(64u, max(8u, (uint32_t)__popcll(busy))); }
 
 // Pointer held by another lane.
 template <class T>
@@ -338,7 +347,7 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
     // Each iteration: (1) lanes with a node to visit test its four child boxes, push the
     // hit internal children but the nearest, queue the hit leaves and move to the
     // nearest (a lane with nothing left is parked until its queued leaves are tested);
-    // (2) the leaf queue is flushed when full, before a refill, or when no lane is busy,
+    // (2) the leaf queue is flushed at flush_at, before a refill, or when no lane is busy,
     // and parked lanes with no queued leaves write their hit; (3) idle lanes take new
     // rays (starting at the root) once enough of them are idle.  The best hit of a lane's
     // ray sits in LDS: key (t bits, leaf), the smaller the better, and the barycentrics,
@@ -372,7 +381,7 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
         const uint64_t busy = __ballot(cur >= 0);
         const bool refill_now =
             wc.left != 0u && (busy == 0ull || 64u - (uint32_t)__popcll(busy) >= a.refill);
-        if (qn != 0u && (qn >= 64u || refill_now || busy == 0ull)) {
+        if (qn != 0u && (qn >= flush_at(busy) || refill_now || busy == 0ull)) {
             __builtin_amdgcn_wave_barrier();
             for (uint32_t b = 0; b < qn; b += 64u) {
                 const uint32_t e = b + lane;
@@ -582,7 +591,7 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
     // point light (the general variant only; the other has no point lights)
     float tmax = kShadowTMax;
     // Same iteration as the closest-hit kernel: box steps queue their leaves, the queue
-    // is flushed when full, before a refill or when no lane is busy, and parked lanes
+    // is flushed at flush_at, before a refill or when no lane is busy, and parked lanes
     // finish once their leaves are tested.  The hit internal child whose box the ray enters
     // farthest away is entered (occluders are found sooner there than near the ray's own
     // surface: C1 shadow rays visit 8.9 nodes instead of 11.3 in slot order) and the others
@@ -616,7 +625,7 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
         const bool refill_now =
             wc.left != 0u && (busy == 0ull || 64u - (uint32_t)__popcll(busy) >= a.refill);
         bool occ = false;
-        if (qn != 0u && (qn >= 64u || refill_now || busy == 0ull)) {
+        if (qn != 0u && (qn >= flush_at(busy) || refill_now || busy == 0ull)) {
             __builtin_amdgcn_wave_barrier();
             for (uint32_t b = 0; b < qn; b += 64u) {
                 const uint32_t e = b + lane;
