@@ -100,7 +100,7 @@ bi_pt_status ensure_build_buffers(bi_pt_ctx* ctx) {
     BI_TRY(dalloc(ctx, ctx->tri_v, (size_t)9 * n));
     BI_TRY(dalloc(ctx, ctx->tri_n, (size_t)9 * n));
     BI_TRY(dalloc(ctx, ctx->tri_mat, n));
-    BI_TRY(dalloc(ctx, ctx->cb_ord, 8));
+    BI_TRY(dalloc(ctx, ctx->cb_ord, bounds_words()));
     BI_TRY(dalloc(ctx, ctx->cb_out, 8));
     BI_TRY(dalloc(ctx, ctx->keys0, n));
     BI_TRY(dalloc(ctx, ctx->keys1, n));

@@ -31,7 +31,7 @@ struct BuildArgs {
     float* tri_v;
     float* tri_n;
     uint32_t* tri_mat;
-    uint32_t* cbounds_ord;   // 6 order-preserving uint32 (min xyz, max xyz)
+    uint32_t* cbounds_ord;   // bounds_words() words: order-preserving bounds (min xyz, max xyz)
     float* cbounds_out;      // 6 floats (may be null)
     uint32_t* keys[2];
     uint32_t* vals[2];
@@ -60,6 +60,7 @@ struct BuildArgs {
 void launch_build_lbvh(const BuildArgs& a, hipStream_t s);
 // BVH4 nodes with exact boxes of a built BVH2 (inspection): n triangles, max(n - 1, 1) nodes.
 void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s);
+uint32_t bounds_words();
 uint32_t sort_hist_entries(uint32_t n);
 uint32_t treelet_start_cap(uint32_t n);
 
