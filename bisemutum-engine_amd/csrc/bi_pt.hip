@@ -106,7 +106,7 @@ bi_pt_status ensure_build_buffers(bi_pt_ctx* ctx) {
     BI_TRY(dalloc(ctx, ctx->keys1, n));
     BI_TRY(dalloc(ctx, ctx->vals0, n));
     BI_TRY(dalloc(ctx, ctx->vals1, n));
-    BI_TRY(dalloc(ctx, ctx->hist, sort_hist_entries(n)));
+    BI_TRY(dalloc(ctx, ctx->sort_counters, sort_words(n)));
     BI_TRY(dalloc(ctx, ctx->nodes, ni));
     BI_TRY(dalloc(ctx, ctx->nodes4, ni));
     BI_TRY(dalloc(ctx, ctx->parent, ni + n));
@@ -145,7 +145,7 @@ bi_pt_status build_bvh(bi_pt_ctx* ctx, hipStream_t s, uint32_t* error, uint32_t 
     a.keys[1] = ctx->keys1.p;
     a.vals[0] = ctx->vals0.p;
     a.vals[1] = ctx->vals1.p;
-    a.hist = ctx->hist.p;
+    a.sort_counters = ctx->sort_counters.p;
     a.nodes = ctx->nodes.p;
     a.nodes4 = ctx->nodes4.p;
     a.parent = ctx->parent.p;
@@ -270,7 +270,7 @@ bi_pt_status bi_pt_destroy(bi_pt_ctx* ctx) {
     dfree(ctx, ctx->sky_row_alias); dfree(ctx, ctx->sky_tex_alias);
     dfree(ctx, ctx->tri_v); dfree(ctx, ctx->tri_n); dfree(ctx, ctx->cb_out); dfree(ctx, ctx->tri_mat);
     dfree(ctx, ctx->cb_ord); dfree(ctx, ctx->keys0); dfree(ctx, ctx->keys1); dfree(ctx, ctx->vals0);
-    dfree(ctx, ctx->vals1); dfree(ctx, ctx->hist); dfree(ctx, ctx->refit_cnt); dfree(ctx, ctx->nodes);
+    dfree(ctx, ctx->vals1); dfree(ctx, ctx->sort_counters); dfree(ctx, ctx->refit_cnt); dfree(ctx, ctx->nodes);
     dfree(ctx, ctx->nodes4); dfree(ctx, ctx->parent); dfree(ctx, ctx->leaf_geo); dfree(ctx, ctx->leaf_shade);
     dfree(ctx, ctx->tl_cost); dfree(ctx, ctx->tl_height); dfree(ctx, ctx->tl_snap); dfree(ctx, ctx->tl_starts);
     dfree(ctx, ctx->rq_job); dfree(ctx, ctx->rq_cnt); dfree(ctx, ctx->rq_path); dfree(ctx, ctx->rq_hits);

@@ -91,7 +91,8 @@ std::string device_error_text(uint32_t flags) {
     if (flags & 8u) m += " traversal step bound exceeded;";
     if (flags & 16u) m += " treelet start list overflow;";
     if (flags & 32u) m += " shade look-back wait limit;";
-    if (flags & ~(1u | 4u | 8u | 16u | 32u)) m += " flags " + std::to_string(flags) + ";";
+    if (flags & 64u) m += " sort look-back wait limit;";
+    if (flags & ~(1u | 4u | 8u | 16u | 32u | 64u)) m += " flags " + std::to_string(flags) + ";";
     return m;
 }
 

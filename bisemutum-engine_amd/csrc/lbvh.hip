@@ -6,9 +6,10 @@
 // its own; this is the build's design:
 //   1. flatten    instances -> world-space triangles (+ cofactor normals), centroid bounds
 //   2. morton     30-bit Morton code of each triangle's bounding-box centre
-//   3. sort       stable LSD radix sort of (code, triangle) with 8-bit digits:
-//                 LDS histogram -> device scan -> LDS-ranked scatter, the rank of
-//                 equal digits inside a wavefront taken from 8 ballots
+//   3. sort       stable LSD radix sort of (code, triangle) with 8-bit digits, one launch
+//                 per digit: all digits' histograms come from the Morton kernel, a tile's
+//                 place among the tiles from a look-back over their counts, and the
+//                 rank of equal digits inside a wavefront from 8 ballots
 //   4. karras     binary radix tree over the sorted codes (Karras 2012), index
 //                 tie-break for equal codes
 //   5. leaves     leaf intersection/shading records in sorted order, then the
@@ -36,9 +37,11 @@ __device__ __forceinline__ float ord2f(uint32_t o) {
 // The six order-preserving bounds (minima xyz, maxima xyz) sit on lines of their own, so
 // that their atomics do not queue behind each other.
 constexpr uint32_t kBoundStride = 32;
-__global__ void k_init_bounds(uint32_t* cb) {
-    const uint32_t t = threadIdx.x;
+// Start values of a build: bounds, and zeros for the sort's counters (`words` of them).
+__global__ __launch_bounds__(256) void k_build_init(uint32_t* cb, uint32_t* sort, uint32_t words) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t < 6) cb[t * kBoundStride] = t < 3 ? 0xffffffffu : 0u;
+    if (t < words) sort[t] = 0u;
 }
 
 __global__ __launch_bounds__(256) void k_flatten(const float* __restrict__ pos, const float* __restrict__ nrm,
@@ -162,121 +165,180 @@ __global__ __launch_bounds__(256) void k_leaf_attrs(const uint32_t* __restrict__
     if (leaf_tan) leaf_tan[k] = g;
 }
 
+// The sort: kSortPasses digits of 8 bits, lowest first.  A tile is kSortTile keys.
+constexpr uint32_t kSortPasses = 4;
+constexpr uint32_t kSortItems = 8;
+constexpr uint32_t kSortTile = 256u * kSortItems;
+// The sort's counters in one buffer (zero at the start): every digit's histogram
+// [pass][256], the tickets [pass], then the tiles' look-back words [pass][tile][256].
+constexpr uint32_t kSortTickets = kSortPasses * 256u;
+constexpr uint32_t kSortTiles = kSortTickets + 64u;
+// Look-back word: the tile's own count or its inclusive prefix, in 30 bits.
+constexpr uint32_t kTileCount = 1u << 30, kTilePrefix = 2u << 30, kTileValue = (1u << 30) - 1u;
+
+// Morton codes of a tile of triangles and the histograms of their digits: the order of the
+// keys does not matter to a digit's histogram, so all passes' are known before the first.
 __global__ __launch_bounds__(256) void k_morton(const float* __restrict__ tri_v, uint32_t n,
                                                 const uint32_t* __restrict__ cb, uint32_t* __restrict__ keys,
-                                                uint32_t* __restrict__ vals, float* __restrict__ cb_out) {
-    uint32_t t = blockIdx.x * 256u + threadIdx.x;
+                                                uint32_t* __restrict__ vals, float* __restrict__ cb_out,
+                                                uint32_t* __restrict__ hist) {
+    __shared__ uint32_t s_hist[kSortPasses][256];
+    for (uint32_t p = 0; p < kSortPasses; ++p) s_hist[p][threadIdx.x] = 0u;
+    __syncthreads();
     float cmin[3], inv_ext[3];
     for (int a = 0; a < 3; ++a) {
         cmin[a] = ord2f(cb[a * kBoundStride]);
         float e = ord2f(cb[(3 + a) * kBoundStride]) - cmin[a];
         inv_ext[a] = e > 0.0f ? 1.0f / e : 0.0f;
     }
-    if (t == 0 && cb_out) {
-        for (int a = 0; a < 6; ++a) cb_out[a] = ord2f(cb[a * kBoundStride]);
-    }
-    if (t >= n) return;
-    const float* w = tri_v + 9 * (size_t)t;
-    uint32_t q[3];
-    for (int a = 0; a < 3; ++a) {
-        float l = sel_min(sel_min(w[a], w[3 + a]), w[6 + a]);
-        float h = sel_max(sel_max(w[a], w[3 + a]), w[6 + a]);
-        float ce = (l + h) * 0.5f;
-        float f = (ce - cmin[a]) * inv_ext[a] * 1024.0f;
-        int qi = (int)f;
-        q[a] = (uint32_t)(qi < 0 ? 0 : (qi > 1023 ? 1023 : qi));
-    }
-    keys[t] = morton3(q[0], q[1], q[2]);
-    vals[t] = t;
-}
-
-constexpr uint32_t kSortThreads = 256;
-constexpr uint32_t kSortItems = 16;
-constexpr uint32_t kSortTile = kSortThreads * kSortItems;
-
-__global__ __launch_bounds__(256) void k_radix_hist(const uint32_t* __restrict__ kin, uint32_t n, uint32_t shift,
-                                                    uint32_t nblocks, uint32_t* __restrict__ hist) {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    uint32_t base = blockIdx.x * kSortTile;
+    if (blockIdx.x == 0 && threadIdx.x < 6 && cb_out) cb_out[threadIdx.x] = ord2f(cb[threadIdx.x * kBoundStride]);
+#pragma unroll
     for (uint32_t r = 0; r < kSortItems; ++r) {
-        uint32_t i = base + r * kSortThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(kin[i] >> shift) & 255u], 1u);
+        const uint32_t t = blockIdx.x * kSortTile + r * 256u + threadIdx.x;
+        if (t >= n) continue;
+        const float* w = tri_v + 9 * (size_t)t;
+        uint32_t q[3];
+        for (int a = 0; a < 3; ++a) {
+            float l = sel_min(sel_min(w[a], w[3 + a]), w[6 + a]);
+            float h = sel_max(sel_max(w[a], w[3 + a]), w[6 + a]);
+            float ce = (l + h) * 0.5f;
+            float f = (ce - cmin[a]) * inv_ext[a] * 1024.0f;
+            int qi = (int)f;
+            q[a] = (uint32_t)(qi < 0 ? 0 : (qi > 1023 ? 1023 : qi));
+        }
+        const uint32_t key = morton3(q[0], q[1], q[2]);
+        keys[t] = key;
+        vals[t] = t;
+        for (uint32_t p = 0; p < kSortPasses; ++p) atomicAdd(&s_hist[p][(key >> (8u * p)) & 255u], 1u);
     }
     __syncthreads();
-    hist[threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-// Exclusive scan of m entries in place, one workgroup of 1024 lanes.
-__global__ __launch_bounds__(1024) void k_scan_single(uint32_t* __restrict__ a, uint32_t m) {
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t carry_s;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (threadIdx.x == 0) carry_s = 0;
-    __syncthreads();
-    for (uint32_t start = 0; start < m; start += 1024u) {
-        uint32_t i = start + threadIdx.x;
-        uint32_t v = i < m ? a[i] : 0u;
-        uint32_t inc = v;
-        for (int off = 1; off < 64; off <<= 1) {
-            uint32_t y = __shfl_up(inc, off);
-            if (lane >= (uint32_t)off) inc += y;
-        }
-        if (lane == 63) wsum[wave] = inc;
-        __syncthreads();
-        uint32_t wbase = 0, total = 0;
-        for (uint32_t w = 0; w < 16; ++w) {
-            uint32_t s = wsum[w];
-            if (w < wave) wbase += s;
-            total += s;
-        }
-        uint32_t carry = carry_s;
-        if (i < m) a[i] = carry + wbase + inc - v;
-        __syncthreads();
-        if (threadIdx.x == 0) carry_s = carry + total;
-        __syncthreads();
+    for (uint32_t p = 0; p < kSortPasses; ++p) {
+        const uint32_t c = s_hist[p][threadIdx.x];
+        if (c) atomicAdd(hist + p * 256u + threadIdx.x, c);
     }
 }
 
-__global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restrict__ kin,
-                                                       const uint32_t* __restrict__ vin,
-                                                       uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                       const uint32_t* __restrict__ hist, uint32_t n,
-                                                       uint32_t nblocks, uint32_t shift) {
-    __shared__ uint32_t s_off[256];
-    __shared__ uint32_t s_wcnt[4][256];
+// Keys of digit d in the tiles before `tile`: thread d reads the tiles' words backwards,
+// eight at a time (the loads overlap), down to the nearest inclusive prefix.  A tile is
+// taken by ticket, so every lower tile has started and publishes its count without
+// waiting for anyone; the wait is bounded all the same (error flag 64, and the scatter
+// writes nothing out of range).
+constexpr uint32_t kSortSpinMax = 1u << 22;
+__device__ __forceinline__ uint32_t tile_look_back(const uint32_t* words, uint32_t tile, uint32_t d, uint32_t* error) {
+    uint32_t sum = 0, spins = 0;
+    int q = (int)tile - 1;
+    while (q >= 0) {
+        uint32_t w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            w[j] = q - j >= 0 ? __hip_atomic_load(words + (size_t)(q - j) * 256u + d, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : kTilePrefix;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (w[j] == 0u) {   // not published yet: read again from here
+                if (++spins > kSortSpinMax) {
+                    atomicOr(error, 64u);
+                    return sum;
+                }
+                __builtin_amdgcn_s_sleep(1);
+                break;
+            }
+            sum += w[j] & kTileValue;
+            if (w[j] & kTilePrefix) return sum;
+            --q;
+        }
+    }
+    return sum;
+}
+
+// One digit of the sort, one launch.  Each wavefront ranks a run of 64 * kSortItems keys,
+// 64 at a time, with its own digit counters in LDS (no workgroup barrier between the
+// rounds); the four wavefronts' counts give the tile's, which goes to the look-back.
+//
+// Latency-bound at these sizes.  Three launches per digit (histograms of 4096-key tiles, a
+// one-workgroup scan, a scatter with three barriers per 256 keys) took 155 us for 262k
+// keys, 98 us for 20k and 278 us for 800k; four of these 49, 31 and 90 us.
+__global__ __launch_bounds__(256) void k_sort_digit(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                    uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                    uint32_t n, uint32_t pass, uint32_t ntiles, uint32_t* counters,
+                                                    uint32_t* error) {
+    __shared__ uint32_t s_cnt[4][256];
+    __shared__ uint32_t s_tile;
+    __shared__ uint32_t s_wave[4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    s_off[tid] = hist[tid * nblocks + blockIdx.x];
-    for (int w = 0; w < 4; ++w) s_wcnt[w][tid] = 0;
+    if (tid == 0) s_tile = atomicAdd(counters + kSortTickets + pass, 1u);
+    for (uint32_t w = 0; w < 4; ++w) s_cnt[w][tid] = 0u;
+    // exclusive prefix of the digit's histogram: where each digit's keys start
+    const uint32_t total = counters[pass * 256u + tid];
+    uint32_t start = total;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(start, off);
+        if (lane >= (uint32_t)off) start += y;
+    }
+    if (lane == 63) s_wave[wave] = start;
     __syncthreads();
-    const uint32_t base = blockIdx.x * kSortTile;
-    const uint64_t lt = (1ull << lane) - 1ull;
+    start -= total;
+    for (uint32_t w = 0; w < wave; ++w) start += s_wave[w];
+    const uint32_t tile = s_tile, shift = 8u * pass;
+    if (tile >= ntiles) return;   // cannot happen: one ticket per workgroup
+    const uint32_t first = tile * kSortTile + wave * (64u * kSortItems) + lane;
+    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
+#pragma unroll
     for (uint32_t r = 0; r < kSortItems; ++r) {
-        uint32_t i = base + r * kSortThreads + tid;
-        bool valid = i < n;
-        uint32_t key = valid ? kin[i] : 0u;
-        uint32_t val = valid ? vin[i] : 0u;
-        uint32_t d = (key >> shift) & 255u;
+        const uint32_t i = first + r * 64u;
+        key[r] = i < n ? kin[i] : 0u;
+        val[r] = i < n ? vin[i] : 0u;
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; ++r) {
+        const bool valid = first + r * 64u < n;
+        const uint32_t d = (key[r] >> shift) & 255u;
         uint64_t m = __ballot(valid);
+#pragma unroll
         for (int b = 0; b < 8; ++b) {
-            bool bit = (d >> b) & 1u;
-            uint64_t bal = __ballot(bit);
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bal = __ballot(bit);
             m &= bit ? bal : ~bal;
         }
-        uint32_t rank = __popcll(m & lt);
-        if (valid && rank == 0) s_wcnt[wave][d] = __popcll(m);
-        __syncthreads();
-        if (valid) {
-            uint32_t dest = s_off[d] + rank;
-            for (uint32_t w = 0; w < wave; ++w) dest += s_wcnt[w][d];
-            kout[dest] = key;
-            vout[dest] = val;
+        // the wavefront's count of d before this round; its first lane with d adds the round's
+        const uint32_t before = s_cnt[wave][d];
+        const uint32_t in_round = (uint32_t)__popcll(m & below);
+        rank[r] = before + in_round;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && in_round == 0u) s_cnt[wave][d] = before + (uint32_t)__popcll(m);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // thread d: the tile's count of digit d, its place among the tiles, the wavefronts' starts
+    uint32_t c[4], count = 0;
+    for (uint32_t w = 0; w < 4; ++w) {
+        c[w] = s_cnt[w][tid];
+        count += c[w];
+    }
+    uint32_t* words = counters + kSortTiles + (size_t)pass * ntiles * 256u;
+    uint32_t* mine = words + (size_t)tile * 256u + tid;
+    uint32_t excl = 0;
+    if (tile > 0) {
+        __hip_atomic_store(mine, kTileCount | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        excl = tile_look_back(words, tile, tid, error);
+    }
+    __hip_atomic_store(mine, kTilePrefix | (excl + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t at = start + excl;
+    for (uint32_t w = 0; w < 4; ++w) {
+        s_cnt[w][tid] = at;
+        at += c[w];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kSortItems; ++r) {
+        if (first + r * 64u >= n) continue;
+        const uint32_t dest = s_cnt[wave][(key[r] >> shift) & 255u] + rank[r];
+        if (dest < n) {
+            kout[dest] = key[r];
+            vout[dest] = val[r];
         }
-        __syncthreads();
-        s_off[tid] += s_wcnt[0][tid] + s_wcnt[1][tid] + s_wcnt[2][tid] + s_wcnt[3][tid];
-        for (int w = 0; w < 4; ++w) s_wcnt[w][tid] = 0;
-        __syncthreads();
     }
 }
 
@@ -1037,23 +1099,22 @@ __global__ __launch_bounds__(256) void k_collapse4_exact(const BvhNode* __restri
 }  // namespace
 
 uint32_t bounds_words() { return 6u * kBoundStride; }
+uint32_t sort_words(uint32_t n) { return kSortTiles + kSortPasses * 256u * ((n + kSortTile - 1u) / kSortTile); }
 
 void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
     const uint32_t n = a.num_tris;
     if (n == 0) return;
     const uint32_t g256 = (n + 255) / 256;
-    hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, s, a.cbounds_ord);
+    const uint32_t tiles = (n + kSortTile - 1u) / kSortTile, words = sort_words(n);
+    hipLaunchKernelGGL(k_build_init, dim3((words + 255u) / 256u), dim3(256), 0, s, a.cbounds_ord, a.sort_counters, words);
     hipLaunchKernelGGL(k_flatten, dim3(g256), dim3(256), 0, s, a.positions, a.normals, a.indices, a.instances,
                        a.num_instances, n, a.tri_v, a.tri_n, a.tri_mat, a.cbounds_ord);
-    hipLaunchKernelGGL(k_morton, dim3(g256), dim3(256), 0, s, a.tri_v, n, a.cbounds_ord, a.keys[0], a.vals[0],
-                       a.cbounds_out);
-    const uint32_t nblocks = (n + kSortTile - 1) / kSortTile;
+    hipLaunchKernelGGL(k_morton, dim3(tiles), dim3(256), 0, s, a.tri_v, n, a.cbounds_ord, a.keys[0], a.vals[0],
+                       a.cbounds_out, a.sort_counters);
     int cur = 0;
-    for (uint32_t shift = 0; shift < 30; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(256), 0, s, a.keys[cur], n, shift, nblocks, a.hist);
-        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(1024), 0, s, a.hist, 256u * nblocks);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(256), 0, s, a.keys[cur], a.vals[cur],
-                           a.keys[cur ^ 1], a.vals[cur ^ 1], a.hist, n, nblocks, shift);
+    for (uint32_t pass = 0; pass < kSortPasses; ++pass) {
+        hipLaunchKernelGGL(k_sort_digit, dim3(tiles), dim3(256), 0, s, a.keys[cur], a.vals[cur], a.keys[cur ^ 1],
+                           a.vals[cur ^ 1], n, pass, tiles, a.sort_counters, a.error);
         cur ^= 1;
     }
     // 4 passes: the sorted keys/values end in buffer 0
@@ -1087,7 +1148,5 @@ void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipS
 }
 
 uint32_t treelet_start_cap(uint32_t n) { return n / 6u + 1u; }
-
-uint32_t sort_hist_entries(uint32_t n) { return 256u * ((n + kSortTile - 1) / kSortTile); }
 
 }  // namespace bipt

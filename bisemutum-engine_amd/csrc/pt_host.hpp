@@ -195,7 +195,7 @@ struct bi_pt_ctx : bipt::Owner {
     bool sky_set = false;
     // build buffers
     bipt::DevBuf<float> tri_v, tri_n, cb_out;
-    bipt::DevBuf<uint32_t> tri_mat, cb_ord, keys0, keys1, vals0, vals1, hist, refit_cnt;
+    bipt::DevBuf<uint32_t> tri_mat, cb_ord, keys0, keys1, vals0, vals1, sort_counters, refit_cnt;
     bipt::DevBuf<bipt::BvhNode> nodes;
     bipt::DevBuf<bipt::TravNode> nodes4;
     bipt::DevBuf<int32_t> parent;

@@ -35,7 +35,7 @@ struct BuildArgs {
     float* cbounds_out;      // 6 floats (may be null)
     uint32_t* keys[2];
     uint32_t* vals[2];
-    uint32_t* hist;
+    uint32_t* sort_counters;   // sort_words(num_tris) words
     BvhNode* nodes;
     TravNode* nodes4;
     int32_t* parent;
@@ -61,7 +61,7 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s);
 // BVH4 nodes with exact boxes of a built BVH2 (inspection): n triangles, max(n - 1, 1) nodes.
 void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s);
 uint32_t bounds_words();
-uint32_t sort_hist_entries(uint32_t n);
+uint32_t sort_words(uint32_t n);
 uint32_t treelet_start_cap(uint32_t n);
 
 // Jobs of a wave: records, path bases (num_jobs + 1 entries, the last = paths in the
