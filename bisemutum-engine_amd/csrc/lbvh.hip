@@ -342,6 +342,11 @@ __global__ __launch_bounds__(256) void k_sort_digit(const uint32_t* __restrict__
     }
 }
 
+// The refit's workgroups take kRefitBlock consecutive leaves.  An internal node whose leaves
+// all belong to one workgroup is local to it (its own index then lies among theirs).
+constexpr int kRefitBlock = 256;
+__device__ __forceinline__ bool refit_local(int first, int last) { return first / kRefitBlock == last / kRefitBlock; }
+
 __device__ __forceinline__ int kdelta(const uint32_t* __restrict__ codes, int n, int i, int j) {
     if (j < 0 || j >= n) return -1;
     uint32_t a = codes[i], b = codes[j];
@@ -386,13 +391,18 @@ __global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ cod
     int right = (max(i, j) == gamma + 1) ? ~(gamma + 1) : gamma + 1;
     nodes[i].child[0] = left;
     nodes[i].child[1] = right;
-    nodes[i].pad[0] = nodes[i].pad[1] = 0;
-    // child boxes start as NaN: the refit reads a sibling's box once it is no longer NaN
-    for (int a = 0; a < 12; ++a) nodes[i].box[a] = __uint_as_float(kBoxPending);
+    const int first = min(i, j), last = max(i, j);   // the node's leaves
+    nodes[i].pad[0] = first;
+    nodes[i].pad[1] = last;
+    // child boxes of nodes that several workgroups of the refit share start as NaN: the
+    // refit reads a sibling's box once it is no longer NaN
+    if (!refit_local(first, last)) {
+        for (int a = 0; a < 12; ++a) nodes[i].box[a] = __uint_as_float(kBoxPending);
+        refit_cnt[i] = 0;
+    }
     parent[left < 0 ? (n - 1) + ~left : left] = i;
     parent[right < 0 ? (n - 1) + ~right : right] = i;
     if (i == 0) parent[0] = -1;
-    refit_cnt[i] = 0;
     // subtree cost and height, published by the refit when the node is complete
     sub_cost[i] = __uint_as_float(kBoxPending);
     sub_height[i] = -1;
@@ -413,15 +423,66 @@ __device__ __forceinline__ float half_area_box(const float* b) {
     return (dx * dy + dy * dz) + dz * dx;
 }
 
-__global__ __launch_bounds__(256) void k_leaves(const uint32_t* __restrict__ order, const float* __restrict__ tri_v,
-                                                const float* __restrict__ tri_n,
-                                                const uint32_t* __restrict__ tri_mat,
-                                                const MaterialRec* __restrict__ mats, int n,
-                                                LeafGeo* __restrict__ geo, LeafShade* __restrict__ shade,
-                                                BvhNode* nodes, const int32_t* __restrict__ parent,
-                                                uint32_t* refit_cnt, float* sub_cost, int32_t* sub_height,
-                                                uint32_t* error) {
-    int k = blockIdx.x * 256 + threadIdx.x;
+// A subtree the refit carries upward: box, surface-area cost, height.
+struct Carried {
+    float box[6];
+    float cost;
+    int height;
+};
+// The sibling's record at a shared node: its box words, and its cost and height (a
+// triangle's follow from its box; an internal node's are published by its thread).  All
+// words are read at once and read again until none is pending.
+__device__ __forceinline__ Carried wait_sibling(const float* box, int sib, const float* sub_cost,
+                                                const int32_t* sub_height, uint32_t* error) {
+    Carried o;
+    for (uint32_t spins = 0;; ++spins) {
+        uint32_t w[6], cost = 0u;
+        int height = 0;
+        for (int a = 0; a < 6; ++a) w[a] = ld_box(box + a);
+        if (sib >= 0) {
+            cost = ld_box(sub_cost + sib);
+            height = __hip_atomic_load(sub_height + sib, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        bool pending = cost == kBoxPending || height < 0;
+        for (int a = 0; a < 6; ++a) {
+            pending = pending || w[a] == kBoxPending;
+            o.box[a] = __uint_as_float(w[a]);
+        }
+        o.cost = sib >= 0 ? __uint_as_float(cost) : half_area_box(o.box);
+        o.height = height;
+        if (!pending) return o;
+        if (spins > (1u << 20)) {
+            atomicOr(error, 4u);
+            o.height = max(o.height, 0);
+            return o;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+// Leaf records in sorted order, and the bottom-up refit: every leaf's thread climbs, the
+// second arrival at a node continues.  Nodes local to a workgroup (all but a few per
+// workgroup) meet in LDS: both children leave their box, cost and height there, the second
+// arrival writes the whole node.  The others meet in device memory by relaxed agent-scope
+// words with a NaN "pending" value.  A meeting there costs several trips past the XCDs'
+// separate L2s (about 3 us a level, and one fine-grained access per word of every node:
+// 262k triangles 131 us, 800k 303 us); with the local ones in LDS 97 and 179 us, and with a
+// sibling's words read together and the links of the next node ahead 64 and 144 us.
+__global__ __launch_bounds__(kRefitBlock) void k_leaves(const uint32_t* __restrict__ order,
+                                                        const float* __restrict__ tri_v,
+                                                        const float* __restrict__ tri_n,
+                                                        const uint32_t* __restrict__ tri_mat,
+                                                        const MaterialRec* __restrict__ mats, int n,
+                                                        LeafGeo* __restrict__ geo, LeafShade* __restrict__ shade,
+                                                        BvhNode* nodes, const int32_t* __restrict__ parent,
+                                                        uint32_t* refit_cnt, float* sub_cost, int32_t* sub_height,
+                                                        uint32_t* error) {
+    __shared__ Carried s_child[kRefitBlock][2];
+    __shared__ uint32_t s_cnt[kRefitBlock];
+    s_cnt[threadIdx.x] = 0u;
+    __syncthreads();
+    const int b0 = (int)blockIdx.x * kRefitBlock;
+    int k = b0 + (int)threadIdx.x;
     if (k >= n) return;
     uint32_t t = order[k];
     const float* w = tri_v + 9 * (size_t)t;
@@ -436,83 +497,73 @@ __global__ __launch_bounds__(256) void k_leaves(const uint32_t* __restrict__ ord
     // alpha-tested and translucent triangles are marked for the traversal's any-hit test
     // (the instance flags force_opaque / force_non_opaque of accel.cpp:108-116, per material)
     g.v[9] = __uint_as_float(mats[tri_mat[t]].blend_mode != kBlendOpaque ? kLeafNonOpaque : 0u);
+    Carried c;
+    for (int a = 0; a < 3; ++a) {
+        c.box[a] = sel_min(sel_min(v[a], v[3 + a]), v[6 + a]) + 0.0f;
+        c.box[3 + a] = sel_max(sel_max(v[a], v[3 + a]), v[6 + a]) + 0.0f;
+    }
+    for (int a = 0; a < 6; ++a) g.v[10 + a] = c.box[a];
+    geo[k] = g;
     LeafShade sh;
     for (int a = 0; a < 9; ++a) sh.n[a] = tri_n[9 * (size_t)t + a];
     sh.material = tri_mat[t];
     sh.pad[0] = sh.pad[1] = 0;
     shade[k] = sh;
-    float box[6];
-    for (int a = 0; a < 3; ++a) {
-        box[a] = sel_min(sel_min(v[a], v[3 + a]), v[6 + a]) + 0.0f;
-        box[3 + a] = sel_max(sel_max(v[a], v[3 + a]), v[6 + a]) + 0.0f;
-    }
-    for (int a = 0; a < 6; ++a) g.v[10 + a] = box[a];
-    geo[k] = g;
     if (n == 1) {
-        for (int a = 0; a < 6; ++a) { nodes[0].box[a] = box[a]; nodes[0].box[6 + a] = box[a]; }
+        for (int a = 0; a < 6; ++a) { nodes[0].box[a] = c.box[a]; nodes[0].box[6 + a] = c.box[a]; }
         return;
     }
+    // links and leaves of a node (child, child, first, last), read once, ahead of the meeting
+    auto info = [&](int node) { return *reinterpret_cast<const int4*>(nodes[node].child); };
     int p = parent[(n - 1) + k];
-    int slot = nodes[p].child[0] == ~k ? 0 : 1;
-    // surface-area cost and height of the subtree this thread carries upward (a
-    // triangle: its box's surface, height 0)
-    float cost = half_area_box(box);
-    int height = 0;
+    int4 pi = info(p);
+    int me = ~k;
+    // a triangle's cost is its box's surface, its height 0
+    c.cost = half_area_box(c.box);
+    c.height = 0;
     for (;;) {
-        for (int a = 0; a < 6; ++a) st_box(&nodes[p].box[6 * slot + a], box[a]);
-        uint32_t old = __hip_atomic_fetch_add(&refit_cnt[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (old == 0) return;   // the sibling subtree is still being built; it continues upward
-        // second arrival: the sibling has issued its box; wait until every word is visible
-        const float* ob = nodes[p].box + 6 * (1 - slot);
-        float other[6];
-        for (int a = 0; a < 6; ++a) {
-            uint32_t bits = ld_box(ob + a);
-            uint32_t spins = 0;
-            while (bits == kBoxPending) {
-                if (++spins > (1u << 20)) { atomicOr(error, 4u); bits = 0u; break; }
-                __builtin_amdgcn_s_sleep(1);
-                bits = ld_box(ob + a);
-            }
-            other[a] = __uint_as_float(bits);
+        const int q = p == 0 ? -1 : parent[p];
+        const int4 qi = info(q < 0 ? 0 : q);
+        const int slot = pi.x == me ? 0 : 1;
+        Carried o;   // the sibling's
+        if (refit_local(pi.z, pi.w)) {
+            // the record is written before the count moves, and read after it
+            const int at = p - b0;
+            s_child[at][slot] = c;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            if (atomicAdd(&s_cnt[at], 1u) == 0u) return;   // the sibling continues upward
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            o = s_child[at][1 - slot];
+            const float* b = slot == 0 ? c.box : o.box;
+            const float* b2 = slot == 0 ? o.box : c.box;
+            float4* nb = reinterpret_cast<float4*>(nodes[p].box);
+            nb[0] = make_float4(b[0], b[1], b[2], b[3]);
+            nb[1] = make_float4(b[4], b[5], b2[0], b2[1]);
+            nb[2] = make_float4(b2[2], b2[3], b2[4], b2[5]);
+        } else {
+            for (int a = 0; a < 6; ++a) st_box(&nodes[p].box[6 * slot + a], c.box[a]);
+            uint32_t old = __hip_atomic_fetch_add(&refit_cnt[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (old == 0) return;   // the sibling subtree is still being built; it continues upward
+            o = wait_sibling(nodes[p].box + 6 * (1 - slot), slot == 0 ? pi.y : pi.x, sub_cost, sub_height, error);
         }
         for (int a = 0; a < 3; ++a) {
-            box[a] = sel_min(box[a], other[a]) + 0.0f;
-            box[3 + a] = sel_max(box[3 + a], other[3 + a]) + 0.0f;
+            c.box[a] = sel_min(c.box[a], o.box[a]) + 0.0f;
+            c.box[3 + a] = sel_max(c.box[3 + a], o.box[3 + a]) + 0.0f;
         }
-        // the sibling subtree's cost and height: a triangle's from its box, an internal
-        // node's once its thread has published them
-        const int sib = nodes[p].child[1 - slot];
-        float sib_cost;
-        int sib_height;
-        if (sib < 0) {
-            sib_cost = half_area_box(other);
-            sib_height = 0;
+        const float c0 = slot == 0 ? c.cost : o.cost, c1 = slot == 0 ? o.cost : c.cost;
+        c.cost = (half_area_box(c.box) + c0) + c1;
+        c.height = 1 + max(c.height, o.height);
+        if (q < 0 || refit_local(qi.z, qi.w)) {   // nobody else reads them in this launch
+            sub_cost[p] = c.cost;
+            sub_height[p] = c.height;
         } else {
-            uint32_t bits = ld_box(sub_cost + sib);
-            uint32_t spins = 0;
-            while (bits == kBoxPending) {
-                if (++spins > (1u << 20)) { atomicOr(error, 4u); bits = 0u; break; }
-                __builtin_amdgcn_s_sleep(1);
-                bits = ld_box(sub_cost + sib);
-            }
-            sib_cost = __uint_as_float(bits);
-            sib_height = __hip_atomic_load(sub_height + sib, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            spins = 0;
-            while (sib_height < 0) {
-                if (++spins > (1u << 20)) { atomicOr(error, 4u); sib_height = 0; break; }
-                __builtin_amdgcn_s_sleep(1);
-                sib_height = __hip_atomic_load(sub_height + sib, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            st_box(sub_cost + p, c.cost);
+            __hip_atomic_store(sub_height + p, c.height, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        const float c0 = slot == 0 ? cost : sib_cost, c1 = slot == 0 ? sib_cost : cost;
-        cost = (half_area_box(box) + c0) + c1;
-        height = 1 + max(height, sib_height);
-        st_box(sub_cost + p, cost);
-        __hip_atomic_store(sub_height + p, height, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (p == 0) return;
-        int q = parent[p];
-        slot = nodes[q].child[0] == p ? 0 : 1;
+        if (q < 0) return;
+        me = p;
         p = q;
+        pi = qi;
     }
 }
 
@@ -1120,7 +1171,7 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
     // 4 passes: the sorted keys/values end in buffer 0
     hipLaunchKernelGGL(k_karras, dim3(g256), dim3(256), 0, s, a.keys[cur], (int)n, a.nodes, a.parent, a.refit_cnt,
                        a.tl_cost, a.tl_height);
-    hipLaunchKernelGGL(k_leaves, dim3(g256), dim3(256), 0, s, a.vals[cur], a.tri_v, a.tri_n, a.tri_mat,
+    hipLaunchKernelGGL(k_leaves, dim3((n + kRefitBlock - 1) / kRefitBlock), dim3(kRefitBlock), 0, s, a.vals[cur], a.tri_v, a.tri_n, a.tri_mat,
                        a.materials, (int)n, a.leaf_geo, a.leaf_shade, a.nodes, a.parent, a.refit_cnt, a.tl_cost,
                        a.tl_height, a.error);
     if (a.leaf_uv || a.leaf_tan)
