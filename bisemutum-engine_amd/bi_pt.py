@@ -613,7 +613,7 @@ class PathTracer:
         return t.cpu().numpy(), tri.cpu().numpy().view(np.uint32), u.cpu().numpy(), v.cpu().numpy()
 
     def trace_closest_noalloc(self, origins, dirs, tmax=1000.0, stream=None):
-        """trace_closest through bi_pt_trace_closest_noalloc (the library's static scratch;
+        """trace_closest through bi_pt_trace_closest_noalloc (no allocation, nothing built;
         the scene's LBVH must be current)."""
         torch = self.torch
         cols, r, dev = self._query_rays(origins, dirs)

@@ -7,7 +7,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -185,31 +184,24 @@ bi_pt_status build_bvh_now(bi_pt_ctx* ctx) {
 
 namespace {
 
-// Ray queries: the job record of the context's scene and the path bases {0, n} (one job),
-// written by a kernel so the record travels as a launch argument.
-__global__ void k_put_query_job(bipt::JobRec rec, uint32_t n, unsigned char* dst) {
-    if (threadIdx.x != 0) return;
-    *reinterpret_cast<bipt::JobRec*>(dst) = rec;
-    uint32_t* bases = reinterpret_cast<uint32_t*>(dst + sizeof(bipt::JobRec));
-    bases[0] = 0u;
-    bases[1] = n;
-    bases[2] = 0u;
-    bases[3] = 0u;
-}
-
-// Closest-hit records -> caller's arrays: t (+inf on a miss), the triangle's index in the
-// scene's instance order (leaf -> sorted order), barycentrics.
-__global__ __launch_bounds__(256) void k_query_hits(const bipt::HitRec* __restrict__ hits,
-                                                    const uint32_t* __restrict__ order, uint32_t n, float* t,
-                                                    uint32_t* tri, float* u, float* v) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    const bipt::HitRec h = hits[i];
-    const bool hit = h.leaf != bipt::kLeafMiss;
-    if (t) t[i] = hit ? h.t : __builtin_inff();
-    tri[i] = hit ? order[h.leaf] : bipt::kLeafMiss;
-    if (u) u[i] = hit ? h.u : 0.0f;
-    if (v) v[i] = hit ? h.v : 0.0f;
+// A query's launch: the context's scene and the caller's rays.  It needs no scratch (each
+// wavefront has its own range of rays), so queries of one context on several streams share
+// nothing but the scene.
+QueryArgs query_args(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* rays, float tmax) {
+    QueryArgs a{};
+    a.bvh = bvh_view(ctx);
+    if (ctx->num_tris == 0) a.bvh.nodes = ctx->eng.empty_tree.p;
+    a.q = RayQueue{const_cast<float*>(rays->ox), const_cast<float*>(rays->oy), const_cast<float*>(rays->oz),
+                   const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz), nullptr};
+    a.count = n;
+    a.tmax = tmax;
+    a.loop.parts = kWorkParts;
+    a.loop.refill = 40;
+    a.loop.any_hit = ctx->non_opaque ? 1u : 0u;
+    a.loop.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
+    a.loop.step_bound = trace_step_bound(ctx->num_tris);
+    a.loop.error = &ctx->eng.counters.p[kCntError];
+    return a;
 }
 
 // Checks a query and makes sure the context's BVH is current (built on s).
@@ -273,7 +265,6 @@ bi_pt_status bi_pt_destroy(bi_pt_ctx* ctx) {
     dfree(ctx, ctx->vals1); dfree(ctx, ctx->sort_counters); dfree(ctx, ctx->refit_cnt); dfree(ctx, ctx->nodes);
     dfree(ctx, ctx->nodes4); dfree(ctx, ctx->parent); dfree(ctx, ctx->leaf_geo); dfree(ctx, ctx->leaf_shade);
     dfree(ctx, ctx->tl_cost); dfree(ctx, ctx->tl_height); dfree(ctx, ctx->tl_snap); dfree(ctx, ctx->tl_starts);
-    dfree(ctx, ctx->rq_job); dfree(ctx, ctx->rq_cnt); dfree(ctx, ctx->rq_path); dfree(ctx, ctx->rq_hits);
     dfree(ctx, ctx->sums);
     engine_free(ctx, ctx->eng);
     delete ctx;
@@ -1120,80 +1111,44 @@ bi_pt_status bi_pt_debug_trace(bi_pt_ctx* ctx, uint32_t n, const float* rays, in
     for (uint32_t i = 0; i < n; ++i)
         if (rays[8 * i + 3] != 0.001f || rays[8 * i + 7] != tmax)
             return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "debug trace needs tmin = 0.001 and one tmax");
-    DevBuf<float> f[6];
-    DevBuf<uint32_t> path, cnt, out;
-    DevBuf<HitRec> hrec;
-    for (int k = 0; k < 6; ++k) BI_TRY(dalloc(ctx, f[k], n));
-    BI_TRY(dalloc(ctx, hrec, n));
-    BI_TRY(dalloc(ctx, path, n));
-    BI_TRY(dalloc(ctx, cnt, 4 + kWorkParts * kWorkStride));
-    BI_TRY(dalloc(ctx, out, n));
+    DevBuf<float> f[9];   // rays, then t, u, v
+    DevBuf<uint32_t> out;
+    bi_pt_status status = BI_PT_OK;
+    for (int k = 0; k < 9 && status == BI_PT_OK; ++k) status = dalloc(ctx, f[k], n);
+    if (status == BI_PT_OK) status = dalloc(ctx, out, n);
     std::vector<float> col(n);
     const int src[6] = {0, 1, 2, 4, 5, 6};
-    bi_pt_status status = BI_PT_OK;
     for (int k = 0; k < 6 && status == BI_PT_OK; ++k) {
         for (uint32_t i = 0; i < n; ++i) col[i] = rays[8 * i + src[k]];
         if (hipMemcpy(f[k].p, col.data(), n * 4, hipMemcpyHostToDevice) != hipSuccess) status = BI_PT_ERROR_HIP;
     }
-    std::vector<uint32_t> hn(4 + kWorkParts * kWorkStride, 0u);
-    hn[0] = n;
-    if (status == BI_PT_OK && hipMemcpy(cnt.p, hn.data(), hn.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
-        status = BI_PT_ERROR_HIP;
-    RayQueue q{f[0].p, f[1].p, f[2].p, f[3].p, f[4].p, f[5].p, path.p};
     if (status == BI_PT_OK) {
+        const bi_pt_rays r{f[0].p, f[1].p, f[2].p, f[3].p, f[4].p, f[5].p};
+        QueryArgs a = query_args(ctx, n, &r, tmax);
+        a.triangle = out.p;   // leaves: no order
         if (any_hit) {
-            launch_debug_anyhit(bvh_view(ctx), q, n, tmax, out.p, &ctx->eng.counters.p[kCntError], nullptr);
-            if (hipMemcpy(hit_leaf, out.p, n * 4, hipMemcpyDeviceToHost) != hipSuccess) status = BI_PT_ERROR_HIP;
+            launch_query_any(a, nullptr);
         } else {
-            // one job: this scene, extent tmax; path ids are only used to find the job
-            JobRec rec{};
-            rec.nodes = ctx->num_tris ? ctx->nodes4.p : ctx->eng.empty_tree.p;
-            rec.leaf_geo = ctx->leaf_geo.p;
-            rec.leaf_shade = ctx->leaf_shade.p;
-            rec.materials = ctx->mats.p;
-            rec.leaf_uv = scene_leaf_uv(ctx);
-            rec.tex = scene_tex(ctx);
-            rec.num_tris = ctx->num_tris;
-            rec.ray_length = tmax;
-            const uint32_t bases[4] = {0u, n, 0u, 0u};
-            DevBuf<unsigned char> jb;
-            BI_TRY(dalloc(ctx, jb, sizeof(JobRec) + sizeof bases));
-            if (hipMemcpy(jb.p, &rec, sizeof rec, hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemcpy(jb.p + sizeof(JobRec), bases, sizeof bases, hipMemcpyHostToDevice) != hipSuccess)
+            a.t = f[6].p;
+            a.u = f[7].p;
+            a.v = f[8].p;
+            launch_query_closest(a, nullptr);
+        }
+        auto down = [&](void* dst, const void* from) {
+            if (dst && status == BI_PT_OK && hipMemcpy(dst, from, n * 4, hipMemcpyDeviceToHost) != hipSuccess)
                 status = BI_PT_ERROR_HIP;
-            TraceArgs ta{};
-            ta.jobs = WaveJobs{reinterpret_cast<const JobRec*>(jb.p),
-                               reinterpret_cast<const uint32_t*>(jb.p + sizeof(JobRec)),
-                               reinterpret_cast<const uint32_t*>(jb.p + sizeof(JobRec)) + 2, 1u, n};
-            ta.q = q;
-            ta.count_in = cnt.p;
-            ta.work = cnt.p + 4;   // zeroed part counters
-            ta.parts = kWorkParts;
-            ta.refill = 32;
-            ta.any_hit = ctx->non_opaque ? 1u : 0u;
-    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
-    ta.step_bound = trace_step_bound(ctx->num_tris);
-            ta.hits = HitBuf{hrec.p};
-            ta.error = &ctx->eng.counters.p[kCntError];
-            if (status == BI_PT_OK) launch_trace_closest(ta, n, false, 16, 256, nullptr);
-            std::vector<HitRec> h(n);
-            if (hipMemcpy(h.data(), hrec.p, n * sizeof(HitRec), hipMemcpyDeviceToHost) != hipSuccess) {
-                status = BI_PT_ERROR_HIP;
-            } else {
-                for (uint32_t i = 0; i < n; ++i) {
-                    hit_leaf[i] = h[i].leaf;
-                    if (hit_t) hit_t[i] = h[i].t;
-                    if (hit_u) hit_u[i] = h[i].u;
-                    if (hit_v) hit_v[i] = h[i].v;
-                }
-            }
-            dfree(ctx, jb);
+        };
+        down(hit_leaf, out.p);
+        if (!any_hit) {
+            down(hit_t, f[6].p);
+            down(hit_u, f[7].p);
+            down(hit_v, f[8].p);
+            if (hit_t)   // a miss keeps the ray's extent here
+                for (uint32_t i = 0; i < n; ++i)
+                    if (hit_leaf[i] == kLeafMiss) hit_t[i] = tmax;
         }
     }
-    for (int k = 0; k < 6; ++k) dfree(ctx, f[k]);
-    dfree(ctx, hrec);
-    dfree(ctx, path);
-    dfree(ctx, cnt);
+    for (auto& b : f) dfree(ctx, b);
     dfree(ctx, out);
     if (status != BI_PT_OK) return fail(ctx, status, "debug trace failed");
     return BI_PT_OK;
@@ -1205,89 +1160,16 @@ bi_pt_status bi_pt_trace_closest(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* r
     BI_TRY(query_prepare(ctx, n, rays, tmax, s));
     if (n == 0) return BI_PT_OK;
     if (!hit_triangle) return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "null hit_triangle");
-    BI_TRY(dalloc(ctx, ctx->rq_job, sizeof(JobRec) + 4 * sizeof(uint32_t)));
-    BI_TRY(dalloc(ctx, ctx->rq_cnt, 4 + kWorkParts * kWorkStride));
-    BI_TRY(dalloc(ctx, ctx->rq_path, n));
-    BI_TRY(dalloc(ctx, ctx->rq_hits, n));
-    JobRec rec{};
-    rec.nodes = ctx->num_tris ? ctx->nodes4.p : ctx->eng.empty_tree.p;
-    rec.leaf_geo = ctx->leaf_geo.p;
-    rec.leaf_shade = ctx->leaf_shade.p;
-    rec.materials = ctx->mats.p;
-    rec.leaf_uv = scene_leaf_uv(ctx);
-    rec.tex = scene_tex(ctx);
-    rec.num_tris = ctx->num_tris;
-    rec.ray_length = tmax;
-    hipLaunchKernelGGL(k_put_query_job, dim3(1), dim3(64), 0, s, rec, n, ctx->rq_job.p);
-    launch_fill_u32(ctx->rq_cnt.p, 0u, 4 + kWorkParts * kWorkStride, s);   // count, then zeroed part counters
-    launch_fill_u32(ctx->rq_cnt.p, n, 1, s);
-    launch_fill_u32(ctx->rq_path.p, 0u, n, s);
-    TraceArgs ta{};
-    ta.jobs = WaveJobs{reinterpret_cast<const JobRec*>(ctx->rq_job.p),
-                       reinterpret_cast<const uint32_t*>(ctx->rq_job.p + sizeof(JobRec)),
-                       reinterpret_cast<const uint32_t*>(ctx->rq_job.p + sizeof(JobRec)) + 2, 1u, n};
-    ta.q = RayQueue{const_cast<float*>(rays->ox), const_cast<float*>(rays->oy), const_cast<float*>(rays->oz),
-                    const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz),
-                    ctx->rq_path.p};
-    ta.count_in = ctx->rq_cnt.p;
-    ta.work = ctx->rq_cnt.p + 4;
-    ta.parts = kWorkParts;
-    ta.refill = 32;
-    ta.any_hit = ctx->non_opaque ? 1u : 0u;
-    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
-    ta.step_bound = trace_step_bound(ctx->num_tris);
-    ta.hits = HitBuf{ctx->rq_hits.p};
-    ta.error = &ctx->eng.counters.p[kCntError];
-    launch_trace_closest(ta, n, false, 16, 256, s);
-    hipLaunchKernelGGL(k_query_hits, dim3((n + 255u) / 256u), dim3(256), 0, s, ctx->rq_hits.p,
-                       ctx->num_tris ? ctx->vals0.p : ctx->rq_path.p, n, hit_t, hit_triangle, hit_u, hit_v);
+    QueryArgs a = query_args(ctx, n, rays, tmax);
+    a.order = ctx->vals0.p;
+    a.t = hit_t;
+    a.triangle = hit_triangle;
+    a.u = hit_u;
+    a.v = hit_v;
+    launch_query_closest(a, s);
     BI_HIP_TRY(ctx, hipGetLastError());
     return BI_PT_OK;
 }
-
-}  // extern "C"
-
-// ---- closest-hit queries without device allocation ------------------------------
-// The scratch of bi_pt_trace_closest (the job record and its path bases, the ray count
-// and the persistent lanes' part counters, one hit record per ray) lives in this static
-// device array instead of context buffers.  Each GPU holds its own copy for the life of
-// the process; every call on a GPU uses that GPU's copy, so calls that overlap on one GPU
-// race (callers serialise them, e.g. on one stream).
-namespace {
-
-constexpr size_t kNoAllocJobBytes = 1024;     // JobRec + 4 path/pixel bases
-constexpr size_t kNoAllocCntBytes = 2048;     // count + part counters
-constexpr size_t kNoAllocBytes =
-    kNoAllocJobBytes + kNoAllocCntBytes + (size_t)BI_PT_NOALLOC_MAX_RAYS * sizeof(HitRec);
-static_assert(sizeof(JobRec) + 4 * sizeof(uint32_t) <= kNoAllocJobBytes, "job record fits its scratch slot");
-static_assert((4 + kWorkParts * kWorkStride) * sizeof(uint32_t) <= kNoAllocCntBytes, "counters fit");
-static_assert(kNoAllocJobBytes % 256 == 0 && kNoAllocCntBytes % 256 == 0, "slots keep 256-B alignment");
-
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
-
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-unsigned char* g_scratch_ptr[kMaxDevices] = {};
-
-// The device address of this GPU's scratch (looked up once per device, with the device
-// current; host code uses this address, never the array's name).
-bi_pt_status noalloc_scratch(Owner* own, int device, unsigned char** out) {
-    if (device < 0 || device >= kMaxDevices) return fail(own, BI_PT_ERROR_UNSUPPORTED, "device ordinal out of range");
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    if (!g_scratch_ptr[device]) {
-        void* p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return fail(own, BI_PT_ERROR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        g_scratch_ptr[device] = static_cast<unsigned char*>(p);
-    }
-    *out = g_scratch_ptr[device];
-    return BI_PT_OK;
-}
-
-}  // namespace
-
-extern "C" {
 
 bi_pt_status bi_pt_trace_closest_noalloc(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* rays, float tmax,
                                          float* hit_t, uint32_t* hit_triangle, float* hit_u, float* hit_v,
@@ -1312,44 +1194,13 @@ bi_pt_status bi_pt_trace_closest_noalloc(bi_pt_ctx* ctx, uint32_t n, const bi_pt
     if (n == 0) return BI_PT_OK;
     if (!hit_triangle) return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "null hit_triangle");
     BI_HIP_TRY(ctx, hipSetDevice(ctx->device));
-    unsigned char* base = nullptr;
-    BI_TRY(noalloc_scratch(ctx, ctx->device, &base));
-    unsigned char* job = base;
-    uint32_t* cnt = reinterpret_cast<uint32_t*>(base + kNoAllocJobBytes);
-    HitRec* hits = reinterpret_cast<HitRec*>(base + kNoAllocJobBytes + kNoAllocCntBytes);
-    JobRec rec{};
-    rec.nodes = ctx->num_tris ? ctx->nodes4.p : ctx->eng.empty_tree.p;
-    rec.leaf_geo = ctx->leaf_geo.p;
-    rec.leaf_shade = ctx->leaf_shade.p;
-    rec.materials = ctx->mats.p;
-    rec.leaf_uv = scene_leaf_uv(ctx);
-    rec.tex = scene_tex(ctx);
-    rec.num_tris = ctx->num_tris;
-    rec.ray_length = tmax;
-    // the previous call's contents are stale: the record, the count and the part
-    // counters are written afresh (fill kernels, no memset nodes under capture)
-    hipLaunchKernelGGL(k_put_query_job, dim3(1), dim3(64), 0, s, rec, n, job);
-    launch_fill_u32(cnt, 0u, 4 + kWorkParts * kWorkStride, s);
-    launch_fill_u32(cnt, n, 1, s);
-    TraceArgs ta{};
-    ta.jobs = WaveJobs{reinterpret_cast<const JobRec*>(job), reinterpret_cast<const uint32_t*>(job + sizeof(JobRec)),
-                       reinterpret_cast<const uint32_t*>(job + sizeof(JobRec)) + 2, 1u, n};
-    // one job: the kernel never reads path ids
-    ta.q = RayQueue{const_cast<float*>(rays->ox), const_cast<float*>(rays->oy), const_cast<float*>(rays->oz),
-                    const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz), nullptr};
-    ta.count_in = cnt;
-    ta.work = cnt + 4;
-    ta.parts = kWorkParts;
-    ta.refill = 32;
-    ta.any_hit = ctx->non_opaque ? 1u : 0u;
-    ta.one = ctx->num_tris <= kSmallTreeTris ? 1u : 0u;
-    ta.step_bound = trace_step_bound(ctx->num_tris);
-    ta.hits = HitBuf{hits};
-    ta.error = &ctx->eng.counters.p[kCntError];
-    launch_trace_closest(ta, n, false, 16, 256, s);
-    // a miss never reads the order; an empty scene has no order, any valid address serves
-    hipLaunchKernelGGL(k_query_hits, dim3((n + 255u) / 256u), dim3(256), 0, s, hits,
-                       ctx->num_tris ? ctx->vals0.p : cnt, n, hit_t, hit_triangle, hit_u, hit_v);
+    QueryArgs a = query_args(ctx, n, rays, tmax);
+    a.order = ctx->vals0.p;
+    a.t = hit_t;
+    a.triangle = hit_triangle;
+    a.u = hit_u;
+    a.v = hit_v;
+    launch_query_closest(a, s);
     BI_HIP_TRY(ctx, hipGetLastError());
     return BI_PT_OK;
 }
@@ -1365,9 +1216,9 @@ bi_pt_status bi_pt_trace_occlusion(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays*
         BI_HIP_TRY(ctx, hipGetLastError());
         return BI_PT_OK;
     }
-    RayQueue q{const_cast<float*>(rays->ox), const_cast<float*>(rays->oy), const_cast<float*>(rays->oz),
-               const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz), nullptr};
-    launch_debug_anyhit(bvh_view(ctx), q, n, tmax, occluded, &ctx->eng.counters.p[kCntError], s);
+    QueryArgs a = query_args(ctx, n, rays, tmax);
+    a.triangle = occluded;
+    launch_query_any(a, s);
     BI_HIP_TRY(ctx, hipGetLastError());
     return BI_PT_OK;
 }

@@ -682,13 +682,13 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 ta.q = qin;
                 ta.count_in = primary ? nullptr : cnt_in;
                 ta.hits = hits;
-                ta.work = &cnt[kCntTraceWork];
-                ta.parts = parts;
-                ta.refill = refill;
-                ta.any_hit = any_hit ? 1u : 0u;
-                ta.one = one;
-                ta.step_bound = trace_step_bound(max_tris);
-                ta.error = &cnt[kCntError];
+                ta.loop.work = &cnt[kCntTraceWork];
+                ta.loop.parts = parts;
+                ta.loop.refill = refill;
+                ta.loop.any_hit = any_hit ? 1u : 0u;
+                ta.loop.one = one;
+                ta.loop.step_bound = trace_step_bound(max_tris);
+                ta.loop.error = &cnt[kCntError];
                 BI_TRY(mark(0));
                 launch_trace_closest(ta, J.num_paths, primary, lds_stack, block, s);
                 ++launches_closest;
@@ -747,13 +747,13 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 sha.count_in = cnt_sh;
                 sha.ps = ps;
                 sha.ray_counters = rays;
-                sha.work = shadow_work;
-                sha.parts = parts;
-                sha.refill = refill;
-                sha.any_hit = (any_hit || any_point) ? 1u : 0u;
-                sha.one = one;
-                sha.step_bound = ta.step_bound;
-                sha.error = &cnt[kCntError];
+                sha.loop.work = shadow_work;
+                sha.loop.parts = parts;
+                sha.loop.refill = refill;
+                sha.loop.any_hit = (any_hit || any_point) ? 1u : 0u;
+                sha.loop.one = one;
+                sha.loop.step_bound = ta.loop.step_bound;
+                sha.loop.error = &cnt[kCntError];
                 if (overlap) {   // fork: the shadow rays trace beside the next closest-hit launch
                     BI_HIP_TRY(own, hipEventRecord(eng.ev_shade, s));
                     BI_HIP_TRY(own, hipStreamWaitEvent(eng.aux_s, eng.ev_shade, 0));

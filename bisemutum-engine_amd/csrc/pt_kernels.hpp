@@ -103,18 +103,24 @@ PT_HD PathKey path_key(const JobRec& J, uint32_t local) {
     return PathKey{q, pixel_of(q, J.cam.width, J.cam.height), J.sample0 + sl};
 }
 
+// The traversal loop of a launch: how its persistent lanes share the rays.
+struct TraceLoop {
+    uint32_t* work;             // part counters of the persistent lanes (zero at launch); null: every
+                                // wavefront has its own range of rays
+    uint32_t parts;             // queue parts (1..kWorkPartsMax)
+    uint32_t refill;            // idle lanes before a refill (1..64)
+    uint32_t any_hit;           // nonzero: some scene of the call has non-opaque triangles (shadow
+                                // launches: or point lights)
+    uint32_t one;               // nonzero: one scene of at most kSmallTreeTris triangles
+    uint32_t step_bound;        // steps without a finished ray that only corrupt links can reach (trace_step_bound)
+    uint32_t* error;
+};
 struct TraceArgs {
     WaveJobs jobs;
     RayQueue q;                 // input queue (unused for primary rays)
     const uint32_t* count_in;   // device count (null: primary, count = jobs.num_paths)
     HitBuf hits;
-    uint32_t* work;             // part counters of the persistent lanes (zero at launch)
-    uint32_t parts;             // queue parts (1..kWorkPartsMax)
-    uint32_t refill;            // idle lanes before a refill (1..64)
-    uint32_t any_hit;           // nonzero: some scene of the call has non-opaque triangles
-    uint32_t one;               // nonzero: one job whose scene has at most kSmallTreeTris triangles
-    uint32_t step_bound;        // steps without a finished ray that only corrupt links can reach (trace_step_bound)
-    uint32_t* error;
+    TraceLoop loop;
 };
 // A ray enters each node of its tree at most once and then waits for its leaves' tests:
 // tris is the most triangles of a scene of the launch.
@@ -123,8 +129,20 @@ PT_HD uint32_t trace_step_bound(uint32_t tris) { return tris + 4u; }
 void launch_trace_closest(const TraceArgs& a, uint32_t capacity, bool primary, uint32_t lds_stack, uint32_t block,
                           hipStream_t s);
 
-void launch_debug_anyhit(const BvhView& bvh, const RayQueue& q, uint32_t n, float tmax, uint32_t* out,
-                         uint32_t* error, hipStream_t s);
+// Ray queries: `count` rays of one extent, one scene.
+struct QueryArgs {
+    BvhView bvh;
+    RayQueue q;                 // path unused
+    uint32_t count;
+    float tmax;
+    const uint32_t* order;      // leaf -> triangle (null: the leaf itself)
+    float* t;                   // nullable
+    uint32_t* triangle;         // or, for occlusion, 1 / 0
+    float *u, *v;               // nullable
+    TraceLoop loop;
+};
+void launch_query_closest(const QueryArgs& a, hipStream_t s);
+void launch_query_any(const QueryArgs& a, hipStream_t s);
 
 struct ShadowArgs {
     WaveJobs jobs;
@@ -132,13 +150,7 @@ struct ShadowArgs {
     const uint32_t* count_in;
     PathState ps;
     uint64_t* ray_counters;     // sky shadow rays move from [2] (all shadow rays) to [3]
-    uint32_t* work;             // part counters of the persistent lanes (zero at launch)
-    uint32_t parts;             // queue parts (1..kWorkPartsMax)
-    uint32_t refill;            // idle lanes before a refill (1..64)
-    uint32_t any_hit;           // nonzero: some scene of the call has non-opaque triangles or point lights
-    uint32_t one;               // nonzero: one job whose scene has at most kSmallTreeTris triangles
-    uint32_t step_bound;        // steps without a finished ray that only corrupt links can reach (trace_step_bound)
-    uint32_t* error;
+    TraceLoop loop;
 };
 void launch_trace_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds_stack, uint32_t block, hipStream_t s);
 

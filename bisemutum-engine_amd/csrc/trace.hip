@@ -25,6 +25,8 @@
 // 12.9 ms per frame from 64-B nodes (4 loads), near and far planes by the ray's signs and
 // fused multiply-adds, winners' barycentrics kept in LDS instead of a second triangle test,
 // and a step whose masks stay in scalar registers (215 -> 150 VALU instructions).
+#include <algorithm>
+
 #include "pt_kernels.hpp"
 
 namespace bipt {
@@ -61,7 +63,6 @@ __device__ __forceinline__ TravRay trav_ray(V3 o, V3 d) {
     trav_ray_axis(r, 2, o.z, inv.z);
     return r;
 }
-__device__ __forceinline__ V3 trav_inv(const TravRay& r) { return v3(r.inv[0], r.inv[1], r.inv[2]); }
 
 // A node's record in registers.
 struct NodeRegs {
@@ -117,7 +118,9 @@ __device__ __forceinline__ bool leaf_non_opaque(const LeafRegs& r) {
 }
 // Any-hit test of a non-opaque leaf hit at barycentric numerators (un, vn) / det by the
 // ray (o, d) of a job: whether its surface is present for that ray.
-__device__ __forceinline__ bool leaf_present(const JobRec& J, uint32_t leaf, float un, float vn, float det, V3 o,
+// (Scene: JobRec or BvhView.)
+template <class Scene>
+__device__ __forceinline__ bool leaf_present(const Scene& J, uint32_t leaf, float un, float vn, float det, V3 o,
                                              V3 d) {
     const MaterialRec& M = J.materials[J.leaf_shade[leaf].material];
     return surface_present(M, J.tex, J.leaf_uv, leaf, un / det, vn / det, opacity_random(J.seed, o, d));
@@ -178,20 +181,54 @@ struct ShortStack {
 };
 
 // Ray fetch for the lanes that ask (the caller decides when a wavefront refills: once
-// `refill` lanes are idle, or no lane is busy): one atomic per refill.  The queue is
-// split into `parts` contiguous parts, each with its own counter on its own 128-B
-// line; a wavefront starts on the part of its workgroup's XCD (workgroups go to the
-// XCDs round-robin) and moves on to the following parts when its part runs dry, so
-// no single counter sees every refill.  Returns the new ray index for a lane that
-// asked and got one, kNoRay otherwise; every part is drained once `left` is 0.
+// `refill` lanes are idle, or no lane is busy).  The rays are split into `parts` contiguous
+// parts; a wavefront starts on the part of its workgroup's XCD (workgroups go to the XCDs
+// round-robin).
+//
+// Shared parts: each part has a counter on its own 128-B line, one atomic per refill, and a
+// wavefront moves on to the following parts when its part runs dry, so no single counter
+// sees every refill.
+//
+// Own runs (no counters, no atomics, nothing that two launches could share): wavefront w of
+// a part takes the part's rays 64 w .. 64 w + 63, then those a whole row of wavefronts
+// further on, so that neighbouring rays (of like cost, reading like nodes) are spread over the
+// wavefronts of the XCD.  Launches without counters (`work` null) deal their rays out that
+// way, and so do launches whose wavefronts hold every ray at once; those deal thinly, 8 to
+// 64 rays each on about one wavefront per SIMD, because a step of a wavefront with few rays
+// waits for fewer cache lookups.  Box room, 320x240, 1 spp, depth 4 (launches of 77k rays
+// and fewer): frame 783 -> 663 us.  Queries: 64 rays 55 -> 39 us (of it the scratch's four
+// small launches), 2.07 M reflection rays 443 -> 413 us; with one contiguous range per
+// wavefront 508 us (ranges of unlike cost); 1.84 M occlusion rays of 2 m, before one ray per
+// lane in a plain loop, 458 -> 261 us.
+//
+// Returns the new ray index for a lane that asked and got one, kNoRay otherwise; nothing is
+// left once `left` is 0.
 struct WorkCursor {
     uint32_t part;    // part the wavefront draws from
     uint32_t left;    // parts not yet found empty
     uint32_t parts;
     uint32_t chunk;   // rays per part (the last parts may hold fewer)
+    bool own;         // own runs of the part
+    uint32_t next;    // rays of its runs already taken
+    uint32_t run;     // rays per run (64 unless there is only one)
+    uint32_t first;   // the first run's offset in the part
+    uint32_t row;     // from one run to the next
 };
-__device__ __forceinline__ WorkCursor work_cursor(uint32_t count, uint32_t parts) {
-    return WorkCursor{blockIdx.x % parts, parts, parts, (count + parts - 1u) / parts};
+constexpr uint32_t kThinWaves = 1024;   // one wavefront per SIMD
+template <int B>
+__device__ __forceinline__ WorkCursor work_cursor(const uint32_t* work, uint32_t count, uint32_t parts) {
+    const uint32_t chunk = (count + parts - 1u) / parts, part = blockIdx.x % parts;
+    const uint32_t waves = gridDim.x / parts * (B / 64);   // a part's (at least one workgroup per part)
+    const uint32_t thin = min(64u, max(8u, (count + kThinWaves - 1u) / kThinWaves));
+    const bool fits = (uint64_t)thin * waves >= chunk;
+    if (!fits && work) return WorkCursor{part, parts, parts, chunk, false, 0u, 0u, 0u, 0u};
+    const uint32_t run = fits ? thin : 64u;
+    // (a last, incomplete row of workgroups has nothing to do)
+    const uint32_t wave = blockIdx.x / parts * (B / 64) +
+                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t first = wave * run;
+    const bool any = wave < waves && first < chunk;
+    return WorkCursor{part, any ? 1u : 0u, parts, chunk, true, 0u, run, first, waves * run};
 }
 __device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bool want, WorkCursor& wc) {
     const uint64_t m = __ballot(want);
@@ -199,6 +236,15 @@ __device__ __forceinline__ uint32_t fetch_ray(uint32_t* work, uint32_t count, bo
     const uint32_t lane = __lane_id();
     const uint32_t leader = (uint32_t)__builtin_ctzll(m);
     const uint32_t rank = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    if (wc.own) {
+        // (one run: next + rank may pass its end; several: runs are 64 rays)
+        const uint32_t k = wc.next + rank, turn = k >> 6;
+        const bool mine = wc.run == 64u || k < wc.run;
+        const uint32_t in_part = wc.first + turn * wc.row + (k & 63u), idx = wc.part * wc.chunk + in_part;
+        wc.next += (uint32_t)__popcll(m);
+        if ((wc.run != 64u && wc.next >= wc.run) || wc.first + (wc.next >> 6) * wc.row >= wc.chunk) wc.left = 0u;
+        return want && mine && in_part < wc.chunk && idx < count ? idx : kNoRay;
+    }
     while (wc.left != 0u) {
         const uint32_t lo = min(wc.part * wc.chunk, count);
         const uint32_t hi = min(lo + wc.chunk, count);
@@ -329,17 +375,82 @@ __device__ __forceinline__ void node_step(const TravNode* nodes, int& cur, const
     for (int k = 0; k < 4; ++k) append_leaf(queue, qn, leaf[k], n.ch[k], lane);
 }
 
+// Rays of a wave's paths: camera rays (made here, from the path's pixel and sample) or the
+// extension queue; hits go to the wave's hit records.
+template <bool PRIMARY>
+struct PathRays {
+    using Scene = JobRec;
+    const TraceArgs& a;
+    __device__ __forceinline__ uint32_t count() const { return PRIMARY ? a.jobs.num_paths : *a.count_in; }
+    __device__ __forceinline__ const JobRec* scene() const { return a.jobs.rec; }
+    // one job: its record sits at a uniform address (scalar loads); several: the path's job
+    // is looked up per lane
+    template <bool ONE>
+    __device__ __forceinline__ const JobRec* start(uint32_t i, V3& o, V3& d, float& tmax) const {
+        const JobRec* J = a.jobs.rec;
+        uint32_t local = i;
+        if (!ONE && a.jobs.num_jobs != 1u) {
+            const uint32_t path = PRIMARY ? i : a.q.path[i];
+            const uint32_t jid = job_of(a.jobs.path_base, a.jobs.num_jobs, path);
+            J = a.jobs.rec + jid;
+            local = path - a.jobs.path_base[jid];
+        }
+        tmax = J->ray_length;
+        if constexpr (PRIMARY) {
+            const PathKey k = path_key(*J, local);
+            float jx = 0.5f, jy = 0.5f;
+            if (J->flags & 1u) {
+                Pcg jr = pcg_keyed(J->seed, k.pixel, k.sample, kJitterBounce);
+                jx = pcg_float(jr);
+                jy = pcg_float(jr);
+            }
+            camera_ray(J->cam, k.pixel % J->cam.width, k.pixel / J->cam.width, jx, jy, &o, &d);
+        } else {
+            o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
+            d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
+        }
+        return J;
+    }
+    __device__ __forceinline__ void finish(uint32_t i, HitRec h) const { a.hits.rec[i] = h; }
+};
+// Rays of a query (the caller's arrays); results go straight to the caller's arrays: t (+inf
+// on a miss), the triangle's index in the scene's order, barycentrics; or whether anything
+// was hit.
+struct QueryRays {
+    using Scene = BvhView;
+    const QueryArgs& a;
+    __device__ __forceinline__ uint32_t count() const { return a.count; }
+    __device__ __forceinline__ const BvhView* scene() const { return &a.bvh; }
+    template <bool ONE>
+    __device__ __forceinline__ const BvhView* start(uint32_t i, V3& o, V3& d, float& tmax) const {
+        o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
+        d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
+        tmax = a.tmax;
+        return &a.bvh;
+    }
+    __device__ __forceinline__ void finish(uint32_t i, HitRec h) const {
+        const bool hit = h.leaf != kLeafMiss;
+        if (a.t) a.t[i] = hit ? h.t : __builtin_inff();
+        a.triangle[i] = hit && a.order ? a.order[h.leaf] : h.leaf;
+        if (a.u) a.u[i] = h.u;
+        if (a.v) a.v[i] = h.v;
+    }
+    __device__ __forceinline__ void finish_any(uint32_t i, bool occ) const { a.triangle[i] = occ ? 1u : 0u; }
+};
+
 // AH: the call's scenes hold non-opaque (alpha-tested or translucent) triangles, whose
 // hits pass the any-hit test; without them the test and its registers are compiled out.
-// ONE: every ray of the launch belongs to job 0 and its nodes lie within 4 GB, so the
+// ONE: every ray of the launch belongs to one scene whose nodes lie within 4 GB, so the
 // scene pointers are uniform (scalar registers) instead of per lane.
-template <bool PRIMARY, bool AH, int L, int B, bool ONE>
-__device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
+// S: where rays come from and hits go (PathRays, QueryRays): the scene of ray 0, a ray's
+// origin, direction, extent and scene, and its finished hit.
+template <bool AH, int L, int B, bool ONE, class S>
+__device__ __forceinline__ void trace_closest_body(const S& src, const TraceLoop& a) {
     __shared__ int lds[L][B];
     __shared__ uint2 s_queue[B / 64][kLeafQueue];
     __shared__ unsigned long long s_key[B / 64][64];
     __shared__ float2 s_uv[B / 64][64];
-    const uint32_t count = PRIMARY ? a.jobs.num_paths : *a.count_in;
+    const uint32_t count = src.count();
     const float tmin = kTMin;
     // Each lane keeps its ray's scene (BVH nodes, leaf records, triangle count): a wave
     // may hold rays of several jobs.  A job without triangles points at a one-node tree
@@ -358,13 +469,13 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
     float2* uv = s_uv[w];
     uint32_t qn = 0;
     uint32_t ray = kNoRay;
-    WorkCursor wc = work_cursor(count, a.parts);
+    WorkCursor wc = work_cursor<B>(a.work, count, a.parts);
     V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f);
     TravRay rb = trav_ray(o, d);
     float tbest = 0.0f;
-    const TravNode* nodes = a.jobs.rec[0].nodes;
-    const LeafGeo* geo = a.jobs.rec[0].leaf_geo;
-    const JobRec* jr = a.jobs.rec;   // the lane's job (materials for any-hit tests)
+    const typename S::Scene* scene = src.scene();   // the lane's scene (materials for any-hit tests)
+    const TravNode* nodes = scene->nodes;
+    const LeafGeo* geo = scene->leaf_geo;
     ShortStack<L, B> st;
     st.bottom = (LdsInt*)&lds[0][threadIdx.x];
     LdsInt* top = st.bottom;
@@ -406,8 +517,8 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
                 if constexpr (AH) {
                     const bool nop = cand && leaf_non_opaque(lr);
                     if (__ballot(nop) != 0ull) {
-                        const JobRec* oj = ONE ? jr : shfl_ptr(jr, owner);
-                        if (nop) cand = leaf_present(*oj, leaf, un, vn, det, oo, dd);
+                        const typename S::Scene* os = ONE ? scene : shfl_ptr(scene, owner);
+                        if (nop) cand = leaf_present(*os, leaf, un, vn, det, oo, dd);
                     }
                 }
                 const unsigned long long mine = ((unsigned long long)__float_as_uint(t) << 32) | leaf;
@@ -423,7 +534,7 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
             dry = 0;
             if (cur == kParked) {
                 const float2 buv = uv[lane];
-                a.hits.rec[ray] = HitRec{tbest, (uint32_t)key[lane], buv.x, buv.y};
+                src.finish(ray, HitRec{tbest, (uint32_t)key[lane], buv.x, buv.y});
                 cur = kIdle;
             }
         }
@@ -431,37 +542,12 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
         if (refill_now) got = fetch_ray(a.work, count, cur == kIdle, wc);
         const bool fresh = got != kNoRay;
         if (fresh) {
-            // one job: its record sits at a uniform address (scalar loads); several: the
-            // path's job is looked up per lane
             float tmax = 0.0f;
-            auto setup = [&](const JobRec& J, uint32_t local) {
-                if constexpr (!ONE) {
-                    nodes = J.nodes;
-                    geo = J.leaf_geo;
-                    jr = &J;
-                }
-                tmax = J.ray_length;
-                if (PRIMARY) {
-                    const PathKey k = path_key(J, local);
-                    float jx = 0.5f, jy = 0.5f;
-                    if (J.flags & 1u) {
-                        Pcg jr = pcg_keyed(J.seed, k.pixel, k.sample, kJitterBounce);
-                        jx = pcg_float(jr);
-                        jy = pcg_float(jr);
-                    }
-                    camera_ray(J.cam, k.pixel % J.cam.width, k.pixel / J.cam.width, jx, jy, &o, &d);
-                }
-            };
-            if (ONE || a.jobs.num_jobs == 1u) {
-                setup(a.jobs.rec[0], got);
-            } else {
-                const uint32_t path = PRIMARY ? got : a.q.path[got];
-                const uint32_t jid = job_of(a.jobs.path_base, a.jobs.num_jobs, path);
-                setup(a.jobs.rec[jid], path - a.jobs.path_base[jid]);
-            }
-            if (!PRIMARY) {
-                o = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
-                d = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
+            const typename S::Scene* sc = src.template start<ONE>(got, o, d, tmax);
+            if constexpr (!ONE) {
+                scene = sc;
+                nodes = sc->nodes;
+                geo = sc->leaf_geo;
             }
             ray = got;
             rb = trav_ray(o, d);
@@ -477,76 +563,17 @@ __device__ __forceinline__ void trace_closest_body(const TraceArgs& a) {
 
 template <bool PRIMARY, bool AH, int L, int B>
 __global__ __launch_bounds__(B) void k_trace_closest(TraceArgs a) {
-    trace_closest_body<PRIMARY, AH, L, B, false>(a);
+    trace_closest_body<AH, L, B, false>(PathRays<PRIMARY>{a}, a.loop);
 }
 // One job, opaque scene, 256-thread blocks and a 12-deep LDS stack (the defaults): the
 // scene pointers sit in scalar registers, which frees six vector registers per lane.
 template <bool PRIMARY>
-__global__ __launch_bounds__(256) void k_trace_closest_one(TraceArgs a) {
-    trace_closest_body<PRIMARY, false, 12, 256, true>(a);
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_trace_closest_one(TraceArgs a) {
+    trace_closest_body<false, 12, 256, true>(PathRays<PRIMARY>{a}, a.loop);
 }
-
-// Any-hit traversal of one ray (inspection kernel).  The answer does not depend on the
-// visiting order (no pruning by a running distance); the order is the shadow kernel's:
-// the hit internal child entered farthest along the ray first, the others pushed in slot
-// order.
-template <int L>
-__device__ __forceinline__ bool occluded(const BvhView& bvh, int (*lds)[256], V3 o, V3 d, float tmin, float tmax,
-                                         uint32_t* error) {
-    if (bvh.num_tris == 0) return false;
-    const TravRay rb = trav_ray(o, d);
-    ShortStack<L> st;
-    st.bottom = (LdsInt*)&lds[0][threadIdx.x];
-    LdsInt* top = st.bottom;
-    int node = 0;
-    for (uint32_t steps = 1;; ++steps) {
-        if (steps > bvh.num_tris) {   // corrupt links: end the ray instead of looping
-            atomicOr(error, 8u);
-            return false;
-        }
-        NodeRegs n;
-        load_node<false>(n, bvh.nodes, node);
-        const TravPlanes p = node_planes(n, rb);
-        int next = kParked;
-        bool in[4], lf[4];
-        float tfar = -1.0f;   // the shadow kernel's order: the farthest-entered hit internal child first
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float tn;
-            const bool h = trav_visit(p, k, tmax, &tn);
-            in[k] = h && n.ch[k] > 0;
-            lf[k] = h && n.ch[k] < 0;
-            if (in[k] && tn > tfar) {
-                tfar = tn;
-                next = n.ch[k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (!lf[k]) continue;
-            float t, un, vn, det;
-            const uint32_t leaf = (uint32_t)~n.ch[k];
-            const LeafRegs lr = load_leaf(bvh.leaf_geo, leaf);
-            if (tri_test(lr, o, d, &t, &un, &vn, &det) && t >= tmin && t <= tmax &&
-                box_exact(lr, bvh.leaf_geo, leaf, o, trav_inv(rb), tmin, tmax) &&
-                (!leaf_non_opaque(lr) ||
-                 surface_present(bvh.materials[bvh.leaf_shade[leaf].material], bvh.tex, bvh.leaf_uv, leaf, un / det,
-                                 vn / det, opacity_random(bvh.seed, o, d))))
-                return true;
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (in[k] && n.ch[k] != next && !st.push(top, n.ch[k])) {
-                atomicOr(error, 1u);
-                return false;
-            }
-        }
-        if (next == kParked) {
-            if (top == st.bottom) return false;
-            next = st.pop(top);
-        }
-        node = next;
-    }
+template <bool AH, bool ONE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AH ? 5 : 6))) void k_query_closest(QueryArgs a) {
+    trace_closest_body<AH, 12, 256, ONE>(QueryRays{a}, a.loop);
 }
 
 // Adds shadow ray i's contribution unless it is occluded; returns whether it is a sky ray.
@@ -578,17 +605,54 @@ __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bo
     return kind == kKindSky;
 }
 
-// AH (the general variant): any-hit tests of non-opaque leaves and rays that end at a
-// point light; launched when a scene of the call has either.
-template <bool AH, int L, int B, bool ONE>
-__device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
+// A segment's shadow rays; a finished ray adds its contribution to its path.
+struct ShadowRays {
+    using Scene = JobRec;
+    const ShadowArgs& a;
+    uint32_t& sky_rays;   // ray statistics: sky shadow rays this lane finished
+    __device__ __forceinline__ uint32_t count() const { return *a.count_in; }
+    __device__ __forceinline__ const JobRec* scene() const { return a.jobs.rec; }
+    // A sky ray's direction is in the queue; a light's ray is rebuilt from the light as the
+    // shading built it (without point lights, every light is directional and every extent
+    // unbounded).
+    template <bool AH, bool ONE>
+    __device__ __forceinline__ const JobRec* start(uint32_t i, V3& o, V3& d, float& tmax) const {
+        const uint32_t pk = a.q.pk[i], kind = pk & 7u;
+        const JobRec& J = ONE || a.jobs.num_jobs == 1u ? a.jobs.rec[0]
+                                                       : a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, pk >> 3)];
+        o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
+        tmax = kShadowTMax;
+        if (kind == kKindSky) {
+            d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
+        } else if constexpr (AH) {
+            light_shadow_ray(J.lights[kind], o, &d, &tmax);
+        } else {
+            const LightRec& Lk = J.lights[kind];
+            d = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
+        }
+        return &J;
+    }
+    __device__ __forceinline__ void finish_any(uint32_t i, bool occ) const { sky_rays += apply_shadow(a, i, occ) ? 1u : 0u; }
+};
+// Rays of an occlusion query.
+struct AnyQueryRays : QueryRays {
+    template <bool AH, bool ONE>
+    __device__ __forceinline__ const BvhView* start(uint32_t i, V3& o, V3& d, float& tmax) const {
+        return QueryRays::start<ONE>(i, o, d, tmax);
+    }
+};
+
+// AH (the general variant): any-hit tests of non-opaque leaves and rays of finite extent
+// (towards point lights, occlusion queries); launched when a scene of the call has either.
+template <bool AH, int L, int B, bool ONE, class S>
+__device__ __forceinline__ void trace_any_body(const S& src, const TraceLoop& a) {
     __shared__ int lds[L][B];
     __shared__ uint2 s_queue[B / 64][kLeafQueue];
     __shared__ uint32_t s_occ[B / 64][64];
-    const uint32_t count = *a.count_in;
+    const uint32_t count = src.count();
     const float tmin = kTMin;
     // a ray's extent: unbounded towards the sky and directional lights, the distance to a
-    // point light (the general variant only; the other has no point lights)
+    // point light or a query's (the general variant only)
     float tmax = kShadowTMax;
     // Same iteration as the closest-hit kernel: box steps queue their leaves, the queue
     // is flushed at flush_at, before a refill or when no lane is busy, and parked lanes
@@ -603,18 +667,17 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
     occf[lane] = 0u;
     uint32_t qn = 0;
     uint32_t ray = kNoRay;
-    WorkCursor wc = work_cursor(count, a.parts);
+    WorkCursor wc = work_cursor<B>(a.work, count, a.parts);
     V3 o = v3(0.f, 0.f, 0.f), d = v3(0.f, 0.f, 1.f);
     TravRay rb = trav_ray(o, d);
-    const TravNode* nodes = a.jobs.rec[0].nodes;   // the lane's ray's scene (see k_trace_closest)
-    const LeafGeo* geo = a.jobs.rec[0].leaf_geo;
-    const JobRec* jr = a.jobs.rec;
+    const typename S::Scene* scene = src.scene();   // the lane's ray's scene (see trace_closest_body)
+    const TravNode* nodes = scene->nodes;
+    const LeafGeo* geo = scene->leaf_geo;
     ShortStack<L, B> st;
     st.bottom = (LdsInt*)&lds[0][threadIdx.x];
     LdsInt* top = st.bottom;
     int cur = kIdle;
     uint32_t dry = 0;   // steps since a ray of the wavefront finished
-    uint32_t sky_rays = 0;   // ray statistics: sky shadow rays this lane finished
     for (;;) {
         node_step<false, ONE, L, B>(nodes, cur, rb, tmax, st, top, queue, qn, lane, a.error);
         if (++dry > a.step_bound) {   // corrupt links (see k_trace_closest)
@@ -646,8 +709,8 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
                 if constexpr (AH) {
                     const bool nop = cand && leaf_non_opaque(lr);
                     if (__ballot(nop) != 0ull) {
-                        const JobRec* oj = ONE ? jr : shfl_ptr(jr, owner);
-                        if (nop) cand = leaf_present(*oj, leaf, un, vn, det, oo, dd);
+                        const typename S::Scene* os = ONE ? scene : shfl_ptr(scene, owner);
+                        if (nop) cand = leaf_present(*os, leaf, un, vn, det, oo, dd);
                     }
                 }
                 if (cand) occf[owner] = 1u;
@@ -661,7 +724,7 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
         if (__ballot(done) != 0ull) {
             dry = 0;
             if (done) {
-                sky_rays += apply_shadow(a, ray, occ) ? 1u : 0u;
+                src.finish_any(ray, occ);
                 cur = kIdle;
             }
         }
@@ -669,30 +732,13 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
         if (refill_now) got = fetch_ray(a.work, count, cur == kIdle, wc);
         const bool fresh = got != kNoRay;
         if (fresh) {
-            auto setup = [&](const JobRec& J) {
-                if constexpr (!ONE) {
-                    nodes = J.nodes;
-                    geo = J.leaf_geo;
-                    jr = &J;
-                }
-            };
-            const uint32_t pk = a.q.pk[got];
-            const JobRec& J = ONE || a.jobs.num_jobs == 1u ? a.jobs.rec[0]
-                                                    : a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, pk >> 3)];
-            setup(J);
-            o = v3(a.q.ox[got], a.q.oy[got], a.q.oz[got]);
-            // a sky ray's direction is in the queue; a light's ray is rebuilt from the
-            // light as the shading built it (without point lights, every light is
-            // directional and every extent unbounded)
-            const uint32_t kind = pk & 7u;
-            if (kind == kKindSky) {
-                d = v3(a.q.dx[got], a.q.dy[got], a.q.dz[got]);
-                if constexpr (AH) tmax = kShadowTMax;
-            } else if constexpr (AH) {
-                light_shadow_ray(J.lights[kind], o, &d, &tmax);
-            } else {
-                const LightRec& Lk = J.lights[kind];
-                d = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
+            float extent;
+            const typename S::Scene* sc = src.template start<AH, ONE>(got, o, d, extent);
+            if constexpr (AH) tmax = extent;
+            if constexpr (!ONE) {
+                scene = sc;
+                nodes = sc->nodes;
+                geo = sc->leaf_geo;
             }
             ray = got;
             rb = trav_ray(o, d);
@@ -701,11 +747,17 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
         }
         if (wc.left == 0u && __ballot(cur != kIdle) == 0ull) break;
     }
+}
+
+template <bool AH, int L, int B, bool ONE>
+__device__ __forceinline__ void trace_shadow(const ShadowArgs& a) {
+    uint32_t sky_rays = 0;
+    trace_any_body<AH, L, B, ONE>(ShadowRays{a, sky_rays}, a.loop);
     // the shade launch counted every shadow ray as a light shadow ray: move the sky
     // rays over, one atomic pair per workgroup
     for (int off = 32; off >= 1; off >>= 1) sky_rays += __shfl_xor(sky_rays, off);
     __shared__ uint32_t s_sky[B / 64];
-    if (lane == 0) s_sky[w] = sky_rays;
+    if (__lane_id() == 0) s_sky[threadIdx.x >> 6] = sky_rays;
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t tot = 0;
@@ -719,20 +771,14 @@ __device__ __forceinline__ void trace_shadow_body(const ShadowArgs& a) {
 
 template <bool AH, int L, int B>
 __global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
-    trace_shadow_body<AH, L, B, false>(a);
+    trace_shadow<AH, L, B, false>(a);
 }
 // One job, opaque scene, the default stack and block (as k_trace_closest_one).
-__global__ __launch_bounds__(256) void k_trace_shadow_one(ShadowArgs a) { trace_shadow_body<false, 12, 256, true>(a); }
-
-template <int L>
-__global__ __launch_bounds__(256) void k_debug_anyhit(BvhView bvh, RayQueue q, uint32_t n, float tmax,
-                                                      uint32_t* out, uint32_t* error) {
-    __shared__ int lds[L][256];
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    V3 o = v3(q.ox[i], q.oy[i], q.oz[i]);
-    V3 d = v3(q.dx[i], q.dy[i], q.dz[i]);
-    out[i] = occluded<L>(bvh, lds, o, d, kTMin, tmax, error) ? 1u : 0u;
+__global__ __launch_bounds__(256) void k_trace_shadow_one(ShadowArgs a) { trace_shadow<false, 12, 256, true>(a); }
+// Occlusion queries: their extent is the caller's, so the general variant.
+template <bool ONE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONE ? 6 : 5))) void k_query_any(QueryArgs a) {
+    trace_any_body<true, 12, 256, ONE>(AnyQueryRays{{a}}, a.loop);
 }
 
 // Workgroups that stay resident on the whole chip for a kernel (persistent grid).
@@ -750,42 +796,41 @@ uint32_t resident_groups(K kernel, int block) {
     return (uint32_t)(cus * per_cu);
 }
 
+// Workgroups of a launch of up to n rays: at least those that deal few rays out thinly
+// (work_cursor), at most what stays resident, in whole rows of one workgroup per part.
+template <int B, class K>
+uint32_t launch_groups(K kernel, uint32_t& resident, uint32_t n, uint32_t parts) {
+    if (resident == 0) resident = resident_groups(kernel, B);
+    constexpr uint32_t per = B / 64;
+    const uint32_t thin = std::min((n + 8u * per - 1u) / (8u * per), kThinWaves / per);
+    const uint32_t rows = (std::max((n + B - 1u) / B, thin) + parts - 1u) / parts;
+    return std::max(std::min(rows, resident / parts), 1u) * parts;
+}
+
 template <bool P, bool AH, int L, int B>
 void closest_lb(const TraceArgs& a, uint32_t capacity, hipStream_t s) {
-    uint32_t groups = (capacity + B - 1u) / B;
     static uint32_t resident = 0;
-    if (resident == 0) resident = resident_groups(k_trace_closest<P, AH, L, B>, B);
-    if (groups > resident) groups = resident;
-    if (groups == 0) groups = 1;
+    const uint32_t groups = launch_groups<B>(k_trace_closest<P, AH, L, B>, resident, capacity, a.loop.parts);
     hipLaunchKernelGGL((k_trace_closest<P, AH, L, B>), dim3(groups), dim3(B), 0, s, a);
 }
 
 template <bool P>
 void closest_one(const TraceArgs& a, uint32_t capacity, hipStream_t s) {
-    uint32_t groups = (capacity + 255u) / 256u;
     static uint32_t resident = 0;
-    if (resident == 0) resident = resident_groups(k_trace_closest_one<P>, 256);
-    if (groups > resident) groups = resident;
-    if (groups == 0) groups = 1;
+    const uint32_t groups = launch_groups<256>(k_trace_closest_one<P>, resident, capacity, a.loop.parts);
     hipLaunchKernelGGL((k_trace_closest_one<P>), dim3(groups), dim3(256), 0, s, a);
 }
 
 void shadow_one(const ShadowArgs& a, uint32_t capacity, hipStream_t s) {
-    uint32_t groups = (capacity + 255u) / 256u;
     static uint32_t resident = 0;
-    if (resident == 0) resident = resident_groups(k_trace_shadow_one, 256);
-    if (groups > resident) groups = resident;
-    if (groups == 0) groups = 1;
+    const uint32_t groups = launch_groups<256>(k_trace_shadow_one, resident, capacity, a.loop.parts);
     hipLaunchKernelGGL(k_trace_shadow_one, dim3(groups), dim3(256), 0, s, a);
 }
 
 template <bool AH, int L, int B>
 void shadow_lb(const ShadowArgs& a, uint32_t capacity, hipStream_t s) {
-    uint32_t groups = (capacity + B - 1u) / B;
     static uint32_t resident = 0;
-    if (resident == 0) resident = resident_groups(k_trace_shadow<AH, L, B>, B);
-    if (groups > resident) groups = resident;
-    if (groups == 0) groups = 1;
+    const uint32_t groups = launch_groups<B>(k_trace_shadow<AH, L, B>, resident, capacity, a.loop.parts);
     hipLaunchKernelGGL((k_trace_shadow<AH, L, B>), dim3(groups), dim3(B), 0, s, a);
 }
 
@@ -827,33 +872,54 @@ void dispatch_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds, uint3
 void launch_trace_closest(const TraceArgs& a, uint32_t capacity, bool primary, uint32_t lds_stack, uint32_t block,
                           hipStream_t s) {
     if (capacity == 0) return;
-    if (a.one && !a.any_hit && block == 256 && lds_stack > 8 && lds_stack <= 12) {
+    if (a.loop.one && !a.loop.any_hit && block == 256 && lds_stack > 8 && lds_stack <= 12) {
         if (primary) closest_one<true>(a, capacity, s);
         else closest_one<false>(a, capacity, s);
         return;
     }
     if (primary) {
-        if (a.any_hit) dispatch_closest<true, true>(a, capacity, lds_stack, block, s);
+        if (a.loop.any_hit) dispatch_closest<true, true>(a, capacity, lds_stack, block, s);
         else dispatch_closest<true, false>(a, capacity, lds_stack, block, s);
     } else {
-        if (a.any_hit) dispatch_closest<false, true>(a, capacity, lds_stack, block, s);
+        if (a.loop.any_hit) dispatch_closest<false, true>(a, capacity, lds_stack, block, s);
         else dispatch_closest<false, false>(a, capacity, lds_stack, block, s);
     }
 }
 
-void launch_debug_anyhit(const BvhView& bvh, const RayQueue& q, uint32_t n, float tmax, uint32_t* out,
-                         uint32_t* error, hipStream_t s) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_debug_anyhit<16>, dim3((n + 255u) / 256u), dim3(256), 0, s, bvh, q, n, tmax, out, error);
+namespace {
+
+template <bool AH, bool ONE>
+void query_closest(const QueryArgs& a, hipStream_t s) {
+    static uint32_t resident = 0;
+    const uint32_t groups = launch_groups<256>(k_query_closest<AH, ONE>, resident, a.count, a.loop.parts);
+    hipLaunchKernelGGL((k_query_closest<AH, ONE>), dim3(groups), dim3(256), 0, s, a);
+}
+template <bool ONE>
+void query_any(const QueryArgs& a, hipStream_t s) {
+    static uint32_t resident = 0;
+    const uint32_t groups = launch_groups<256>(k_query_any<ONE>, resident, a.count, a.loop.parts);
+    hipLaunchKernelGGL((k_query_any<ONE>), dim3(groups), dim3(256), 0, s, a);
+}
+
+}  // namespace
+
+void launch_query_closest(const QueryArgs& a, hipStream_t s) {
+    if (a.count == 0) return;
+    if (a.loop.any_hit) a.loop.one ? query_closest<true, true>(a, s) : query_closest<true, false>(a, s);
+    else a.loop.one ? query_closest<false, true>(a, s) : query_closest<false, false>(a, s);
+}
+void launch_query_any(const QueryArgs& a, hipStream_t s) {
+    if (a.count == 0) return;
+    a.loop.one ? query_any<true>(a, s) : query_any<false>(a, s);
 }
 
 void launch_trace_shadow(const ShadowArgs& a, uint32_t capacity, uint32_t lds, uint32_t block, hipStream_t s) {
     if (capacity == 0) return;
-    if (a.one && !a.any_hit && block == 256 && lds > 8 && lds <= 12) {
+    if (a.loop.one && !a.loop.any_hit && block == 256 && lds > 8 && lds <= 12) {
         shadow_one(a, capacity, s);
         return;
     }
-    if (a.any_hit) dispatch_shadow<true>(a, capacity, lds, block, s);
+    if (a.loop.any_hit) dispatch_shadow<true>(a, capacity, lds, block, s);
     else dispatch_shadow<false>(a, capacity, lds, block, s);
 }
 

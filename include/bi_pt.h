@@ -670,13 +670,10 @@ bi_pt_status bi_pt_trace_closest(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* r
                                  uint32_t* hit_triangle, float* hit_u, float* hit_v, bi_pt_stream stream);
 /* bi_pt_trace_closest for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart
- * in the reference.  Same arguments and results; its scratch (job record, part counters,
- * one 16-B hit record per ray) is a static device array of the library (4 MiB + 3 KiB,
- * held by each GPU the library runs on until the process ends), so at most
- * BI_PT_NOALLOC_MAX_RAYS rays per call (more: INVALID_ARGUMENT), and it builds nothing:
- * the scene's LBVH must be current (rendered or queried since the scene last changed;
- * else UNSUPPORTED).  Calls on one GPU share the scratch: calls that overlap on one GPU
- * race, so serialise them (for example on one stream). */
+ * in the reference.  Same arguments and results.  Neither call needs scratch once the
+ * scene's LBVH is built; this one also builds nothing: the LBVH must be current (rendered
+ * or queried since the scene last changed; else UNSUPPORTED).  At most
+ * BI_PT_NOALLOC_MAX_RAYS rays per call (more: INVALID_ARGUMENT). */
 #define BI_PT_NOALLOC_MAX_RAYS (1u << 18)
 bi_pt_status bi_pt_trace_closest_noalloc(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* rays, float tmax,
                                          float* hit_t, uint32_t* hit_triangle, float* hit_u, float* hit_v,

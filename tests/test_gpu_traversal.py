@@ -1,7 +1,7 @@
 """Closest-hit and occlusion queries on trees and rays at the edges of the traversal's node
 format, against the restatement, bit for bit: trees of one to a few nodes, scenes far from
 the origin and of extreme size, rays along an axis, from a face, and rays that are no
-numbers; query sizes around a wavefront and a workgroup."""
+numbers; query sizes around a wavefront, a workgroup and more than the chip holds at once."""
 import dataclasses
 
 import numpy as np
@@ -40,7 +40,7 @@ def edge_rays(rng, n, scale, shift):
 
 @pytest.mark.parametrize("tris,rays,scale,shift", [
     (1, 64, 1.0, 0.0), (2, 65, 1.0, 0.0), (3, 1, 1.0, 0.0), (5, 257, 1.0, 0.0), (8, 63, 1.0, 0.0), (300, 20000, 1.0, 0.0),
-    (300, 20000, 1.0, 4e4), (300, 20000, 1e6, 0.0), (300, 20000, 1e11, 3e12), (4000, 70001, 1.0, 100.0),
+    (300, 20000, 1.0, 4e4), (300, 20000, 1e6, 0.0), (300, 20000, 1e11, 3e12), (4000, 70001, 1.0, 100.0), (40, 600001, 1.0, 0.0),
 ])
 def test_queries_match_restatement(oracle_lib, tris, rays, scale, shift):
     print(f"case: {tris} triangles x {scale:g} + {shift:g}, {rays} rays", flush=True)
