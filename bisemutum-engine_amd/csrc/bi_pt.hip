@@ -192,7 +192,7 @@ QueryArgs query_args(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* rays, float t
     a.bvh = bvh_view(ctx);
     if (ctx->num_tris == 0) a.bvh.nodes = ctx->eng.empty_tree.p;
     a.q = RayQueue{const_cast<float*>(rays->ox), const_cast<float*>(rays->oy), const_cast<float*>(rays->oz),
-                   const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz), nullptr};
+                   const_cast<float*>(rays->dx), const_cast<float*>(rays->dy), const_cast<float*>(rays->dz), nullptr, nullptr};
     a.count = n;
     a.tmax = tmax;
     a.loop.parts = kWorkParts;

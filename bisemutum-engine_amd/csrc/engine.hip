@@ -48,13 +48,13 @@ bi_pt_status engine_init(Owner* own, Engine& eng) {
 
 void engine_free(Owner* own, Engine& eng) {
     for (int k = 0; k < 6; ++k) { dfree(own, eng.qa[k]); dfree(own, eng.qb[k]); }
-    for (int k = 0; k < 4; ++k) dfree(own, eng.ps_f[k]);
     for (int t = 0; t < 2; ++t) {
-        for (int k = 0; k < 9; ++k) dfree(own, eng.sq_f[t][k]);
-        dfree(own, eng.sq_pk[t]);
+        for (int k = 0; k < 6; ++k) dfree(own, eng.sq_f[t][k]);
+        dfree(own, eng.sq_cp[t]);
     }
     dfree(own, eng.acc);
     dfree(own, eng.qa_path); dfree(own, eng.qb_path);
+    dfree(own, eng.qa_beta); dfree(own, eng.qb_beta);
     dfree(own, eng.hit_rec); dfree(own, eng.tile_state);
     dfree(own, eng.counters); dfree(own, eng.plan); dfree(own, eng.empty_tree);
     if (eng.ready) {
@@ -152,9 +152,9 @@ uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult) {
     uint64_t b = 0;
     b += 12 * c * 4 + 2 * c * 4;                 // queues A and B: 6 floats + path id each
     b += c * sizeof(HitRec);                     // hit records
-    b += 4 * c * 4;                              // path state
-    b += (uint64_t)slots * 3 * c * 4;            // radiance accumulators
-    b += 2 * (uint64_t)sh_mult * c * (9 * 4 + 4);   // two shadow queue sets
+    b += 2 * c * 16;                             // throughput and pdf of queues A and B
+    b += (uint64_t)slots * c * 16;               // radiance accumulators
+    b += 2 * (uint64_t)sh_mult * c * (6 * 4 + 16);   // two shadow queue sets
     b += tiles * 8;                              // look-back words of the shade tiles
     return b;
 }
@@ -173,12 +173,13 @@ bi_pt_status ensure_wave_buffers(Owner* own, Engine& eng, uint32_t cap, uint32_t
     BI_TRY(dalloc(own, eng.qa_path, cap));
     BI_TRY(dalloc(own, eng.qb_path, cap));
     BI_TRY(dalloc(own, eng.hit_rec, cap));
-    for (int k = 0; k < 4; ++k) BI_TRY(dalloc(own, eng.ps_f[k], cap));
-    BI_TRY(dalloc(own, eng.acc, (size_t)slots * 3u * cap));
+    BI_TRY(dalloc(own, eng.qa_beta, cap));
+    BI_TRY(dalloc(own, eng.qb_beta, cap));
+    BI_TRY(dalloc(own, eng.acc, (size_t)slots * cap));
     const size_t shcap = (size_t)cap * sh_mult;
     for (int t = 0; t < 2; ++t) {
-        for (int k = 0; k < 9; ++k) BI_TRY(dalloc(own, eng.sq_f[t][k], shcap));
-        BI_TRY(dalloc(own, eng.sq_pk[t], shcap));
+        for (int k = 0; k < 6; ++k) BI_TRY(dalloc(own, eng.sq_f[t][k], shcap));
+        BI_TRY(dalloc(own, eng.sq_cp[t], shcap));
     }
     BI_TRY(dalloc(own, eng.tile_state, (cap + 255u) / 256u + 1u));
     eng.wave_cap = cap;
@@ -187,8 +188,8 @@ bi_pt_status ensure_wave_buffers(Owner* own, Engine& eng, uint32_t cap, uint32_t
     return BI_PT_OK;
 }
 
-RayQueue queue_of(DevBuf<float>* f, DevBuf<uint32_t>& path) {
-    return RayQueue{f[0].p, f[1].p, f[2].p, f[3].p, f[4].p, f[5].p, path.p};
+RayQueue queue_of(DevBuf<float>* f, DevBuf<uint32_t>& path, DevBuf<float4>& beta) {
+    return RayQueue{f[0].p, f[1].p, f[2].p, f[3].p, f[4].p, f[5].p, path.p, beta.p};
 }
 
 // Per-job facts of a call.
@@ -617,13 +618,13 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
             BI_HIP_TRY(own, hipMemcpyAsync(nrc->bounds.p, prep[0].scene->cb_out.p, 6 * sizeof(float),
                                            hipMemcpyDeviceToDevice, s));
 
-        PathState ps{eng.ps_f[0].p, eng.ps_f[1].p, eng.ps_f[2].p, eng.ps_f[3].p, eng.acc.p, eng.wave_cap};
+        PathState ps{eng.acc.p, eng.wave_cap};
         HitBuf hits{eng.hit_rec.p};
-        RayQueue qA = queue_of(eng.qa, eng.qa_path), qB = queue_of(eng.qb, eng.qb_path);
+        RayQueue qA = queue_of(eng.qa, eng.qa_path, eng.qa_beta), qB = queue_of(eng.qb, eng.qb_path, eng.qb_beta);
         ShadowQueue sqs[2];
         for (int t = 0; t < 2; ++t)
             sqs[t] = ShadowQueue{eng.sq_f[t][0].p, eng.sq_f[t][1].p, eng.sq_f[t][2].p, eng.sq_f[t][3].p, eng.sq_f[t][4].p,
-                                 eng.sq_f[t][5].p, eng.sq_f[t][6].p, eng.sq_f[t][7].p, eng.sq_f[t][8].p, eng.sq_pk[t].p};
+                                 eng.sq_f[t][5].p, eng.sq_cp[t].p};
         // shadow launches overlap the next segment's closest hit, except when timing kernel
         // classes, recording queues, or training the cache (whose reset of a training path's
         // accumulators at the cache segment must follow the earlier shadow additions)
@@ -736,6 +737,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                     na.fwd = nrc->fwd.p;
                     na.bounds = nrc->bounds.p;
                     na.ps = ps;
+                    na.beta = primary ? nullptr : qin.beta;
                     launch_nrc_infer(na, s);
                 }
 
@@ -773,8 +775,9 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                     const uint32_t next = hc[(b & 1u) ? kCntExtB : kCntExtA];
                     auto& shq = eng.rec_sh.back()[b];
                     shq.resize(hc[kCntShadow]);
-                    if (!shq.empty())
-                        BI_HIP_TRY(own, hipMemcpy(shq.data(), eng.sq_pk[0].p, shq.size() * 4, hipMemcpyDeviceToHost));
+                    if (!shq.empty())   // the fourth word of each contribution record
+                        BI_HIP_TRY(own, hipMemcpy2D(shq.data(), 4, &eng.sq_cp[0].p->w, 16, 4, shq.size(),
+                                                    hipMemcpyDeviceToHost));
                     if (b + 1 < D) {
                         auto& ex = eng.rec_ext.back()[b + 1];
                         ex.resize(next);

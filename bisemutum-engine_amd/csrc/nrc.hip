@@ -185,7 +185,6 @@ __global__ __launch_bounds__(256) void k_nrc_infer(NrcInferArgs a) {
     f32x4 o[4];
     output_layer(fwd, X, o, lane);
     if (lane < 16) {
-        const size_t cap = a.ps.cap;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t row = 16u * r + (uint32_t)lane;
@@ -199,12 +198,10 @@ __global__ __launch_bounds__(256) void k_nrc_infer(NrcInferArgs a) {
             }
             const uint32_t path = s_tag[wave][row];
             if (path == kNoPath) continue;
-            V3 c = v3(a.ps.bx[path] * fmaxf(o[r][0], 0.0f), a.ps.by[path] * fmaxf(o[r][1], 0.0f),
-                      a.ps.bz[path] * fmaxf(o[r][2], 0.0f));
+            const float4 b = a.beta ? a.beta[e] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+            V3 c = v3(b.x * fmaxf(o[r][0], 0.0f), b.y * fmaxf(o[r][1], 0.0f), b.z * fmaxf(o[r][2], 0.0f));
             if (!finite3(c)) c = v3(0.0f, 0.0f, 0.0f);
-            a.ps.acc[path] = c.x;
-            a.ps.acc[cap + path] = c.y;
-            a.ps.acc[2 * cap + path] = c.z;
+            a.ps.acc[path] = make_float4(c.x, c.y, c.z, 0.0f);
         }
     }
 }

@@ -93,8 +93,9 @@ struct Knobs {
 // Queues and per-wave buffers, sized for the largest wave rendered so far.
 struct Engine {
     uint32_t wave_cap = 0, wave_slots = 0, wave_sh_mult = 0;
-    DevBuf<float> qa[6], qb[6], ps_f[4], acc, sq_f[2][9];
-    DevBuf<uint32_t> qa_path, qb_path, sq_pk[2];
+    DevBuf<float> qa[6], qb[6], sq_f[2][6];
+    DevBuf<float4> qa_beta, qb_beta, acc, sq_cp[2];
+    DevBuf<uint32_t> qa_path, qb_path;
     DevBuf<HitRec> hit_rec;
     DevBuf<uint64_t> tile_state;           // look-back words of the shade launch's tiles
     DevBuf<uint32_t> counters;             // kCntSlots (ray counters at kCntRays as 4 x u64)

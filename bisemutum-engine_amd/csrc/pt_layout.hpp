@@ -14,8 +14,9 @@
 //              material) and, where needed, leaf texture coordinates (32 B) and tangents
 //              (48 B) in sorted leaf order
 //   per wave   SoA ray queues (o.xyz, d.xyz, path id), 16-B hit records (t, leaf, u, v),
-//              SoA path state (throughput, last BSDF pdf), per-kind radiance accumulators,
-//              SoA shadow queue (o.xyz, d.xyz, contribution.xyz, path<<3|kind)
+//              throughput and last BSDF pdf (16 B, in queue order), per-kind radiance
+//              accumulators (16 B), shadow queues (SoA o.xyz, d.xyz; 16 B contribution.xyz and
+//              path<<3|kind)
 // Nodes are read whole by one lane (4 x 16-B loads); rays, hits and path state are
 // read by consecutive lanes at consecutive addresses (coalesced).
 #pragma once
@@ -307,10 +308,13 @@ struct JobRec {
     SceneTex rect_tex_levels;     // their mip levels: level records, texel pool, sRGB table
 };
 
-// Ray queue in SoA form.
+// Ray queue: origins, directions and path ids in SoA form (read together, by consecutive
+// lanes), and each path's throughput xyz and last BSDF pdf, which travel with its ray so that
+// the shading reads them in queue order too.
 struct RayQueue {
     float *ox, *oy, *oz, *dx, *dy, *dz;
     uint32_t* path;
+    float4* beta;
 };
 // Hit record of one ray, one 16-B store: a lane finishes its ray at its own time, so
 // the records of a wavefront land scattered; one record per ray keeps that to one
@@ -324,14 +328,19 @@ struct HitBuf {
     HitRec* rec;
 };
 // A shadow ray's direction is stored for sky rays only; a light's ray takes it from the
-// light (a directional light's direction, or from the origin towards a point light).
+// light (a directional light's direction, or from the origin towards a point light).  The
+// contribution xyz and the word path << 3 | kind are one 16-B record: a finished ray's lane
+// reads them alone, out of step with its neighbours (as with HitRec), and a wavefront's
+// finish then looks up one cache line per lane instead of four.
 struct ShadowQueue {
-    float *ox, *oy, *oz, *dx, *dy, *dz, *cx, *cy, *cz;
-    uint32_t* pk;   // path << 3 | kind
+    float *ox, *oy, *oz, *dx, *dy, *dz;
+    float4* cp;
 };
+__device__ __forceinline__ uint32_t shadow_pk(const float4& cp) { return __float_as_uint(cp.w); }
+// Radiance accumulators [kind][cap] by path, xyz (16 B each: the scattered additions of the
+// shadow kernel and the misses are one load and one store).
 struct PathState {
-    float *bx, *by, *bz, *pdf;
-    float* acc;       // [kind][3][cap]
+    float4* acc;
     uint32_t cap;
 };
 

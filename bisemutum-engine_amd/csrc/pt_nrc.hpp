@@ -32,7 +32,8 @@ struct NrcInferArgs {
     uint32_t num;               // launch capacity
     const void* fwd;            // forward fragments (bf16)
     const float* bounds;        // scene box: lo xyz, hi xyz
-    PathState ps;               // radiance kind 0 and throughput of the queried paths
+    PathState ps;               // radiance kind 0 of the queried paths
+    const float4* beta;         // throughput per entry (null: camera rays, one)
     float* raw_out;             // non-null: raw network outputs, 3 per entry (all entries)
 };
 void launch_nrc_infer(const NrcInferArgs& a, hipStream_t s);

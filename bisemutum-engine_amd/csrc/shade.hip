@@ -43,6 +43,7 @@ template <uint32_t NL>
 struct ShadeOut {
     uint32_t mask = 0, path = 0;
     V3 P, ext, sky;
+    float4 beta;
     V3 c[NL + 1];   // shadow contribution of light l at [l], of the sky at [NL]
 };
 
@@ -130,16 +131,14 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         beta = v3(1.0f, 1.0f, 1.0f);
         pdf_prev = 0.0f;
         for (uint32_t k = 0; k < nslots; ++k) {
-            float* acc = a.ps.acc + (size_t)k * 3u * cap;
-            acc[path] = 0.0f;
-            acc[cap + path] = 0.0f;
-            acc[2 * cap + path] = 0.0f;
+            a.ps.acc[k * cap + path] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
     } else {
         o = v3(a.qin.ox[i], a.qin.oy[i], a.qin.oz[i]);
         d = v3(a.qin.dx[i], a.qin.dy[i], a.qin.dz[i]);
-        beta = v3(a.ps.bx[path], a.ps.by[path], a.ps.bz[path]);
-        pdf_prev = a.ps.pdf[path];
+        const float4 b = a.qin.beta[i];
+        beta = v3(b.x, b.y, b.z);
+        pdf_prev = b.w;
     }
     const HitRec hit = a.hits.rec[i];
     const uint32_t leaf = hit.leaf;
@@ -149,9 +148,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         float w = 1.0f;
         if (!primary && J.sky_nee) w = power_heuristic(pdf_prev, sky_pdf(J.sky, d));
         V3 c = (beta * ls) * w;
-        a.ps.acc[path] = c.x;
-        a.ps.acc[cap + path] = c.y;
-        a.ps.acc[2 * cap + path] = c.z;
+        a.ps.acc[path] = make_float4(c.x, c.y, c.z, 0.0f);
         if (want_depth) J.depth_out[pixel] = 0.0f;
     } else {
         const float t = hit.t, hu = hit.u, hv = hit.v;
@@ -185,10 +182,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             J.cache_rec[key.q] = r;
             beta = v3(1.0f, 1.0f, 1.0f);
             for (uint32_t k = 0; k < nslots; ++k) {
-                float* acc = a.ps.acc + (size_t)k * 3u * cap;
-                acc[path] = 0.0f;
-                acc[cap + path] = 0.0f;
-                acc[2 * cap + path] = 0.0f;
+                a.ps.acc[k * cap + path] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             }
         }
         Frame fr = make_frame(N);
@@ -204,10 +198,9 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             V3 c = (le * f) * beta;
             if (!any_pos(c)) continue;
             if (L.sm_index < 0) {
-                float* acc = a.ps.acc + (size_t)(l + 1u) * 3u * cap;
-                acc[path] = acc[path] + c.x;
-                acc[cap + path] = acc[cap + path] + c.y;
-                acc[2 * cap + path] = acc[2 * cap + path] + c.z;
+                float4* acc = a.ps.acc + (l + 1u) * cap + path;
+                const float4 s = *acc;
+                *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
                 continue;
             }
             out.c[l] = c;
@@ -217,13 +210,12 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         // lighting times the throughput added in light order to the slot after the sky's
         if constexpr (RECT) {
             if (J.num_rects) {
-                float* acc = a.ps.acc + (size_t)(nl + 2u) * 3u * cap;
-                V3 sum = v3(acc[path], acc[cap + path], acc[2 * cap + path]);
+                float4* acc = a.ps.acc + (nl + 2u) * cap + path;
+                const float4 s = *acc;
+                V3 sum = v3(s.x, s.y, s.z);
                 for (uint32_t r = 0; r < J.num_rects; ++r)
                     sum = sum + rect_light_lit(J.rects[r], J.ltc, J.rect_tex, J.rect_tex_levels, P, fr, V, m) * beta;
-                acc[path] = sum.x;
-                acc[cap + path] = sum.y;
-                acc[2 * cap + path] = sum.z;
+                *acc = make_float4(sum.x, sum.y, sum.z, 0.0f);
             }
         }
         // sky NEE only where the next segment is sampled too (the reference sees the
@@ -260,8 +252,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             V3 nb = beta * w;
             if (max3(nb) > 0.0f) {
                 out.ext = Lext;
-                a.ps.bx[path] = nb.x; a.ps.by[path] = nb.y; a.ps.bz[path] = nb.z;
-                a.ps.pdf[path] = pdf;
+                out.beta = make_float4(nb.x, nb.y, nb.z, pdf);
                 mask |= kMaskExt;
             }
         }
@@ -286,6 +277,7 @@ __device__ __forceinline__ void emit_entry(const ShadeArgs& a, const ShadeOut<NL
         a.qout.ox[e] = out.P.x; a.qout.oy[e] = out.P.y; a.qout.oz[e] = out.P.z;
         a.qout.dx[e] = out.ext.x; a.qout.dy[e] = out.ext.y; a.qout.dz[e] = out.ext.z;
         a.qout.path[e] = out.path;
+        a.qout.beta[e] = out.beta;
     }
 #pragma unroll
     for (uint32_t k = 0; k <= NL; ++k) {
@@ -295,8 +287,8 @@ __device__ __forceinline__ void emit_entry(const ShadeArgs& a, const ShadeOut<NL
         if (sky) {   // a light's ray takes its direction from the light in the shadow kernel
             a.sq.dx[o] = out.sky.x; a.sq.dy[o] = out.sky.y; a.sq.dz[o] = out.sky.z;
         }
-        a.sq.cx[o] = out.c[k].x; a.sq.cy[o] = out.c[k].y; a.sq.cz[o] = out.c[k].z;
-        a.sq.pk[o] = (out.path << 3) | (sky ? kKindSky : k);
+        a.sq.cp[o] = make_float4(out.c[k].x, out.c[k].y, out.c[k].z,
+                                 __uint_as_float((out.path << 3) | (sky ? kKindSky : k)));
         ++o;
     }
 }
@@ -455,8 +447,8 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a) {
         const size_t p = (size_t)pbase + (size_t)s * npix + q;
         V3 r = v3(0.f, 0.f, 0.f);
         for (uint32_t k = 0; k < nslots; ++k) {
-            const float* acc = a.ps.acc + (size_t)k * 3u * cap;
-            V3 c = v3(acc[p], acc[cap + p], acc[2 * cap + p]);
+            const float4 v = a.ps.acc[k * cap + p];
+            V3 c = v3(v.x, v.y, v.z);
             r = k == 0 ? c : r + c;
         }
         sum = sum + r;

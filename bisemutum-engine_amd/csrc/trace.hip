@@ -578,8 +578,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AH ? 5 : 6)
 
 // Adds shadow ray i's contribution unless it is occluded; returns whether it is a sky ray.
 __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bool occ) {
-    const uint32_t pk = a.q.pk[i];
-    const uint32_t path = pk >> 3, kind = pk & 7u;
+    const float4 cp = a.q.cp[i];
+    const uint32_t pk = shadow_pk(cp), path = pk >> 3, kind = pk & 7u;
     float keep = 1.0f;
     uint32_t nl;
     if (a.jobs.num_jobs == 1u) {   // uniform record address: scalar loads
@@ -590,18 +590,16 @@ __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bo
         nl = J.num_lights;
         if (occ && kind != kKindSky) keep = J.keep[kind];
     }
-    V3 c = v3(a.q.cx[i], a.q.cy[i], a.q.cz[i]);
+    V3 c = v3(cp.x, cp.y, cp.z);
     if (occ) {
         if (kind == kKindSky) return true;
         if (!(keep > 0.0f)) return false;
         c = c * keep;
     }
     const uint32_t slot = kind == kKindSky ? nl + 1u : kind + 1u;
-    const size_t cap = a.ps.cap;
-    float* acc = a.ps.acc + (size_t)slot * 3u * cap;
-    acc[path] = acc[path] + c.x;
-    acc[cap + path] = acc[cap + path] + c.y;
-    acc[2 * cap + path] = acc[2 * cap + path] + c.z;
+    float4* acc = a.ps.acc + (size_t)slot * a.ps.cap + path;
+    const float4 s = *acc;
+    *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
     return kind == kKindSky;
 }
 
@@ -617,7 +615,7 @@ struct ShadowRays {
     // unbounded).
     template <bool AH, bool ONE>
     __device__ __forceinline__ const JobRec* start(uint32_t i, V3& o, V3& d, float& tmax) const {
-        const uint32_t pk = a.q.pk[i], kind = pk & 7u;
+        const uint32_t pk = shadow_pk(a.q.cp[i]), kind = pk & 7u;
         const JobRec& J = ONE || a.jobs.num_jobs == 1u ? a.jobs.rec[0]
                                                        : a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, pk >> 3)];
         o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
