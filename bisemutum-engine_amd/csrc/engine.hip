@@ -361,9 +361,13 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
 
     // non-opaque triangles anywhere in the call select the traversal kernels with any-hit tests
     bool any_hit = false, any_point = false;   // point lights: shadow rays of finite extent
+    bool any_keep = false;                     // lights that an occluder does not hide entirely
     for (uint32_t j = 0; j < n; ++j) {
         any_hit = any_hit || prep[j].scene->non_opaque;
-        for (const LightRec& L : prep[j].scene->lights) any_point = any_point || L.type == kLightPoint;
+        for (const LightRec& L : prep[j].scene->lights) {
+            any_point = any_point || L.type == kLightPoint;
+            any_keep = any_keep || 1.0f - L.shadow_strength > 0.0f;
+        }
     }
 
     // device memory: per-job images, BVH builds, wave buffers, plan
@@ -587,7 +591,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
     std::vector<uint64_t> key;
     if (graph) {
         key = {n, cap, lds_stack, refill, parts, block, (uint64_t)(uintptr_t)eng.plan.p, eng.wave_cap, eng.wave_slots,
-               eng.wave_sh_mult, plan_bytes, (uint64_t)any_hit, (uint64_t)any_point};
+               eng.wave_sh_mult, plan_bytes, (uint64_t)any_hit, (uint64_t)any_point, (uint64_t)any_keep};
         for (uint32_t j = 0; j < n; ++j) {
             const Prep& p = prep[j];
             key.insert(key.end(), {(uint64_t)(uintptr_t)p.ctx, (uint64_t)(uintptr_t)p.scene,
@@ -749,6 +753,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 sha.count_in = cnt_sh;
                 sha.ps = ps;
                 sha.ray_counters = rays;
+                sha.any_keep = any_keep ? 1u : 0u;
                 sha.loop.work = shadow_work;
                 sha.loop.parts = parts;
                 sha.loop.refill = refill;

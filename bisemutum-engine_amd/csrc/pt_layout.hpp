@@ -337,8 +337,10 @@ struct ShadowQueue {
     float4* cp;
 };
 __device__ __forceinline__ uint32_t shadow_pk(const float4& cp) { return __float_as_uint(cp.w); }
-// Radiance accumulators [kind][cap] by path, xyz (16 B each: the scattered additions of the
-// shadow kernel and the misses are one load and one store).
+// Radiance accumulators [slot][cap] by path, xyz (16 B each: the scattered additions of the
+// shadow kernel and the misses are one load and one store).  A kind's slot does not depend
+// on the job's number of lights, so the shadow kernel needs no job to find it.
+constexpr uint32_t kSlotMiss = 0u, kSlotSky = 1u, kSlotLights = 2u;   // light l: kSlotLights + l; rect lights after them
 struct PathState {
     float4* acc;
     uint32_t cap;

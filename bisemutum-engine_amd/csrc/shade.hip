@@ -198,7 +198,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             V3 c = (le * f) * beta;
             if (!any_pos(c)) continue;
             if (L.sm_index < 0) {
-                float4* acc = a.ps.acc + (l + 1u) * cap + path;
+                float4* acc = a.ps.acc + (kSlotLights + l) * cap + path;
                 const float4 s = *acc;
                 *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
                 continue;
@@ -210,7 +210,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         // lighting times the throughput added in light order to the slot after the sky's
         if constexpr (RECT) {
             if (J.num_rects) {
-                float4* acc = a.ps.acc + (nl + 2u) * cap + path;
+                float4* acc = a.ps.acc + (kSlotLights + nl) * cap + path;
                 const float4 s = *acc;
                 V3 sum = v3(s.x, s.y, s.z);
                 for (uint32_t r = 0; r < J.num_rects; ++r)
@@ -343,16 +343,11 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a) {
     if (tile >= ntiles) return;
     const uint32_t i = tile * kTile + tid;
     ShadeOut<NL> out;
-    const JobRec* J = a.jobs.rec;
     if (i < count) {
         const uint32_t path = primary ? i : a.qin.path[i];
-        if (a.jobs.num_jobs == 1u) {
-            shade_entry<NL, RECT>(a, a.jobs.rec[0], i, path, path, primary, out);   // uniform record: scalar loads
-        } else {
-            const uint32_t jid = job_of(a.jobs.path_base, a.jobs.num_jobs, path);
-            J = a.jobs.rec + jid;
-            shade_entry<NL, RECT>(a, *J, i, path, path - a.jobs.path_base[jid], primary, out);
-        }
+        with_job<false>(a.jobs, path, [&](const JobRec& J, uint32_t local) {
+            shade_entry<NL, RECT>(a, J, i, path, local, primary, out);
+        });
     }
     // the tile's emissions: (extension << 16 | shadow) per entry, scanned in entry order
     const uint32_t packed = ((out.mask & kMaskExt) << 16) | (uint32_t)__popc(out.mask >> 1);
@@ -437,7 +432,6 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a) {
     const uint32_t npix = J.npix;
     // a training job's slot q sums into target q
     const uint32_t pixel = (J.flags & kJobTrain) ? q : pixel_of(q, J.cam.width, J.cam.height);
-    const uint32_t nslots = J.num_lights + 2u + (J.num_rects ? 1u : 0u);
     const uint32_t samples = J.samples;
     const uint32_t pbase = a.jobs.path_base[jid];
     float* sums = J.sums;
@@ -445,12 +439,14 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a) {
     V3 sum = v3(sums[3 * (size_t)pixel], sums[3 * (size_t)pixel + 1], sums[3 * (size_t)pixel + 2]);
     for (uint32_t s = 0; s < samples; ++s) {
         const size_t p = (size_t)pbase + (size_t)s * npix + q;
-        V3 r = v3(0.f, 0.f, 0.f);
-        for (uint32_t k = 0; k < nslots; ++k) {
+        auto slot = [&](uint32_t k) {
             const float4 v = a.ps.acc[k * cap + p];
-            V3 c = v3(v.x, v.y, v.z);
-            r = k == 0 ? c : r + c;
-        }
+            return v3(v.x, v.y, v.z);
+        };
+        V3 r = slot(kSlotMiss);
+        for (uint32_t l = 0; l < J.num_lights; ++l) r = r + slot(kSlotLights + l);
+        r = r + slot(kSlotSky);
+        if (J.num_rects) r = r + slot(kSlotLights + J.num_lights);
         sum = sum + r;
     }
     sums[3 * (size_t)pixel] = sum.x;

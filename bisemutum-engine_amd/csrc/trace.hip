@@ -383,33 +383,29 @@ struct PathRays {
     const TraceArgs& a;
     __device__ __forceinline__ uint32_t count() const { return PRIMARY ? a.jobs.num_paths : *a.count_in; }
     __device__ __forceinline__ const JobRec* scene() const { return a.jobs.rec; }
-    // one job: its record sits at a uniform address (scalar loads); several: the path's job
-    // is looked up per lane
     template <bool ONE>
     __device__ __forceinline__ const JobRec* start(uint32_t i, V3& o, V3& d, float& tmax) const {
-        const JobRec* J = a.jobs.rec;
-        uint32_t local = i;
-        if (!ONE && a.jobs.num_jobs != 1u) {
-            const uint32_t path = PRIMARY ? i : a.q.path[i];
-            const uint32_t jid = job_of(a.jobs.path_base, a.jobs.num_jobs, path);
-            J = a.jobs.rec + jid;
-            local = path - a.jobs.path_base[jid];
-        }
-        tmax = J->ray_length;
-        if constexpr (PRIMARY) {
-            const PathKey k = path_key(*J, local);
-            float jx = 0.5f, jy = 0.5f;
-            if (J->flags & 1u) {
-                Pcg jr = pcg_keyed(J->seed, k.pixel, k.sample, kJitterBounce);
-                jx = pcg_float(jr);
-                jy = pcg_float(jr);
+        const uint32_t path = PRIMARY || ONE || a.jobs.num_jobs == 1u ? i : a.q.path[i];
+        const JobRec* rec = nullptr;
+        with_job<ONE>(a.jobs, path, [&](const JobRec& J, uint32_t local) {
+            rec = &J;
+            tmax = J.ray_length;
+            if constexpr (PRIMARY) {
+                const PathKey k = path_key(J, local);
+                float jx = 0.5f, jy = 0.5f;
+                if (J.flags & 1u) {
+                    Pcg jr = pcg_keyed(J.seed, k.pixel, k.sample, kJitterBounce);
+                    jx = pcg_float(jr);
+                    jy = pcg_float(jr);
+                }
+                camera_ray(J.cam, k.pixel % J.cam.width, k.pixel / J.cam.width, jx, jy, &o, &d);
             }
-            camera_ray(J->cam, k.pixel % J->cam.width, k.pixel / J->cam.width, jx, jy, &o, &d);
-        } else {
+        });
+        if constexpr (!PRIMARY) {
             o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
             d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
         }
-        return J;
+        return rec;
     }
     __device__ __forceinline__ void finish(uint32_t i, HitRec h) const { a.hits.rec[i] = h; }
 };
@@ -562,7 +558,7 @@ __device__ __forceinline__ void trace_closest_body(const S& src, const TraceLoop
 }
 
 template <bool PRIMARY, bool AH, int L, int B>
-__global__ __launch_bounds__(B) void k_trace_closest(TraceArgs a) {
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(AH ? 4 : 6))) void k_trace_closest(TraceArgs a) {
     trace_closest_body<AH, L, B, false>(PathRays<PRIMARY>{a}, a.loop);
 }
 // One job, opaque scene, 256-thread blocks and a 12-deep LDS stack (the defaults): the
@@ -580,23 +576,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AH ? 5 : 6)
 __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bool occ) {
     const float4 cp = a.q.cp[i];
     const uint32_t pk = shadow_pk(cp), path = pk >> 3, kind = pk & 7u;
-    float keep = 1.0f;
-    uint32_t nl;
-    if (a.jobs.num_jobs == 1u) {   // uniform record address: scalar loads
-        nl = a.jobs.rec[0].num_lights;
-        if (occ && kind != kKindSky) keep = a.jobs.rec[0].keep[kind];
-    } else {
-        const JobRec& J = a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, path)];
-        nl = J.num_lights;
-        if (occ && kind != kKindSky) keep = J.keep[kind];
-    }
     V3 c = v3(cp.x, cp.y, cp.z);
     if (occ) {
         if (kind == kKindSky) return true;
+        if (!a.any_keep) return false;   // no light of the launch shines through its shadow
+        const uint32_t job = a.jobs.num_jobs == 1u ? 0u : job_of(a.jobs.path_base, a.jobs.num_jobs, path);
+        const float keep = a.jobs.rec[job].keep[kind];
         if (!(keep > 0.0f)) return false;
         c = c * keep;
     }
-    const uint32_t slot = kind == kKindSky ? nl + 1u : kind + 1u;
+    const uint32_t slot = kind == kKindSky ? kSlotSky : kSlotLights + kind;
     float4* acc = a.ps.acc + (size_t)slot * a.ps.cap + path;
     const float4 s = *acc;
     *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
@@ -616,19 +605,21 @@ struct ShadowRays {
     template <bool AH, bool ONE>
     __device__ __forceinline__ const JobRec* start(uint32_t i, V3& o, V3& d, float& tmax) const {
         const uint32_t pk = shadow_pk(a.q.cp[i]), kind = pk & 7u;
-        const JobRec& J = ONE || a.jobs.num_jobs == 1u ? a.jobs.rec[0]
-                                                       : a.jobs.rec[job_of(a.jobs.path_base, a.jobs.num_jobs, pk >> 3)];
         o = v3(a.q.ox[i], a.q.oy[i], a.q.oz[i]);
         tmax = kShadowTMax;
-        if (kind == kKindSky) {
-            d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
-        } else if constexpr (AH) {
-            light_shadow_ray(J.lights[kind], o, &d, &tmax);
-        } else {
-            const LightRec& Lk = J.lights[kind];
-            d = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
-        }
-        return &J;
+        const JobRec* rec = nullptr;
+        with_job<ONE>(a.jobs, pk >> 3, [&](const JobRec& J, uint32_t) {
+            rec = &J;
+            if (kind == kKindSky) {
+                d = v3(a.q.dx[i], a.q.dy[i], a.q.dz[i]);
+            } else if constexpr (AH) {
+                light_shadow_ray(J.lights[kind], o, &d, &tmax);
+            } else {
+                const LightRec& Lk = J.lights[kind];
+                d = v3(Lk.direction[0], Lk.direction[1], Lk.direction[2]);
+            }
+        });
+        return rec;
     }
     __device__ __forceinline__ void finish_any(uint32_t i, bool occ) const { sky_rays += apply_shadow(a, i, occ) ? 1u : 0u; }
 };
@@ -768,7 +759,7 @@ __device__ __forceinline__ void trace_shadow(const ShadowArgs& a) {
 }
 
 template <bool AH, int L, int B>
-__global__ __launch_bounds__(B) void k_trace_shadow(ShadowArgs a) {
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(AH ? 5 : 6))) void k_trace_shadow(ShadowArgs a) {
     trace_shadow<AH, L, B, false>(a);
 }
 // One job, opaque scene, the default stack and block (as k_trace_closest_one).
