@@ -765,8 +765,16 @@ bi_pt_status bi_pt_set_ltc_luts(bi_pt_ctx* ctx, const float* matrix_lut0, const 
         if (!std::isfinite(v)) return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "non-finite LTC table entry");
     if (t == ctx->ltc_host) return BI_PT_OK;
     BI_HIP_TRY(ctx, hipSetDevice(ctx->device));
-    BI_TRY(dalloc(ctx, ctx->ltc, (size_t)4 * kLtcTexels));
-    BI_HIP_TRY(ctx, hipMemcpy(ctx->ltc.p, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice));
+    // on the device a texel's three rows lie together, a norm component in each one's last word
+    std::vector<float> packed((size_t)3 * kLtcTexels * 4);
+    for (uint32_t i = 0; i < kLtcTexels; ++i)
+        for (uint32_t k = 0; k < 3; ++k) {
+            float* p = &packed[((size_t)3 * i + k) * 4];
+            std::memcpy(p, m[k] + (size_t)4 * i, 3 * sizeof(float));
+            p[3] = k < 2 ? norm_lut[2 * i + k] : 0.0f;
+        }
+    BI_TRY(dalloc(ctx, ctx->ltc, (size_t)3 * kLtcTexels));
+    BI_HIP_TRY(ctx, hipMemcpy(ctx->ltc.p, packed.data(), packed.size() * sizeof(float), hipMemcpyHostToDevice));
     ctx->ltc_host.swap(t);
     if (!ctx->rects_host.empty()) {
         ctx->acc_count = 0;

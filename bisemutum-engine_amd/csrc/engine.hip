@@ -731,7 +731,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 sa.bounce = b;
                 const bool cache_now = wave_cached && b == nrc->cache_bounce;
                 sa.nrc_query = cache_now ? nrc->query.p : nullptr;
-                launch_shade(sa, J.num_paths, max_nl, wave_rect, s);
+                launch_shade(sa, J.num_paths, max_nl, s);
                 if (cache_now) {
                     // paths that ended in the cache at this segment: their radiance estimate
                     NrcInferArgs na{};
@@ -744,6 +744,9 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                     na.beta = primary ? nullptr : qin.beta;
                     launch_nrc_infer(na, s);
                 }
+                if (overlap) BI_HIP_TRY(own, hipEventRecord(eng.ev_shade, s));
+                if (wave_rect)   // beside the shadow rays where they have a stream of their own
+                    launch_shade_rect(RectArgs{J, qin, primary ? nullptr : cnt_in, hits, ps, b}, J.num_paths, s);
 
                 BI_TRY(mark(2));
 
@@ -762,7 +765,6 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
                 sha.loop.step_bound = ta.loop.step_bound;
                 sha.loop.error = &cnt[kCntError];
                 if (overlap) {   // fork: the shadow rays trace beside the next closest-hit launch
-                    BI_HIP_TRY(own, hipEventRecord(eng.ev_shade, s));
                     BI_HIP_TRY(own, hipStreamWaitEvent(eng.aux_s, eng.ev_shade, 0));
                     launch_trace_shadow(sha, J.num_paths * sh_mult, lds_stack, block, eng.aux_s);
                     BI_HIP_TRY(own, hipEventRecord(eng.ev_shadow[set], eng.aux_s));

@@ -455,23 +455,27 @@ PT_HD V4 lerp4(V4 a, V4 b, float t) {
     return V4{lerpf(a.x, b.x, t), lerpf(a.y, b.y, t), lerpf(a.z, b.z, t), lerpf(a.w, b.w, t)};
 }
 PT_HD V4 ld4(const float4* t, int i) { const float4 v = t[i]; return V4{v.x, v.y, v.z, v.w}; }
-// Trilinear sample of an 8 x 8 x 64 table (x fastest) at normalised (x, y, z).
-PT_HD V4 ltc_sample(const float4* t, float x, float y, float z) {
+// Trilinear sample of the packed 8 x 8 x 64 table (x fastest; a texel's three records
+// together) at normalised (x, y, z).
+PT_HD void ltc_sample(const float4* t, float x, float y, float z, V4 out[3]) {
     int x0, x1, y0, y1, z0, z1;
     float fx, fy, fz;
     ltc_axis(x, (int)kLtcSize, &x0, &x1, &fx);
     ltc_axis(y, (int)kLtcSize, &y0, &y1, &fy);
     ltc_axis(z, (int)kLtcDepth, &z0, &z1, &fz);
     const int s = (int)kLtcSize, s2 = s * s;
-    V4 e[2];
-#pragma unroll 1
-    for (int k = 0; k < 2; ++k) {   // the two depth slices, each bilinear in x and y
-        const int zo = s2 * (k ? z1 : z0);
-        const V4 c0 = lerp4(ld4(t, x0 + s * y0 + zo), ld4(t, x1 + s * y0 + zo), fx);
-        const V4 c1 = lerp4(ld4(t, x0 + s * y1 + zo), ld4(t, x1 + s * y1 + zo), fx);
-        e[k] = lerp4(c0, c1, fy);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        V4 e[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {   // the two depth slices, each bilinear in x and y
+            const int zo = s2 * (k ? z1 : z0);
+            const V4 c0 = lerp4(ld4(t, 3 * (x0 + s * y0 + zo) + r), ld4(t, 3 * (x1 + s * y0 + zo) + r), fx);
+            const V4 c1 = lerp4(ld4(t, 3 * (x0 + s * y1 + zo) + r), ld4(t, 3 * (x1 + s * y1 + zo) + r), fx);
+            e[k] = lerp4(c0, c1, fy);
+        }
+        out[r] = lerp4(e[0], e[1], fz);
     }
-    return lerp4(e[0], e[1], fz);
 }
 // The tables' transform and (norm, Fresnel) pair at table coordinate (u3, u2, u1, u0):
 // u0 (the major roughness) selects two groups of 8 depth slices, blended by its
@@ -484,25 +488,35 @@ PT_HD void ltc_fetch(const float4* ltc, float u3, float u2, float u1, float u0, 
     const float w = ws - ws_f;
     const float x = (u3 * 7.0f + 0.5f) / 8.0f, y = (u2 * 7.0f + 0.5f) / 8.0f;
     const float z1 = ((u1 * 7.0f + 8.0f * ws_f) + 0.5f) / 64.0f, z2 = ((u1 * 7.0f + 8.0f * ws_c) + 0.5f) / 64.0f;
+    V4 g[3], h[3];
+    ltc_sample(ltc, x, y, z1, g);
+    ltc_sample(ltc, x, y, z2, h);
     V3 r[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const V4 a = ltc_sample(ltc + k * (int)kLtcTexels, x, y, z1), b = ltc_sample(ltc + k * (int)kLtcTexels, x, y, z2);
-        r[k] = v3(lerpf(a.x, b.x, w), lerpf(a.y, b.y, w), lerpf(a.z, b.z, w));
-    }
+    for (int k = 0; k < 3; ++k)
+        r[k] = v3(lerpf(g[k].x, h[k].x, w), lerpf(g[k].y, h[k].y, w), lerpf(g[k].z, h[k].z, w));
     m->r0 = r[0]; m->r1 = r[1]; m->r2 = r[2];
-    const V4 n1 = ltc_sample(ltc + 3 * (int)kLtcTexels, x, y, z1), n2 = ltc_sample(ltc + 3 * (int)kLtcTexels, x, y, z2);
-    *bx = lerpf(n1.x, n2.x, w);
-    *by = lerpf(n1.y, n2.y, w);
+    *bx = lerpf(g[0].w, h[0].w, w);
+    *by = lerpf(g[1].w, h[1].w, w);
 }
+// a or b by value (?: on the records selects an address, which puts both in scratch memory)
+PT_HD V3 sel3(bool s, V3 a, V3 b) { return v3(s ? a.x : b.x, s ? a.y : b.y, s ? a.z : b.z); }
 PT_HD void quad_reverse(V3 q[4]) {
     const V3 a = q[0], b = q[1];
     q[0] = q[3]; q[1] = q[2]; q[2] = b; q[3] = a;
 }
 // get_ltc_matrix_and_brdf (lights.hlsl:203-255): the table coordinate of the view
 // direction and roughness, folded into the first quadrant of azimuth and the larger
-// roughness first, the transform unfolded by row flips; reflections reverse the quad.
-PT_HD void ltc_matrix_brdf(const float4* ltc, V3 lv, float rx, float ry, V3 q[4], M3* m, float* bx, float* by) {
+// roughness first, the transform unfolded by row flips; reflections reverse the quads.
+// The same for every light of a vertex, so it is made once for all of them.
+struct LtcView {
+    M3 mt, mi;      // the transform and its inverse
+    float bx, by;   // norm and Fresnel term
+    bool reverse;
+};
+PT_HD void ltc_view(const float4* ltc, V3 lv, float rx, float ry, LtcView* o) {
+    M3* m = &o->mt;
+    float *bx = &o->bx, *by = &o->by;
     const float theta = pt_acos(lv.z);
     const bool flip_r = ry > rx;
     float phi = pt_atan2(lv.y, lv.x);
@@ -511,27 +525,32 @@ PT_HD void ltc_matrix_brdf(const float4* ltc, V3 lv, float rx, float ry, V3 q[4]
     const float u0 = sel_max((flip_r ? ry : rx) - 0.001f, 0.0f) / (1.0f - 0.001f);
     const float u1 = flip_r ? rx / ry : ry / rx;
     const float u2 = theta / (kPi * 0.5f);
+    // the quadrant chooses the coordinate and the flips around one table fetch (a fetch in
+    // each of four branches is run four times by a wavefront that sees all quadrants)
+    float u3;
+    bool neg0 = false, neg1 = false, rev = false;
     if (phi < kPi * 0.5f) {
-        ltc_fetch(ltc, phi / (kPi * 0.5f), u2, u1, u0, m, bx, by);
+        u3 = phi / (kPi * 0.5f);
     } else if (phi < kPi) {
-        ltc_fetch(ltc, (kPi - phi) / (kPi * 0.5f), u2, u1, u0, m, bx, by);
-        quad_reverse(q);
-        m->r0 = -m->r0;
+        u3 = (kPi - phi) / (kPi * 0.5f);
+        neg0 = rev = true;
     } else if (phi < 1.5f * kPi) {
-        ltc_fetch(ltc, (phi - kPi) / (kPi * 0.5f), u2, u1, u0, m, bx, by);
-        m->r0 = -m->r0;
-        m->r1 = -m->r1;
+        u3 = (phi - kPi) / (kPi * 0.5f);
+        neg0 = neg1 = true;
     } else {
-        ltc_fetch(ltc, (2.0f * kPi - phi) / (kPi * 0.5f), u2, u1, u0, m, bx, by);
-        quad_reverse(q);
-        m->r1 = -m->r1;
+        u3 = (2.0f * kPi - phi) / (kPi * 0.5f);
+        neg1 = rev = true;
     }
+    ltc_fetch(ltc, u3, u2, u1, u0, m, bx, by);
+    if (neg0) m->r0 = -m->r0;
+    if (neg1) m->r1 = -m->r1;
     if (flip_r) {
-        quad_reverse(q);
         const V3 t = m->r0;
         m->r0 = m->r1;
         m->r1 = t;
     }
+    o->reverse = rev != flip_r;
+    o->mi = m3_inverse(*m);
 }
 // theta / sin(theta) of the edge between unit vectors v1 and v2 by the rational fit of
 // ltc_integrate_edge (lights.hlsl:365-381); the edge's term is cross(v1, v2) times it.
@@ -562,21 +581,39 @@ PT_HD float ltc_integrate(V3 P, const Frame& fr, const M3* minv, const V3 q[4], 
         inside |= (v.z > 0.0f ? 1u : 0u) << k;
     }
     if (inside == 0u || inside == 5u || inside == 10u) return 0.0f;   // below, or a diagonal pair
-    V3 c[5];
-    int n = 0;
-    for (int k = 0; k < 4; ++k) {
-        const V3 a = l[k], b = l[(k + 1) & 3];
-        const bool ai = (inside >> k) & 1u, bi = (inside >> ((k + 1) & 3)) & 1u;
-        if (ai) c[n++] = a;
-        if (ai != bi) {
-            const V3 in = ai ? a : b, out = ai ? b : a;
-            c[n++] = v3(in.z * out.x - out.z * in.x, in.z * out.y - out.z * in.y, in.z * out.z - out.z * in.z);
+    // The clipped polygon's vertices at fixed places (no indexed array: it would live in
+    // scratch memory): a quad above the plane as it is, else each emission goes to place n.
+    const V3 zero = v3(0.0f, 0.0f, 0.0f);
+    V3 c[5] = {l[0], l[1], l[2], l[3], zero};
+    int n = 4;
+    if (inside != 15u) {
+        n = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const V3 a = l[k], b = l[(k + 1) & 3];
+            const bool ai = (inside >> k) & 1u, bi = (inside >> ((k + 1) & 3)) & 1u;
+            if (ai) {
+#pragma unroll
+                for (int j = 0; j < 5; ++j) c[j] = sel3(j == n, a, c[j]);
+                ++n;
+            }
+            if (ai != bi) {
+                const V3 in = sel3(ai, a, b), out = sel3(ai, b, a);
+                const V3 x = v3(in.z * out.x - out.z * in.x, in.z * out.y - out.z * in.y, in.z * out.z - out.z * in.z);
+#pragma unroll
+                for (int j = 0; j < 5; ++j) c[j] = sel3(j == n, x, c[j]);
+                ++n;
+            }
         }
     }
-    for (int k = 0; k < n; ++k) c[k] = normalize(c[k]);
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        if (k < n) c[k] = normalize(c[k]);
     float sum = 0.0f, sx = 0.0f, sy = 0.0f;
-    for (int k = 0; k < n; ++k) {
-        const V3 a = c[k], b = c[k + 1 < n ? k + 1 : 0];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        if (k >= n) break;
+        const V3 a = c[k], b = sel3(k + 1 < n, c[(k + 1) % 5], c[0]);
         const float t = ltc_edge_scale(a, b);
         sum = sum + (a.x * b.y - a.y * b.x) * t;
         if (dir) {
@@ -675,12 +712,9 @@ PT_HD V3 ltc_direction(const Frame& fr, const M3* m, V3 s) {
 // A rect light's contribution at a lit surface (rect_light_eval_ltc, lights.hlsl:
 // 471-513, then surface_eval_lut_lit, material/lit.hlsl:37-58): the diffuse integral
 // times (1 - F) base / pi plus the specular one times f0 * norm + f90 * Fresnel term.
-// (Called, not inlined: its table reads and two polygon integrals would otherwise share
-// the shading kernel's registers.)
-inline __device__ __noinline__ V3 rect_light_lit(const RectRec& R, const float4* ltc, const RectTexRec* rtex,
-                                                 const SceneTex& rtl, V3 P, const Frame& fr, V3 V, const Mat& m) {
-    const V3 lv = v3(dot(V, fr.t), dot(V, fr.b), dot(V, fr.n));
-    if (lv.z <= 0.0f) return v3(0.0f, 0.0f, 0.0f);
+// The part of it that is the same for every light of the vertex is in `view`.
+__device__ __forceinline__ V3 rect_light_lit(const RectRec& R, const LtcView& view, const RectTexRec* rtex,
+                                             const SceneTex& rtl, V3 P, const Frame& fr, V3 V, const Mat& m) {
     V3 q[4] = {v3(R.p3[0], R.p3[1], R.p3[2]), v3(R.p2[0], R.p2[1], R.p2[2]), v3(R.p1[0], R.p1[1], R.p1[2]),
                v3(R.p0[0], R.p0[1], R.p0[2])};
     const bool two = R.two_sided != 0u;
@@ -688,17 +722,14 @@ inline __device__ __noinline__ V3 rect_light_lit(const RectRec& R, const float4*
     const bool textured = R.texture_index >= 0;
     V3 sd, ss;
     const float i_d = ltc_integrate(P, fr, nullptr, q, two, textured ? &sd : nullptr);
-    M3 mt;
-    float bx, by;
-    ltc_matrix_brdf(ltc, lv, m.rx, m.ry, q, &mt, &bx, &by);
-    const M3 mi = m3_inverse(mt);
-    const float i_s = ltc_integrate(P, fr, &mi, q, two, textured ? &ss : nullptr);
+    if (view.reverse) quad_reverse(q);
+    const float i_s = ltc_integrate(P, fr, &view.mi, q, two, textured ? &ss : nullptr);
     V3 ld = e * i_d, ls = e * i_s;
     if (textured) {
         // the light's texture seen along each integral's direction (lights.hlsl:495-511)
         const RectTexRec& rt = rtex[R.texture_index];
         if (i_d != 0.0f) ld = ld * rect_tex_lookup(R, rt, rtl, ltc_direction(fr, nullptr, sd), P, 1.0f);
-        if (i_s != 0.0f) ls = ls * rect_tex_lookup(R, rt, rtl, ltc_direction(fr, &mt, ss), P, __builtin_sqrtf(m.rx * m.ry));
+        if (i_s != 0.0f) ls = ls * rect_tex_lookup(R, rt, rtl, ltc_direction(fr, &view.mt, ss), P, __builtin_sqrtf(m.rx * m.ry));
     }
     const float ndotv = dot(fr.n, V);
     if (ndotv <= 0.0f) return v3(0.0f, 0.0f, 0.0f);
@@ -707,7 +738,7 @@ inline __device__ __noinline__ V3 rect_light_lit(const RectRec& R, const float4*
     const V3 fres = m.f0 + (m.f90 - m.f0) * p5;
     const V3 one = v3(1.0f, 1.0f, 1.0f);
     const V3 diffuse = ((one - fres) * m.base) * kInvPi;
-    const V3 specular = m.f0 * bx + m.f90 * by;
+    const V3 specular = m.f0 * view.bx + m.f90 * view.by;
     return diffuse * ld + specular * ls;
 }
 

@@ -108,6 +108,21 @@ __device__ __forceinline__ void with_job(const WaveJobs& jobs, uint32_t path, F 
     }
 }
 
+// As with_job with one copy of f: the wavefront takes its jobs one after the other, each at
+// a uniform address (for code so large that with_job's three copies crowd the instruction
+// cache).
+template <class F>
+__device__ __forceinline__ void each_job(const WaveJobs& jobs, uint32_t path, F f) {
+    uint32_t j = jobs.num_jobs == 1u ? 0u : job_of(jobs.path_base, jobs.num_jobs, path);
+    for (bool done = false; !done;) {
+        const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
+        if (j == j0) {
+            f(jobs.rec[j0], path - (jobs.num_jobs == 1u ? 0u : jobs.path_base[j0]));
+            done = true;
+        }
+    }
+}
+
 // Slot, pixel and sample of a job's local path: images walk their pixels in 8x8 tile
 // order, sample after sample; the cache's training paths take one pixel per slot drawn
 // uniformly from the image (PCG32 keyed by the job seed and slot) and use the slot as
@@ -204,9 +219,19 @@ struct ShadeArgs {
 // covers (count_in entries, or num_entries if count_in is null).
 void launch_shade_reset(uint64_t* tile_state, const uint32_t* count_in, uint32_t num_entries, uint32_t* count_ext,
                         uint32_t* count_shadow, uint32_t capacity, hipStream_t s);
-// max_lights: the most lights of any job in the launch (at most kMaxDirLights); rect: some
-// job of the launch has rect lights.
-void launch_shade(const ShadeArgs& a, uint32_t capacity, uint32_t max_lights, bool rect, hipStream_t s);
+// max_lights: the most lights of any job in the launch (at most kMaxDirLights).
+void launch_shade(const ShadeArgs& a, uint32_t capacity, uint32_t max_lights, hipStream_t s);
+
+// Rect lights of a segment's vertices (waves where some job has them), after its shading.
+struct RectArgs {
+    WaveJobs jobs;
+    RayQueue qin;
+    const uint32_t* count_in;   // null at bounce 0
+    HitBuf hits;
+    PathState ps;
+    uint32_t bounce;
+};
+void launch_shade_rect(const RectArgs& a, uint32_t capacity, hipStream_t s);
 
 struct ResolveArgs {
     WaveJobs jobs;

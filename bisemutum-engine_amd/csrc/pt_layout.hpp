@@ -303,7 +303,7 @@ struct JobRec {
     uint8_t* gb_m0;
     const RectRec* rects;   // num_rects rect lights (their slot follows the sky's)
     uint32_t num_rects;
-    const float4* ltc;      // 4 * kLtcTexels: matrix rows 0, 1, 2, then the norm table
+    const float4* ltc;      // 3 * kLtcTexels: per texel matrix row k (xyz) and norm component k (w; k < 2)
     const RectTexRec* rect_tex;   // the rect lights' textures (null: none)
     SceneTex rect_tex_levels;     // their mip levels: level records, texel pool, sRGB table
 };

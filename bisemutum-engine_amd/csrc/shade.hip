@@ -104,9 +104,20 @@ __device__ __forceinline__ void hit_surface(const JobRec& J, uint32_t leaf, floa
     mat_out = mat_id;
 }
 
+// The camera ray of a path: through its pixel's centre, or jittered by the path's key.
+__device__ __forceinline__ void entry_camera_ray(const JobRec& J, const PathKey& key, V3* o, V3* d) {
+    float jx = 0.5f, jy = 0.5f;
+    if (J.flags & 1u) {
+        Pcg jr = pcg_keyed(J.seed, key.pixel, key.sample, kJitterBounce);
+        jx = pcg_float(jr);
+        jy = pcg_float(jr);
+    }
+    camera_ray(J.cam, key.pixel % J.cam.width, key.pixel / J.cam.width, jx, jy, o, d);
+}
+
 // Shades queue entry i (path `path`, the job's local path `local`) of job J: its rays
 // go to `out` (mask: which of them exist).
-template <uint32_t NL, bool RECT>
+template <uint32_t NL>
 __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J, uint32_t i, uint32_t path,
                                             uint32_t local, bool primary, ShadeOut<NL>& out) {
     const size_t cap = a.ps.cap;
@@ -116,18 +127,12 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
     const uint32_t sample = key.sample;
     const uint32_t nl = J.num_lights;
     if (a.nrc_query) a.nrc_query[i].tag = kNoPath;   // entries without a cache query
-    const uint32_t nslots = nl + 2u + (RECT && J.num_rects ? 1u : 0u);
+    const uint32_t nslots = nl + 2u;   // the rect lights' slot is k_shade_rect's
     V3 o, d, P = v3(0.0f, 0.0f, 0.0f);
     V3 beta;
     float pdf_prev;
     if (primary) {
-        float jx = 0.5f, jy = 0.5f;
-        if (J.flags & 1u) {
-            Pcg jr = pcg_keyed(J.seed, pixel, sample, kJitterBounce);
-            jx = pcg_float(jr);
-            jy = pcg_float(jr);
-        }
-        camera_ray(J.cam, pixel % J.cam.width, pixel / J.cam.width, jx, jy, &o, &d);
+        entry_camera_ray(J, key, &o, &d);
         beta = v3(1.0f, 1.0f, 1.0f);
         pdf_prev = 0.0f;
         for (uint32_t k = 0; k < nslots; ++k) {
@@ -205,18 +210,6 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             }
             out.c[l] = c;
             mask |= 2u << l;
-        }
-        // rect lights (deferred_lighting_secondary.hlsl:73-96): no shadow rays, each light's
-        // lighting times the throughput added in light order to the slot after the sky's
-        if constexpr (RECT) {
-            if (J.num_rects) {
-                float4* acc = a.ps.acc + (kSlotLights + nl) * cap + path;
-                const float4 s = *acc;
-                V3 sum = v3(s.x, s.y, s.z);
-                for (uint32_t r = 0; r < J.num_rects; ++r)
-                    sum = sum + rect_light_lit(J.rects[r], J.ltc, J.rect_tex, J.rect_tex_levels, P, fr, V, m) * beta;
-                *acc = make_float4(sum.x, sum.y, sum.z, 0.0f);
-            }
         }
         // sky NEE only where the next segment is sampled too (the reference sees the
         // sky only through a traced segment that escapes)
@@ -325,7 +318,7 @@ __device__ __forceinline__ uint64_t look_back(const uint64_t* state, uint32_t t,
     }
 }
 
-template <uint32_t NL, bool RECT>
+template <uint32_t NL>
 __device__ __forceinline__ void shade_tile(const ShadeArgs& a) {
     __shared__ uint32_t s_wsum[4];
     __shared__ uint64_t s_base;
@@ -346,7 +339,7 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a) {
     if (i < count) {
         const uint32_t path = primary ? i : a.qin.path[i];
         with_job<false>(a.jobs, path, [&](const JobRec& J, uint32_t local) {
-            shade_entry<NL, RECT>(a, J, i, path, local, primary, out);
+            shade_entry<NL>(a, J, i, path, local, primary, out);
         });
     }
     // the tile's emissions: (extension << 16 | shadow) per entry, scanned in entry order
@@ -398,14 +391,71 @@ __device__ __forceinline__ void shade_tile(const ShadeArgs& a) {
 // One kernel per light bound; the one-light form (the common case) fits 80 registers,
 // 6 wavefronts per SIMD, without spilling.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_shade_l1(ShadeArgs a) {
-    shade_tile<1, false>(a);
+    shade_tile<1>(a);
 }
-__global__ __launch_bounds__(256) void k_shade_l2(ShadeArgs a) { shade_tile<2, false>(a); }
-__global__ __launch_bounds__(256) void k_shade_l4(ShadeArgs a) { shade_tile<kMaxDirLights, false>(a); }
-// With rect lights (launches where some job has them): the LTC integrals inline.
-__global__ __launch_bounds__(256) void k_shade_rect_l1(ShadeArgs a) { shade_tile<1, true>(a); }
-__global__ __launch_bounds__(256) void k_shade_rect_l2(ShadeArgs a) { shade_tile<2, true>(a); }
-__global__ __launch_bounds__(256) void k_shade_rect_l4(ShadeArgs a) { shade_tile<kMaxDirLights, true>(a); }
+__global__ __launch_bounds__(256) void k_shade_l2(ShadeArgs a) { shade_tile<2>(a); }
+__global__ __launch_bounds__(256) void k_shade_l4(ShadeArgs a) { shade_tile<kMaxDirLights>(a); }
+
+// Rect lights (deferred_lighting_secondary.hlsl:73-96) of one segment, after its shading:
+// no shadow rays, each light's lighting times the throughput added in light order to the
+// slot after the lights'.  This kernel alone writes that slot: a camera segment (and a
+// training path's cache segment) starts it from zero, a path that ends in the cache adds
+// nothing.  The surface is found again from the hit record: inside the shading kernel the
+// table integrals held 196 registers, 2 wavefronts per SIMD for all of the shading, whose
+// look-back waits on the slowest tile.  Bound by the table's gathers (48 16-B loads per
+// vertex, whatever the number of lights) and its own latency at 3 wavefronts per SIMD (4:
+// spills).  1280x720, two lights, three segments: 1,087 us of shading before, now 145 us and
+// 360 us here, beside the shadow rays.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_rect(RectArgs a) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const bool primary = a.bounce == 0;
+    if (i >= (primary ? a.jobs.num_paths : *a.count_in)) return;
+    const uint32_t path = primary ? i : a.qin.path[i];
+    each_job(a.jobs, path, [&](const JobRec& J, uint32_t local) {
+        if (!J.num_rects) return;
+        const uint32_t leaf = a.hits.rec[i].leaf;
+        const bool at_cache = a.bounce == J.cache_bounce && leaf != kLeafMiss;
+        const bool ends = at_cache && (J.flags & kJobCache);
+        const bool fresh = primary || (at_cache && (J.flags & kJobTrain));
+        const bool lit = leaf != kLeafMiss && !ends;
+        if (!lit && !primary) return;
+        float4* acc = a.ps.acc + (size_t)(kSlotLights + J.num_lights) * a.ps.cap + path;
+        V3 sum = v3(0.0f, 0.0f, 0.0f);
+        if (lit) {
+            V3 o, d, beta = v3(1.0f, 1.0f, 1.0f);
+            if (primary) {
+                entry_camera_ray(J, path_key(J, local), &o, &d);
+            } else {
+                o = v3(a.qin.ox[i], a.qin.oy[i], a.qin.oz[i]);
+                d = v3(a.qin.dx[i], a.qin.dy[i], a.qin.dz[i]);
+            }
+            if (!fresh) {
+                const float4 b = a.qin.beta[i], s = *acc;
+                beta = v3(b.x, b.y, b.z);
+                sum = v3(s.x, s.y, s.z);
+            }
+            const HitRec hit = a.hits.rec[i];
+            const V3 P = o + d * hit.t;
+            Mat m;
+            V3 N;
+            float rough;
+            uint32_t mat_id;
+            hit_surface(J, leaf, hit.u, hit.v, P, d, m, N, rough, mat_id);
+            const V3 V = normalize(o - P);
+            const Frame fr = make_frame(N);
+            const V3 lv = v3(dot(V, fr.t), dot(V, fr.b), dot(V, fr.n));
+            const bool front = !(lv.z <= 0.0f);
+            LtcView view;
+            if (front) ltc_view(J.ltc, lv, m.rx, m.ry, &view);
+            for (uint32_t r = 0; r < J.num_rects; ++r) {
+                V3 c = v3(0.0f, 0.0f, 0.0f);
+                if (front) c = rect_light_lit(J.rects[r], view, J.rect_tex, J.rect_tex_levels, P, fr, V, m);
+                sum = sum + c * beta;
+            }
+        }
+        *acc = make_float4(sum.x, sum.y, sum.z, 0.0f);
+    });
+}
 
 // Output counts and look-back words of the next shade launch.
 __global__ __launch_bounds__(256) void k_shade_reset(uint64_t* state, const uint32_t* count_in, uint32_t num_entries,
@@ -551,20 +601,21 @@ void launch_shade_reset(uint64_t* tile_state, const uint32_t* count_in, uint32_t
                        num_entries, count_ext, count_shadow);
 }
 
-void launch_shade(const ShadeArgs& a, uint32_t capacity, uint32_t max_lights, bool rect, hipStream_t s) {
+void launch_shade(const ShadeArgs& a, uint32_t capacity, uint32_t max_lights, hipStream_t s) {
     const uint32_t tiles = (capacity + kTile - 1) / kTile;
     const dim3 grid(tiles ? tiles : 1), block(256);
-    if (rect) {
-        if (max_lights <= 1) hipLaunchKernelGGL(k_shade_rect_l1, grid, block, 0, s, a);
-        else if (max_lights <= 2) hipLaunchKernelGGL(k_shade_rect_l2, grid, block, 0, s, a);
-        else hipLaunchKernelGGL(k_shade_rect_l4, grid, block, 0, s, a);
-    } else if (max_lights <= 1) {
+    if (max_lights <= 1) {
         hipLaunchKernelGGL(k_shade_l1, grid, block, 0, s, a);
     } else if (max_lights <= 2) {
         hipLaunchKernelGGL(k_shade_l2, grid, block, 0, s, a);
     } else {
         hipLaunchKernelGGL(k_shade_l4, grid, block, 0, s, a);
     }
+}
+
+void launch_shade_rect(const RectArgs& a, uint32_t capacity, hipStream_t s) {
+    if (capacity == 0) return;
+    hipLaunchKernelGGL(k_shade_rect, dim3((capacity + 255u) / 256u), dim3(256), 0, s, a);
 }
 
 void launch_resolve(const ResolveArgs& a, hipStream_t s) {
