@@ -322,7 +322,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
     // Default capacity 2^25 paths: a 1920x1080 frame of 16 spp is one wave, so each kernel
     // launches once per segment and drains its tail once (measured: 23% more rays/s than
     // 2^22-path waves); buffers are sized to the largest wave actually planned (about
-    // 270 B per path).  At most 2^28 paths, so packed shadow-ray ids fit in 32 bits.
+    // 310 B per path).  At most 2^28 paths, so packed shadow-ray ids fit in 32 bits.
     const Knobs& kn = opt.knobs;
     uint32_t cap = kn.wave_paths ? std::min(kn.wave_paths, kMaxWavePaths) : kDefaultWavePaths;
     cap = std::max(cap, max_npix);
