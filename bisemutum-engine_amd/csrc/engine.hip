@@ -575,7 +575,8 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
     }
 
     // graph replay: the same launch sequence with the same buffers (the plan's contents,
-    // uploaded above, carry everything that changes between calls)
+    // uploaded above, carry everything that changes between calls); the key holds all that
+    // decides which kernels are launched, on how much and with which arguments
     const bool graph = graph_owner && graph_owner->use_graph && !timing && !record;
     // a capture that an error leaves open is ended and its graph dropped, so the caller's
     // stream is usable again
@@ -597,7 +598,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
             key.insert(key.end(), {(uint64_t)(uintptr_t)p.ctx, (uint64_t)(uintptr_t)p.scene,
                                    (uint64_t)(uintptr_t)p.scene->nodes4.p, (uint64_t)(uintptr_t)p.ctx->sums.p,
                                    p.npix, p.spp, p.M, p.nl, p.sh, (uint64_t)p.reset, (uint64_t)p.rebuild,
-                                   p.scene->num_tris, (uint64_t)(jobs[j].gbuf != nullptr)});
+                                   p.scene->num_tris, (uint64_t)(jobs[j].gbuf != nullptr), (uint64_t)(p.nrect > 0)});
         }
         if (graph_owner->graph_exec && key == graph_owner->graph_key) {
             BI_HIP_TRY(own, hipGraphLaunch(graph_owner->graph_exec, s));

@@ -57,3 +57,38 @@ def test_mixed_waves(oracle_lib, sizes, one_light):
         t.close()
     b.close()
     assert all(ok)
+
+
+def test_graph_follows_rect_lights(oracle_lib):
+    """A replayed batch whose second job gains, keeps and loses rect lights while no buffer
+    changes (the first job's three lights already give every path a slot more than the second
+    job uses): each call equals the oracle's image of the scene as it then is."""
+    import torch
+    print("case: graph batch of c0 with three suns and c0, rect lights set and unset on the second", flush=True)
+    suns = scenes.scene_c0()
+    suns.dir_lights = np.stack([scenes.dir_light((0.9, 0.8, 0.7), d) for d in ((0.3, 0.8, 0.4), (-0.4, 0.7, 0.2), (0.1, 0.9, -0.5))])
+    plain, rect = scenes.scene_c0(), rect_c0(seed=2)
+    cam = scenes.camera_c0(40, 24)
+    ts = []
+    for sc in (suns, rect):
+        t = bi_pt.PathTracer()
+        t.set_scene(sc)
+        ts.append(t)
+    ts[1].set_rect_lights(None)
+    b = bi_pt.Batch()
+    b.set_tuning(use_graph=True)
+    stream = torch.cuda.Stream()
+    want = {k: oracle_lib.OracleScene(sc).render32(cam, 4, 21, spp=2)["sums"]
+            for k, sc in (("suns", suns), ("plain", plain), ("rect", rect))}
+    ok = []
+    for lights in (None, None, rect.rect_lights, rect.rect_lights, None):
+        ts[1].set_rect_lights(lights)
+        b.render([bi_pt.Job(t, cam, spp=2, max_bounces=4, seed=21) for t in ts], stream=stream.cuda_stream)
+        stream.synchronize()
+        got = [t.sums(cam.width * cam.height) for t in ts]
+        torch.cuda.synchronize()
+        ok += [radiance_check(got[0], want["suns"]), radiance_check(got[1], want["rect" if lights is not None else "plain"])]
+    for t in ts:
+        t.close()
+    b.close()
+    assert all(ok), ok
