@@ -96,17 +96,24 @@ PT_HD TravNode trav_pack(const float (*box)[6], const int32_t* id, int n) {
 }
 
 // A ray as the visit test reads it: inverse direction, and per axis -(o inv) -/+ 4u |o inv|
-// (u = 2^-24) for the planes met first and last; -inf and +inf where o inv overflows, so
-// that the axis rejects nothing.
+// (u = 2^-24) for the planes met first and last.
+//
+// Where o inv overflows, |o| is above 3.4e18 (|inv| is at most 1e20), so every plane of a
+// framed axis (|p| <= 1.004e18) lies at |(p - o) inv| >= 2.3e38, behind the ray or beyond any
+// extent (at most 1.7e38): cn and cf are then the same infinity, which rejects the node as
+// the exact test does.  (Left unconstrained, one ray with an infinite origin walks the whole
+// tree.)  The same holds where o inv is finite and a sum below overflows.  An axis whose
+// o inv is no number rejects nothing, as in the exact test.
 struct TravRay {
     float inv[3], cn[3], cf[3];
 };
 PT_HD void trav_ray_axis(TravRay& r, int a, float o, float inv) {
     const float oi = o * inv, m = __builtin_fabsf(oi);
-    const bool fine = m <= 1e38f;
+    const float slack = m <= 3.402823466e38f ? m * 0x1p-22f : 0.0f;   // none for an infinity (inf - inf)
+    const bool number = oi == oi;
     r.inv[a] = inv;
-    r.cn[a] = fine ? -oi - m * 0x1p-22f : -__builtin_inff();
-    r.cf[a] = fine ? -oi + m * 0x1p-22f : __builtin_inff();
+    r.cn[a] = number ? -oi - slack : -__builtin_inff();
+    r.cf[a] = number ? -oi + slack : __builtin_inff();
 }
 
 // One node as one ray sees it.  A plane q is met at

@@ -8,6 +8,9 @@ test passes, which `tests/host_wave/trav_host.cpp` counts over boxes and rays of
 that could break it: boxes of any size and distance, flat and single-point boxes, boxes of very
 different size in one node, rays along an axis, from a face or a corner, through corners, with
 zero direction components, at coordinates up to the range's end, and boxes that are no numbers.
+A ray whose origin times inverse direction overflows (an origin that is infinite, or far
+away along an axis that the direction does not follow) must not walk the tree either: the exact
+test rejects it at the root, and the visit test has to as well.
 """
 import functools
 import os
@@ -121,3 +124,55 @@ def test_no_box_is_skipped(host_binary, tmp_path, name):
         assert hit > 0.02 * total
         # planes are rounded by at most two of 252 quanta of the node's extent
         assert visited <= hit * 1.35 + 0.02 * total, (name, hit, visited)
+
+
+def far_rays(name):
+    """Rays that the exact test rejects at any box of ordinary coordinates."""
+    rng = np.random.default_rng(29)
+    n = 20000
+    r = records(n, rng)
+    a, rows = rng.integers(0, 3, n), np.arange(n)
+    if name == "infinite origin":
+        r["o"][rows, a] = rng.choice([-np.inf, np.inf], n)
+        more = rng.random((n, 3)) < 0.5
+        r["o"][more] = rng.choice([-np.inf, np.inf], int(more.sum()))
+        r["d"][rng.random((n, 3)) < 0.2] = 0.0
+    else:   # far away on one to three axes, none of which the direction follows except by chance
+        far = rng.random((n, 3)) < 0.5
+        far[rows, a] = True
+        mag = 10.0 ** rng.uniform(20, 38, (n, 3)) * rng.choice([-1.0, 1.0], (n, 3))
+        r["o"] = np.where(far, mag, r["o"])
+        r["d"] = rng.choice([0.0, -0.0], (n, 3))
+        k = (a + rng.integers(1, 3, n)) % 3
+        r["d"][rows, k] = rng.choice([-1.0, 1.0], n)
+    r["tmax"] = np.where(rng.random(n) < 0.5, 1000.0, 1.7e38)
+    return r
+
+
+@pytest.mark.parametrize("name", ["infinite origin", "far beside the direction"])
+def test_far_rays_visit_nothing(host_binary, tmp_path, name):
+    r = far_rays(name)
+    src = tmp_path / "in.bin"
+    r.tofile(src)
+    got = subprocess.run([str(host_binary), str(src)], check=True, capture_output=True, text=True, timeout=120).stdout
+    total, hit, skipped, visited, order = map(int, got.split())
+    assert total == int(r["n"].sum()) and hit == 0 and skipped == 0 and order == 0
+    assert visited == 0, (name, visited, total)
+
+
+def test_large_products_visit_as_the_exact_test(host_binary, tmp_path):
+    """Origin times inverse direction between 1e38 and the largest FP32 number: still a
+    number, so the axis still rejects what the exact test rejects."""
+    rng = np.random.default_rng(31)
+    n = 20000
+    r = records(n, rng)
+    a, rows = rng.integers(0, 3, n), np.arange(n)
+    r["o"][rows, a] = rng.uniform(1.1e18, 3.3e18, n) * rng.choice([-1.0, 1.0], n)
+    r["d"] = 0.0
+    r["d"][rows, (a + 1) % 3] = rng.choice([-1.0, 1.0], n)
+    r["tmax"] = 1.7e38
+    src = tmp_path / "in.bin"
+    r.tofile(src)
+    got = subprocess.run([str(host_binary), str(src)], check=True, capture_output=True, text=True, timeout=120).stdout
+    total, hit, skipped, visited, order = map(int, got.split())
+    assert skipped == 0 and order == 0 and visited <= hit + 0.001 * total, (hit, visited, total)
