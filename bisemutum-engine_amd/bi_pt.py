@@ -29,7 +29,7 @@ STATUS = {0: "OK", 1: "INVALID_ARGUMENT", 2: "OUT_OF_MEMORY", 3: "HIP", 4: "NO_S
 # every entry point declared in include/bi_pt.h
 EXPORTS = ["bi_pt_create", "bi_pt_destroy", "bi_pt_last_error", "bi_pt_set_scene", "bi_pt_update_transforms",
            "bi_pt_set_lights", "bi_pt_set_point_lights", "bi_pt_set_rect_lights", "bi_pt_set_rect_light_textures", "bi_pt_rect_texture_mips", "bi_pt_set_ltc_luts", "bi_pt_set_sky", "bi_pt_set_sky_cube", "bi_pt_render", "bi_pt_render_gbuffer", "bi_pt_drawables_layout", "bi_pt_set_scene_drawables", "bi_pt_reset_accumulation", "bi_pt_get_stats",
-           "bi_pt_debug_get_bvh", "bi_pt_debug_get_bvh4", "bi_pt_debug_num_tris", "bi_pt_debug_queue", "bi_pt_debug_get_sums",
+           "bi_pt_debug_get_bvh", "bi_pt_debug_get_bvh4", "bi_pt_debug_num_tris", "bi_pt_debug_built_rounds", "bi_pt_debug_queue", "bi_pt_debug_get_sums",
            "bi_pt_debug_trace", "bi_pt_trace_closest", "bi_pt_trace_occlusion", "bi_pt_batch_create", "bi_pt_batch_destroy", "bi_pt_batch_last_error",
            "bi_pt_batch_set_tuning", "bi_pt_batch_get_tuning", "bi_pt_render_batch", "bi_pt_batch_get_stats",
            "bi_pt_batch_autotune", "bi_pt_create_view", "bi_pt_server_create", "bi_pt_server_destroy",
@@ -244,6 +244,8 @@ def lib():
         L.bi_pt_debug_get_bvh4.argtypes = [vp, i32p, f32p]
         L.bi_pt_debug_num_tris.argtypes = [vp]
         L.bi_pt_debug_num_tris.restype = u32
+        L.bi_pt_debug_built_rounds.argtypes = [vp]
+        L.bi_pt_debug_built_rounds.restype = u32
         L.bi_pt_debug_queue.argtypes = [vp, u32, u32, u32, u32p, u32, u32p]
         L.bi_pt_debug_get_sums.argtypes = [vp, f32p]
         L.bi_pt_debug_trace.argtypes = [vp, u32, f32p, C.c_int, f32p, u32p, f32p, f32p]
@@ -292,7 +294,7 @@ def lib():
         L.bi_pt_debug_inject_error.argtypes = [vp, u32]
         L.bi_pt_server_debug_inject_error.argtypes = [vp, u32]
         for name in EXPORTS:
-            if name not in ("bi_pt_last_error", "bi_pt_debug_num_tris", "bi_pt_batch_last_error",
+            if name not in ("bi_pt_last_error", "bi_pt_debug_num_tris", "bi_pt_debug_built_rounds", "bi_pt_batch_last_error",
                             "bi_pt_server_last_error", "bi_pt_server_clock", "bi_pt_nrc_last_error"):
                 getattr(L, name).restype = C.c_int
         _lib = L
@@ -550,6 +552,11 @@ class PathTracer:
     # ---------------------------------------------------------------- inspection
     def num_tris(self):
         return lib().bi_pt_debug_num_tris(self.h)
+
+    def built_rounds(self):
+        """Treelet rounds of the LBVH that stands now (None: none is current)."""
+        r = lib().bi_pt_debug_built_rounds(self.h)
+        return None if r == 0xFFFFFFFF else r
 
     def bvh(self):
         n = self.num_tris()

@@ -215,6 +215,7 @@ bi_pt_status query_prepare(bi_pt_ctx*& ctx, uint32_t n, const bi_pt_rays* rays, 
         return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "ray queries need 0.001 < tmax <= 1.7e38");
     BI_HIP_TRY(ctx, hipSetDevice(ctx->device));
     BI_TRY(engine_init(ctx, ctx->eng));
+    ctx->tree_use.outlived = true;   // renders build trees for queries too from now on
     if (!ctx->bvh_built) {
         BI_TRY(ensure_build_buffers(ctx));
         BI_TRY(build_bvh(ctx, s, &ctx->eng.counters.p[kCntError], ctx->treelet_rounds));
@@ -405,6 +406,7 @@ bi_pt_status bi_pt_set_scene(bi_pt_ctx* ctx, const bi_pt_mesh* meshes, uint32_t 
     ctx->num_mats = num_materials;
     ctx->has_scene = true;
     ctx->bvh_built = false;
+    ctx->tree_use.rendered = false;
     ctx->acc_count = 0;
     ctx->scene_version++;
     return BI_PT_OK;
@@ -1078,6 +1080,11 @@ bi_pt_status bi_pt_debug_get_bvh4(bi_pt_ctx* ctx, int32_t* child4, float* box4) 
     return BI_PT_OK;
 }
 
+uint32_t bi_pt_debug_built_rounds(const bi_pt_ctx* ctx) {
+    if (ctx && ctx->scene_src) ctx = ctx->scene_src;
+    return ctx && ctx->bvh_built ? ctx->built_rounds : 0xffffffffu;
+}
+
 uint32_t bi_pt_debug_num_tris(const bi_pt_ctx* ctx) {
     if (ctx && ctx->scene_src) ctx = ctx->scene_src;
     return ctx ? ctx->num_tris : 0;
@@ -1199,6 +1206,7 @@ bi_pt_status bi_pt_trace_closest_noalloc(bi_pt_ctx* ctx, uint32_t n, const bi_pt
         return fail(ctx, BI_PT_ERROR_UNSUPPORTED,
                     "bi_pt_trace_closest_noalloc needs the scene's LBVH built (render or query the scene once "
                     "after its last change)");
+    ctx->tree_use.outlived = true;
     if (n == 0) return BI_PT_OK;
     if (!hit_triangle) return fail(ctx, BI_PT_ERROR_INVALID_ARGUMENT, "null hit_triangle");
     BI_HIP_TRY(ctx, hipSetDevice(ctx->device));

@@ -204,25 +204,6 @@ struct Prep {
     float* sums;          // running sums (training paths: the cache's targets)
 };
 
-// Treelet rounds that a call's paths repay, at most `configured`.  Round k runs when the call
-// traces at least (2^21 + 32 n) (1 + k (k - 1) / 3) paths of the scene's n triangles (paths of
-// fewer than four segments count in proportion): the first round saves most, the third a
-// tenth of it, and each costs the same.  Frame with 0 / 1 / 2 / 3 rounds, build included:
-//   atrium (262k), 8 segments, 2.1 M paths   5.52 /  5.55 /  5.85 /  6.21 ms
-//                              4.1 M         8.88 /  8.40 /  8.62 /  8.91
-//                             16.6 M        28.68 / 25.21 / 24.91 / 25.10
-//                             33.2 M        55.2  / 47.7  / 46.8  / 46.6
-//   rooms of 20k, 6 segments,  1.8 M         3.01 /  3.05 /  3.27 /  3.49
-//                              7.4 M         7.49 /  7.03 /  7.14 /  7.32
-//   250k                       7.4 M         6.86 /  7.08 /  7.64 /  8.11
-//   900k                       8.3 M        11.31 / 13.34 / 14.85 / 16.38
-uint32_t paid_rounds(uint64_t paths, uint32_t tris, uint32_t configured) {
-    const uint64_t first = (1ull << 21) + 32ull * tris;
-    uint32_t k = 0;
-    while (k < configured && 3ull * paths >= first * (3ull + (uint64_t)k * (k + 1ull))) ++k;
-    return k;
-}
-
 // One job's share of one wave.
 struct Item {
     uint32_t job, sample_off, samples;
@@ -382,19 +363,23 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
             prep[j].sums = ctx->sums.p;
         }
     }
-    // treelet rounds of each scene's build: as many of the configured ones as the call's
-    // paths repay; a kept BVH with fewer rounds than the call wants is rebuilt
+    // treelet rounds of each scene's build (pt_rounds.hpp); a kept BVH with fewer rounds than
+    // the call wants is rebuilt
     for (uint32_t j = 0; j < n; ++j) {
         Prep& p = prep[j];
         bool first = true;
         for (uint32_t k = 0; k < j; ++k) first = first && prep[k].scene != p.scene;
         p.rounds = 0;
         if (!first) continue;
-        uint64_t quarter_paths = 0;
-        for (uint32_t k = j; k < n; ++k)
-            if (prep[k].scene == p.scene)
-                quarter_paths += (uint64_t)prep[k].npix * prep[k].spp * std::min(prep[k].D, 4u);
-        p.rounds = paid_rounds(quarter_paths / 4u, p.scene->num_tris, p.scene->treelet_rounds);
+        uint64_t paths = 0, quarter_paths = 0;   // quarters: paths by their segments, up to four
+        for (uint32_t k = j; k < n; ++k) {
+            if (prep[k].scene != p.scene) continue;
+            const uint64_t of_job = (uint64_t)prep[k].npix * prep[k].spp;
+            paths += of_job;
+            quarter_paths += of_job * std::min(prep[k].D, 4u);
+        }
+        p.rounds = build_rounds(p.scene->tree_use, opt.reuse_bvh, paths, quarter_paths / 4u, p.scene->num_tris,
+                                p.scene->treelet_rounds);
         if (!p.rebuild && p.scene->built_rounds < p.rounds) p.rebuild = true;
         if (p.rebuild)
             if (bi_pt_status e = ensure_build_buffers(p.scene); e != BI_PT_OK) return fail(own, e, p.scene->err);
@@ -852,7 +837,8 @@ finish:
         bi_pt_ctx* ctx = p.ctx;
         const bi_pt_settings* st = jobs[j].st;
         eng.camera_rays += (uint64_t)p.npix * p.spp;
-        if (p.rebuild) p.scene->bvh_built = true;
+        if (p.rebuild) p.scene->bvh_built = p.scene->tree_use.rendered = true;
+        if (opt.reuse_bvh) p.scene->tree_use.outlived = true;
         if (p.role == kRoleTrain) continue;
         ++images;
         image_ctx = ctx;

@@ -12,6 +12,7 @@
 
 #include "../../include/bi_pt.h"
 #include "pt_kernels.hpp"
+#include "pt_rounds.hpp"
 
 namespace bipt {
 
@@ -210,6 +211,7 @@ struct bi_pt_ctx : bipt::Owner {
     uint32_t treelet_rounds = 3;    // bi_pt_set_build_options
     bool bvh_built = false;
     uint32_t built_rounds = 0;      // treelet rounds of the BVH built last
+    bipt::TreeUse tree_use;         // whether trees are traced beyond the call that builds them
     // accumulation
     bipt::DevBuf<float> sums;
     uint32_t acc_w = 0, acc_h = 0;
@@ -238,8 +240,7 @@ namespace bipt {
 inline bi_pt_ctx* scene_of(bi_pt_ctx* c) { return c->scene_src ? c->scene_src : c; }
 
 bi_pt_status ensure_build_buffers(bi_pt_ctx* ctx);
-// rounds: treelet rounds of this build (the context's setting, or fewer for a call that
-// traces too few paths to repay them)
+// rounds: treelet rounds of this build (the context's setting, or what build_rounds gives)
 bi_pt_status build_bvh(bi_pt_ctx* ctx, hipStream_t s, uint32_t* error, uint32_t rounds);
 BvhView bvh_view(const bi_pt_ctx* ctx);
 // Texture inputs of a scene context's kernels.

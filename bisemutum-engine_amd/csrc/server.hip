@@ -123,8 +123,11 @@ bi_pt_status bi_pt_server_add_scene(bi_pt_server* s, bi_pt_ctx* scene, uint32_t*
         return fail(s, BI_PT_ERROR_INVALID_ARGUMENT, "a scene must be a context with a scene of its own");
     if (scene->device != s->device) return fail(s, BI_PT_ERROR_INVALID_ARGUMENT, "scene on another device");
     BI_HIP_TRY(s, hipSetDevice(s->device));
-    // resident: build the BVH now and keep it (jobs render with BI_PT_FLAG_REUSE_BVH)
-    if (!scene->bvh_built) {
+    // resident: build the BVH now, with all its treelet rounds, and keep it (jobs render with
+    // BI_PT_FLAG_REUSE_BVH); the tree of a render that had fewer may still be traced by it
+    scene->tree_use.outlived = true;
+    if (!scene->bvh_built || scene->built_rounds < scene->treelet_rounds) {
+        BI_HIP_TRY(s, hipDeviceSynchronize());
         BI_TRY(engine_init(scene, scene->eng));
         if (bi_pt_status e = ensure_build_buffers(scene); e != BI_PT_OK) return fail(s, e, scene->err);
         if (bi_pt_status e = build_bvh(scene, nullptr, &scene->eng.counters.p[kCntError], scene->treelet_rounds);

@@ -477,7 +477,12 @@ bi_pt_status bi_pt_reset_accumulation(bi_pt_ctx* ctx);
  * driver's).  After the LBVH (Morton codes, radix sort, Karras hierarchy, refit), rounds
  * of treelet restructuring lower the tree's surface-area cost (7-leaf treelets, optimal
  * topology by dynamic programming; Karras & Aila 2013).  Closest hits do not depend on
- * the tree, so images are the same for any setting; only the speed changes. */
+ * the tree, so images are the same for any setting; only the speed changes.  A render
+ * runs fewer rounds, or none, where its paths do not repay them: below max(4 n, 2^20)
+ * paths of n triangles, and, from a scene's second tree on, as long as the context's renders
+ * build anew call after call and nothing else traces their trees (a render with
+ * BI_PT_FLAG_REUSE_BVH, a ray query, the server), by the paths of each call alone.  Builds of
+ * ray queries and of the server run all rounds. */
 typedef struct bi_pt_build_options {
     uint32_t treelet_rounds;   /* 0 = the Morton/Karras tree as built; default 3; at most 16 */
     uint32_t _reserved[3];
@@ -573,7 +578,8 @@ bi_pt_status bi_pt_server_create(const bi_pt_server_desc* desc, bi_pt_server** o
 bi_pt_status bi_pt_server_destroy(bi_pt_server* server);
 const char* bi_pt_server_last_error(const bi_pt_server* server);
 double bi_pt_server_clock(const bi_pt_server* server);
-/* Makes a context's scene resident (its LBVH is built now and kept); the context must
+/* Makes a context's scene resident (its LBVH is built now, unless one with all its treelet
+ * rounds stands, and kept); the context must
  * outlive the server and keep its scene unchanged. */
 bi_pt_status bi_pt_server_add_scene(bi_pt_server* server, bi_pt_ctx* scene, uint32_t* scene_id);
 bi_pt_status bi_pt_server_submit(bi_pt_server* server, const bi_pt_request* request, uint64_t* job_id);
@@ -695,6 +701,8 @@ bi_pt_status bi_pt_debug_get_bvh(bi_pt_ctx* ctx, uint32_t* morton, uint32_t* ord
  * an empty slot holds +inf). */
 bi_pt_status bi_pt_debug_get_bvh4(bi_pt_ctx* ctx, int32_t* child4, float* box4);
 uint32_t bi_pt_debug_num_tris(const bi_pt_ctx* ctx);
+/* Treelet rounds of the LBVH that stands now (0xffffffff: none is current). */
+uint32_t bi_pt_debug_built_rounds(const bi_pt_ctx* ctx);
 /* Queue contents recorded by the last render with BI_PT_FLAG_RECORD_QUEUES:
  * kind 0 = extension queue entering segment `bounce` (path ids), kind 1 = shadow
  * queue of segment `bounce` (path_id << 3 | ray kind; kinds 0-3 lights, 7 sky).

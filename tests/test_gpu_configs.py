@@ -74,8 +74,8 @@ def test_batch_c2_graph_replay_equals_solo_and_oracle(oracle_lib):
 
 def test_batch_c2_trees_equal_oracle(oracle_lib):
     """After one batched call of the 64 scenes (their LBVHs built concurrently on four
-    streams, treelet rounds where the call traces enough paths), every scene's BVH4 is the
-    restatement's, node for node and bit for bit."""
+    streams, treelet rounds where the call traces enough paths for a scene's first tree), every
+    scene's BVH4 is the restatement's, node for node and bit for bit."""
     import torch
     specs = scenes.batch_c2()
     print("case: 64-scene batch, eager call, every BVH4 against the oracle's", flush=True)
@@ -101,6 +101,7 @@ def test_batch_c2_trees_equal_oracle(oracle_lib):
         o.set_treelet_rounds(r)
         oc, ob = o.bvh4()
         o.close()
+        assert t.built_rounds() == r   # the tree that the batch built, not one rebuilt for inspection
         gc, gb = t.bvh4()
         assert np.array_equal(gc, oc) and np.array_equal(gb.view(np.uint32), ob.view(np.uint32)), (k, sc.num_tris, r)
     print(f"64 trees equal ({sum(1 for r in rounds if r)} restructured)", flush=True)
@@ -200,3 +201,53 @@ def test_nrc_c4_atrium_1080p_training_samples(oracle_lib):
     assert np.isfinite(st["last_loss"])
     nrc.close()
     t.close()
+
+
+def test_rounds_of_trees_that_outlive_their_call(c0_scene):
+    """2^20 paths and more, but fewer than repay a round by themselves: the scene's first tree
+    and every tree of a context that renders with a kept tree, queries it or gives it to a server
+    has all rounds; a context that rebuilds call after call has none from the second on.  The
+    images are the same."""
+    print("case: c0 at 1280x820 (1.05 M paths), treelet rounds by the trees' use", flush=True)
+    cam = scenes.camera_c0(1280, 820)
+    kw = dict(spp=1, max_bounces=3, seed=4)
+    imgs = []
+
+    def tracer():
+        t = bi_pt.PathTracer()
+        t.set_scene(c0_scene)
+        assert t.built_rounds() is None
+        return t
+
+    def render(t, **more):
+        t.render(cam, **kw, **more)
+        imgs.append(t.image().copy())
+        return t.built_rounds()
+
+    t = tracer()
+    assert [render(t) for _ in range(3)] == [3, 0, 0]
+    t.update_transforms(c0_scene.instances["xform"])
+    assert render(t) == 0                                        # a moving scene
+    assert render(t, flags=bi_pt.FLAG_REUSE_BVH) == 3            # the kept tree gets its rounds
+    assert render(t, flags=bi_pt.FLAG_REUSE_BVH) == 3
+    assert render(t) == 3                                        # trees of this context are kept
+    t.set_scene(c0_scene)
+    assert render(t) == 3
+    t.close()
+    rays = (np.zeros((4, 3)) + (0.0, 2.0, 0.0), np.eye(4, 3) + 0.1)
+    for query in ("trace_closest", "trace_closest_noalloc", "trace_occlusion"):
+        t = tracer()
+        assert [render(t), render(t)] == [3, 0]
+        getattr(t, query)(*rays)
+        assert render(t) == 3
+        t.close()
+    t = tracer()
+    assert [render(t), render(t)] == [3, 0]
+    srv = bi_pt.Server()
+    srv.add_scene(t)
+    assert t.built_rounds() == 3
+    srv.close()
+    t.stats()
+    t.close()
+    for im in imgs[1:]:
+        assert np.array_equal(im.view(np.uint32), imgs[0].view(np.uint32))

@@ -1,0 +1,55 @@
+"""The rule for a build's treelet rounds (bisemutum-engine_amd/csrc/pt_rounds.hpp), compiled for
+the CPU, at its thresholds: a scene's first tree and trees that are traced beyond the call that
+builds them get all rounds from max(4 n, 2^20) paths on; trees of calls that rebuild one after
+the other get what each call's paths repay."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def rounds(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("rounds") / "rounds_host"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Wextra", "-o", str(exe),
+                    os.path.join(HERE, "host_wave", "rounds_host.cpp")], check=True)
+
+    def run(cases):
+        text = "".join(" ".join(str(int(x)) for x in c) + "\n" for c in cases)
+        return list(map(int, subprocess.run([str(exe)], input=text, check=True, capture_output=True, text=True).stdout.split()))
+    return run
+
+
+KEPT = [(0, 0, 0), (0, 0, 1), (0, 1, 0), (1, 0, 1), (1, 1, 0), (1, 1, 1)]   # rendered, outlived, reuse
+
+
+@pytest.mark.parametrize("use", KEPT)
+def test_kept_trees(rounds, use):
+    cases, want = [], []
+    for n in (0, 1, 20504, 1 << 18, (1 << 18) + 1, 900000, (1 << 29) - 1):
+        need = max(4 * n, 1 << 20)
+        for paths in (1, need - 1, need, 64 * need):
+            for configured in (0, 1, 3, 16):
+                cases.append(use + (paths, paths, n, configured))
+                want.append(configured if paths >= need else 0)
+                cases.append(use + (paths, paths // 4, n, configured))   # short paths do not change it
+                want.append(want[-1])
+    assert rounds(cases) == want
+
+
+def test_trees_of_one_call(rounds):
+    cases, want = [], []
+    for n in (0, 1, 20504, 262144, 900000, (1 << 29) - 1):
+        first = (1 << 21) + 32 * n
+        for k in (1, 2, 3, 4, 16):   # round k runs from first (1 + k (k - 1) / 3) paths on
+            need = -(-first * (3 + k * (k - 1)) // 3)
+            for paths, r in ((need - 1, k - 1), (need, k)):
+                for configured in (0, 1, 3, 16):
+                    cases.append((1, 0, 0, paths, paths, n, configured))
+                    want.append(min(r, configured))
+    assert rounds(cases) == want
+    # never more rounds than a kept tree of the same call
+    kept = rounds([(1, 1, 0) + c[3:] for c in cases])
+    assert all(a <= b for a, b in zip(want, kept))
