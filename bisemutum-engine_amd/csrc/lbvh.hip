@@ -37,11 +37,20 @@ __device__ __forceinline__ float ord2f(uint32_t o) {
 // The six order-preserving bounds (minima xyz, maxima xyz) sit on lines of their own, so
 // that their atomics do not queue behind each other.
 constexpr uint32_t kBoundStride = 32;
-// Start values of a build: bounds, and zeros for the sort's counters (`words` of them).
-__global__ __launch_bounds__(256) void k_build_init(uint32_t* cb, uint32_t* sort, uint32_t words) {
+// The sort's counters in one buffer (zero at the start): every digit's histogram
+// [pass][256], the tickets [pass], whether the sort failed, then the tiles' look-back words
+// [pass][tile][256].
+constexpr uint32_t kSortPasses = 4;
+constexpr uint32_t kSortTickets = kSortPasses * 256u;
+constexpr uint32_t kSortFailed = kSortTickets + 32u;
+constexpr uint32_t kSortTiles = kSortTickets + 64u;
+constexpr uint32_t kErrorSort = 64u;   // device error flag: a tile gave up its look-back
+// Start values of a build: bounds, and zeros for the sort's counters (`words` of them).  While
+// a sort's failure stands unreported in the error word, builds take their sort as failed.
+__global__ __launch_bounds__(256) void k_build_init(uint32_t* cb, uint32_t* sort, uint32_t words, const uint32_t* error) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if (t < 6) cb[t * kBoundStride] = t < 3 ? 0xffffffffu : 0u;
-    if (t < words) sort[t] = 0u;
+    if (t < words) sort[t] = t == kSortFailed ? *error & kErrorSort : 0u;
 }
 
 __global__ __launch_bounds__(256) void k_flatten(const float* __restrict__ pos, const float* __restrict__ nrm,
@@ -166,13 +175,8 @@ __global__ __launch_bounds__(256) void k_leaf_attrs(const uint32_t* __restrict__
 }
 
 // The sort: kSortPasses digits of 8 bits, lowest first.  A tile is kSortTile keys.
-constexpr uint32_t kSortPasses = 4;
 constexpr uint32_t kSortItems = 8;
 constexpr uint32_t kSortTile = 256u * kSortItems;
-// The sort's counters in one buffer (zero at the start): every digit's histogram
-// [pass][256], the tickets [pass], then the tiles' look-back words [pass][tile][256].
-constexpr uint32_t kSortTickets = kSortPasses * 256u;
-constexpr uint32_t kSortTiles = kSortTickets + 64u;
 // Look-back word: the tile's own count or its inclusive prefix, in 30 bits.
 constexpr uint32_t kTileCount = 1u << 30, kTilePrefix = 2u << 30, kTileValue = (1u << 30) - 1u;
 
@@ -221,10 +225,13 @@ __global__ __launch_bounds__(256) void k_morton(const float* __restrict__ tri_v,
 // Keys of digit d in the tiles before `tile`: thread d reads the tiles' words backwards,
 // eight at a time (the loads overlap), down to the nearest inclusive prefix.  A tile is
 // taken by ticket, so every lower tile has started and publishes its count without
-// waiting for anyone; the wait is bounded all the same (error flag 64, and the scatter
-// writes nothing out of range).
+// waiting for anyone; the wait is bounded all the same.  A tile that gives up raises the
+// error flag and marks the sort as failed: its short prefix leaves holes in the sorted arrays,
+// so the hierarchy takes neither keys nor order from them (k_karras).
+// [host-sort begin] (tests compile this region for the CPU)
 constexpr uint32_t kSortSpinMax = 1u << 22;
-__device__ __forceinline__ uint32_t tile_look_back(const uint32_t* words, uint32_t tile, uint32_t d, uint32_t* error) {
+__device__ __forceinline__ uint32_t tile_look_back(const uint32_t* words, uint32_t tile, uint32_t d, uint32_t* failed,
+                                                   uint32_t* error) {
     uint32_t sum = 0, spins = 0;
     int q = (int)tile - 1;
     while (q >= 0) {
@@ -238,7 +245,8 @@ __device__ __forceinline__ uint32_t tile_look_back(const uint32_t* words, uint32
         for (int j = 0; j < 8; ++j) {
             if (w[j] == 0u) {   // not published yet: read again from here
                 if (++spins > kSortSpinMax) {
-                    atomicOr(error, 64u);
+                    atomicOr(error, kErrorSort);
+                    atomicOr(failed, kErrorSort);
                     return sum;
                 }
                 __builtin_amdgcn_s_sleep(1);
@@ -251,6 +259,7 @@ __device__ __forceinline__ uint32_t tile_look_back(const uint32_t* words, uint32
     }
     return sum;
 }
+// [host-sort end]
 
 // One digit of the sort, one launch.  Each wavefront ranks a run of 64 * kSortItems keys,
 // 64 at a time, with its own digit counters in LDS (no workgroup barrier between the
@@ -322,7 +331,7 @@ __global__ __launch_bounds__(256) void k_sort_digit(const uint32_t* __restrict__
     uint32_t excl = 0;
     if (tile > 0) {
         __hip_atomic_store(mine, kTileCount | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        excl = tile_look_back(words, tile, tid, error);
+        excl = tile_look_back(words, tile, tid, counters + kSortFailed, error);
     }
     __hip_atomic_store(mine, kTilePrefix | (excl + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint32_t at = start + excl;
@@ -335,7 +344,7 @@ __global__ __launch_bounds__(256) void k_sort_digit(const uint32_t* __restrict__
     for (uint32_t r = 0; r < kSortItems; ++r) {
         if (first + r * 64u >= n) continue;
         const uint32_t dest = s_cnt[wave][(key[r] >> shift) & 255u] + rank[r];
-        if (dest < n) {
+        if (dest < n) {   // always, unless a look-back gave up
             kout[dest] = key[r];
             vout[dest] = val[r];
         }
@@ -344,21 +353,59 @@ __global__ __launch_bounds__(256) void k_sort_digit(const uint32_t* __restrict__
 
 // The refit's workgroups take kRefitBlock consecutive leaves.  An internal node whose leaves
 // all belong to one workgroup is local to it (its own index then lies among theirs).
+// [host-karras begin] (tests compile this region for the CPU)
 constexpr int kRefitBlock = 256;
 __device__ __forceinline__ bool refit_local(int first, int last) { return first / kRefitBlock == last / kRefitBlock; }
 
-__device__ __forceinline__ int kdelta(const uint32_t* __restrict__ codes, int n, int i, int j) {
+// Length of the common prefix of the sorted codes i and j in the bits of `keep`, equal codes
+// told apart by their index (keep 0: all codes equal).
+__device__ __forceinline__ int kdelta(const uint32_t* __restrict__ codes, uint32_t keep, int n, int i, int j) {
     if (j < 0 || j >= n) return -1;
-    uint32_t a = codes[i], b = codes[j];
+    const uint32_t a = codes[i] & keep, b = codes[j] & keep;
     if (a == b) return 32 + __clz((uint32_t)i ^ (uint32_t)j);
     return __clz(a ^ b);
 }
+// Internal node i of the radix tree over n >= 2 sorted codes (Karras 2012): its children and
+// its leaves.
+struct RadixNode {
+    int left, right, first, last;
+};
+__device__ __forceinline__ RadixNode radix_node(const uint32_t* __restrict__ codes, uint32_t keep, int n, int i) {
+    int d = (kdelta(codes, keep, n, i, i + 1) - kdelta(codes, keep, n, i, i - 1)) >= 0 ? 1 : -1;
+    int dmin = kdelta(codes, keep, n, i, i - d);
+    int lmax = 2;
+    while (kdelta(codes, keep, n, i, i + lmax * d) > dmin) lmax *= 2;
+    int l = 0;
+    for (int t = lmax / 2; t >= 1; t /= 2)
+        if (kdelta(codes, keep, n, i, i + (l + t) * d) > dmin) l += t;
+    int j = i + l * d;
+    int dnode = kdelta(codes, keep, n, i, j);
+    int s = 0;
+    int t = l;
+    do {
+        t = (t + 1) / 2;
+        if (kdelta(codes, keep, n, i, i + (s + t) * d) > dnode) s += t;
+    } while (t > 1);
+    int gamma = i + s * d + (d < 0 ? -1 : 0);
+    RadixNode r;
+    r.first = min(i, j);
+    r.last = max(i, j);
+    r.left = (r.first == gamma) ? ~gamma : gamma;
+    r.right = (r.last == gamma + 1) ? ~(gamma + 1) : gamma + 1;
+    return r;
+}
+// [host-karras end]
 
-__global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ codes, int n,
-                                                BvhNode* __restrict__ nodes, int32_t* __restrict__ parent,
-                                                uint32_t* __restrict__ refit_cnt, float* __restrict__ sub_cost,
-                                                int32_t* __restrict__ sub_height) {
+// The hierarchy.  After a failed sort it is the tree over equal codes in the triangles' own
+// order, which is a valid tree like any other (hits do not depend on it), and the order is
+// written accordingly: whatever the sort's buffers hold is never used as an index.
+__global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ codes, uint32_t* __restrict__ order, int n,
+                                                const uint32_t* __restrict__ sort_failed, BvhNode* __restrict__ nodes,
+                                                int32_t* __restrict__ parent, uint32_t* __restrict__ refit_cnt,
+                                                float* __restrict__ sub_cost, int32_t* __restrict__ sub_height) {
     int i = blockIdx.x * 256 + threadIdx.x;
+    const bool failed = *sort_failed != 0u;
+    if (failed && i < n) order[i] = (uint32_t)i;
     if (n == 1) {
         if (i == 0) {
             nodes[0].child[0] = ~0;
@@ -371,37 +418,19 @@ __global__ __launch_bounds__(256) void k_karras(const uint32_t* __restrict__ cod
         return;
     }
     if (i >= n - 1) return;
-    int d = (kdelta(codes, n, i, i + 1) - kdelta(codes, n, i, i - 1)) >= 0 ? 1 : -1;
-    int dmin = kdelta(codes, n, i, i - d);
-    int lmax = 2;
-    while (kdelta(codes, n, i, i + lmax * d) > dmin) lmax *= 2;
-    int l = 0;
-    for (int t = lmax / 2; t >= 1; t /= 2)
-        if (kdelta(codes, n, i, i + (l + t) * d) > dmin) l += t;
-    int j = i + l * d;
-    int dnode = kdelta(codes, n, i, j);
-    int s = 0;
-    int t = l;
-    do {
-        t = (t + 1) / 2;
-        if (kdelta(codes, n, i, i + (s + t) * d) > dnode) s += t;
-    } while (t > 1);
-    int gamma = i + s * d + (d < 0 ? -1 : 0);
-    int left = (min(i, j) == gamma) ? ~gamma : gamma;
-    int right = (max(i, j) == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-    nodes[i].child[0] = left;
-    nodes[i].child[1] = right;
-    const int first = min(i, j), last = max(i, j);   // the node's leaves
-    nodes[i].pad[0] = first;
-    nodes[i].pad[1] = last;
+    const RadixNode r = radix_node(codes, failed ? 0u : ~0u, n, i);
+    nodes[i].child[0] = r.left;
+    nodes[i].child[1] = r.right;
+    nodes[i].pad[0] = r.first;
+    nodes[i].pad[1] = r.last;
     // child boxes of nodes that several workgroups of the refit share start as NaN: the
     // refit reads a sibling's box once it is no longer NaN
-    if (!refit_local(first, last)) {
+    if (!refit_local(r.first, r.last)) {
         for (int a = 0; a < 12; ++a) nodes[i].box[a] = __uint_as_float(kBoxPending);
         refit_cnt[i] = 0;
     }
-    parent[left < 0 ? (n - 1) + ~left : left] = i;
-    parent[right < 0 ? (n - 1) + ~right : right] = i;
+    parent[r.left < 0 ? (n - 1) + ~r.left : r.left] = i;
+    parent[r.right < 0 ? (n - 1) + ~r.right : r.right] = i;
     if (i == 0) parent[0] = -1;
     // subtree cost and height, published by the refit when the node is complete
     sub_cost[i] = __uint_as_float(kBoxPending);
@@ -1157,7 +1186,8 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
     if (n == 0) return;
     const uint32_t g256 = (n + 255) / 256;
     const uint32_t tiles = (n + kSortTile - 1u) / kSortTile, words = sort_words(n);
-    hipLaunchKernelGGL(k_build_init, dim3((words + 255u) / 256u), dim3(256), 0, s, a.cbounds_ord, a.sort_counters, words);
+    hipLaunchKernelGGL(k_build_init, dim3((words + 255u) / 256u), dim3(256), 0, s, a.cbounds_ord, a.sort_counters, words,
+                       a.error);
     hipLaunchKernelGGL(k_flatten, dim3(g256), dim3(256), 0, s, a.positions, a.normals, a.indices, a.instances,
                        a.num_instances, n, a.tri_v, a.tri_n, a.tri_mat, a.cbounds_ord);
     hipLaunchKernelGGL(k_morton, dim3(tiles), dim3(256), 0, s, a.tri_v, n, a.cbounds_ord, a.keys[0], a.vals[0],
@@ -1169,8 +1199,8 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
         cur ^= 1;
     }
     // 4 passes: the sorted keys/values end in buffer 0
-    hipLaunchKernelGGL(k_karras, dim3(g256), dim3(256), 0, s, a.keys[cur], (int)n, a.nodes, a.parent, a.refit_cnt,
-                       a.tl_cost, a.tl_height);
+    hipLaunchKernelGGL(k_karras, dim3(g256), dim3(256), 0, s, a.keys[cur], a.vals[cur], (int)n,
+                       a.sort_counters + kSortFailed, a.nodes, a.parent, a.refit_cnt, a.tl_cost, a.tl_height);
     hipLaunchKernelGGL(k_leaves, dim3((n + kRefitBlock - 1) / kRefitBlock), dim3(kRefitBlock), 0, s, a.vals[cur], a.tri_v, a.tri_n, a.tri_mat,
                        a.materials, (int)n, a.leaf_geo, a.leaf_shade, a.nodes, a.parent, a.refit_cnt, a.tl_cost,
                        a.tl_height, a.error);

@@ -428,3 +428,31 @@ def test_ray_queries_match_restatement(c0_oracle, c0_scene):
     with pytest.raises(bi_pt.PtError):
         g.trace_closest(rays[:4, 0:3], rays[:4, 4:7], tmax=3.0e38)
     g.close()
+
+
+@pytest.mark.parametrize("tris", [1, 2, 3, 300, 5000])
+def test_build_after_a_failed_sort(oracle_lib, tris):
+    """While the sort's failure flag stands, builds use neither the sort's order nor its keys: the
+    tree is over the triangles in their own order, images are the same, and the flag is reported
+    once; then builds sort again."""
+    print(f"case: {tris} random triangles, sort failure flag raised before the build", flush=True)
+    sc = scenes.scene_random_triangles(tris, 8)
+    cam = scenes.camera_c0(40, 30)
+    g = bi_pt.PathTracer()
+    g.set_scene(sc)
+    o = oracle_lib.OracleScene(sc)
+    want = o.render32(cam, 4, 2, spp=2)["sums"]
+    sorted_order = o.bvh()["order"]
+    g.inject_error(64)
+    g.render(cam, spp=2, max_bounces=4, seed=2)
+    assert np.array_equal(g.sums(cam.width * cam.height).view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(g.bvh()["order"], np.arange(tris))
+    with pytest.raises(bi_pt.PtError) as e:
+        g.stats()
+    assert e.value.status == 5 and "sort" in str(e.value)
+    g.render(cam, spp=2, max_bounces=4, seed=2)
+    assert np.array_equal(g.sums(cam.width * cam.height).view(np.uint32), want.view(np.uint32))
+    g.update_transforms(sc.instances["xform"])
+    assert np.array_equal(g.bvh()["order"], sorted_order)
+    g.stats()
+    g.close()
