@@ -452,6 +452,7 @@ __device__ __forceinline__ float half_area_box(const float* b) {
     return (dx * dy + dy * dz) + dz * dx;
 }
 
+// [host-refit begin] (tests compile this region for the CPU)
 // A subtree the refit carries upward: box, surface-area cost, height.
 struct Carried {
     float box[6];
@@ -460,7 +461,9 @@ struct Carried {
 };
 // The sibling's record at a shared node: its box words, and its cost and height (a
 // triangle's follow from its box; an internal node's are published by its thread).  All
-// words are read at once and read again until none is pending.
+// words are read at once and read again until none is pending.  The wait is bounded (error
+// flag 4); words that have not arrived by then count as 0, since a pending word passed on
+// would run out the wait of every node above.
 __device__ __forceinline__ Carried wait_sibling(const float* box, int sib, const float* sub_cost,
                                                 const int32_t* sub_height, uint32_t* error) {
     Carried o;
@@ -473,21 +476,24 @@ __device__ __forceinline__ Carried wait_sibling(const float* box, int sib, const
             height = __hip_atomic_load(sub_height + sib, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         bool pending = cost == kBoxPending || height < 0;
-        for (int a = 0; a < 6; ++a) {
-            pending = pending || w[a] == kBoxPending;
-            o.box[a] = __uint_as_float(w[a]);
+        for (int a = 0; a < 6; ++a) pending = pending || w[a] == kBoxPending;
+        if (pending && spins <= (1u << 20)) {
+            __builtin_amdgcn_s_sleep(1);
+            continue;
         }
+        if (pending) {
+            atomicOr(error, 4u);
+            for (int a = 0; a < 6; ++a) w[a] = w[a] == kBoxPending ? 0u : w[a];
+            cost = cost == kBoxPending ? 0u : cost;
+            height = max(height, 0);
+        }
+        for (int a = 0; a < 6; ++a) o.box[a] = __uint_as_float(w[a]);
         o.cost = sib >= 0 ? __uint_as_float(cost) : half_area_box(o.box);
         o.height = height;
-        if (!pending) return o;
-        if (spins > (1u << 20)) {
-            atomicOr(error, 4u);
-            o.height = max(o.height, 0);
-            return o;
-        }
-        __builtin_amdgcn_s_sleep(1);
+        return o;
     }
 }
+// [host-refit end]
 
 // Leaf records in sorted order, and the bottom-up refit: every leaf's thread climbs, the
 // second arrival at a node continues.  Nodes local to a workgroup (all but a few per
