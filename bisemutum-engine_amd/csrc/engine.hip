@@ -166,6 +166,7 @@ bi_pt_status ensure_wave_buffers(Owner* own, Engine& eng, uint32_t cap, uint32_t
     cap = std::max(cap, eng.wave_cap);
     slots = std::max(slots, eng.wave_slots);
     sh_mult = std::max(sh_mult, eng.wave_sh_mult);
+    eng.wave_cap = 0;   // a failure below leaves no complete set: the next call starts over
     for (int k = 0; k < 6; ++k) {
         BI_TRY(dalloc(own, eng.qa[k], cap));
         BI_TRY(dalloc(own, eng.qb[k], cap));
@@ -359,7 +360,10 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
         any_cached |= prep[j].role == kRoleCached;
         any_train |= prep[j].role == kRoleTrain;
         if (prep[j].role != kRoleTrain) {
-            if ((e = dalloc(ctx, ctx->sums, (size_t)3 * prep[j].npix)) != BI_PT_OK) return fail(own, e, ctx->err);
+            float* const before = ctx->sums.p;
+            e = dalloc(ctx, ctx->sums, (size_t)3 * prep[j].npix);
+            if (ctx->sums.p != before) ctx->acc_count = 0;   // the running image is gone, also if the call fails
+            if (e != BI_PT_OK) return fail(own, e, ctx->err);
             prep[j].sums = ctx->sums.p;
         }
     }

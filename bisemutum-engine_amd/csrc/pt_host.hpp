@@ -48,21 +48,23 @@ inline bi_pt_status fail(Owner* o, bi_pt_status st, const std::string& msg) {
         if (s_ != BI_PT_OK) return s_;          \
     } while (0)
 
+// Room for n elements; the contents are lost where the buffer grows.  A growth that the budget
+// refuses leaves the buffer as it was.
 template <class T>
 bi_pt_status dalloc(Owner* o, DevBuf<T>& b, size_t n) {
     if (b.p && b.n >= n) return BI_PT_OK;
+    const size_t bytes = n * sizeof(T), held = b.p ? b.n * sizeof(T) : 0;
+    if (n && o->budget && o->allocated - held + bytes > o->budget)
+        return fail(o, BI_PT_ERROR_OUT_OF_MEMORY,
+                    "HBM budget exceeded: need " + std::to_string(bytes) + " B more, budget " +
+                        std::to_string(o->budget) + " B, in use " + std::to_string(o->allocated - held) + " B");
     if (b.p) {
         (void)hipFree(b.p);
-        o->allocated -= b.n * sizeof(T);
+        o->allocated -= held;
         b.p = nullptr;
         b.n = 0;
     }
     if (n == 0) return BI_PT_OK;
-    const size_t bytes = n * sizeof(T);
-    if (o->budget && o->allocated + bytes > o->budget)
-        return fail(o, BI_PT_ERROR_OUT_OF_MEMORY,
-                    "HBM budget exceeded: need " + std::to_string(bytes) + " B more, budget " +
-                        std::to_string(o->budget) + " B, in use " + std::to_string(o->allocated) + " B");
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) return fail(o, BI_PT_ERROR_OUT_OF_MEMORY, std::string("hipMalloc: ") + hipGetErrorString(e));

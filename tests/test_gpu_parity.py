@@ -456,3 +456,33 @@ def test_build_after_a_failed_sort(oracle_lib, tris):
     assert np.array_equal(g.bvh()["order"], sorted_order)
     g.stats()
     g.close()
+
+
+def test_render_after_a_refused_larger_render(oracle_lib, c0_scene):
+    """A call that the budget refuses leaves the context usable: the next call of the first size
+    renders as before.  Where the refusal came before the running image was touched it goes on
+    accumulating, else it starts over."""
+    print("case: c0 under a 32 MiB budget, larger renders refused in between", flush=True)
+    cam = scenes.camera_c0(48, 32)
+    o = oracle_lib.OracleScene(c0_scene)
+    want = {n: o.render32(cam, 5, 6, spp=n)["sums"] for n in (1, 2)}
+    g = bi_pt.PathTracer(hbm_budget_bytes=32 << 20)
+    g.set_scene(c0_scene)
+
+    def small():
+        g.render(cam, spp=1, max_bounces=5, seed=6, accumulate=True)
+        return g.sums(cam.width * cam.height)
+
+    def refused(w, h):
+        with pytest.raises(bi_pt.PtError) as e:
+            g.render(scenes.camera_c0(w, h), spp=4, max_bounces=5, seed=6)
+        assert e.value.status == 2
+
+    assert np.array_equal(small().view(np.uint32), want[1].view(np.uint32))
+    refused(2048, 2048)   # its running image alone (50 MB) is refused
+    assert np.array_equal(small().view(np.uint32), want[2].view(np.uint32))
+    refused(512, 512)     # its running image fits, its ray queues do not
+    assert np.array_equal(small().view(np.uint32), want[1].view(np.uint32))
+    assert np.array_equal(small().view(np.uint32), want[2].view(np.uint32))
+    g.stats()
+    g.close()
