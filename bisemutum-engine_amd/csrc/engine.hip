@@ -153,7 +153,7 @@ uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult) {
     b += 12 * c * 4 + 2 * c * 4;                 // queues A and B: 6 floats + path id each
     b += c * sizeof(HitRec);                     // hit records
     b += 2 * c * 16;                             // throughput and pdf of queues A and B
-    b += (uint64_t)slots * c * 16;               // radiance accumulators
+    b += (uint64_t)slots * c * sizeof(Rgb);      // radiance accumulators
     b += 2 * (uint64_t)sh_mult * c * (6 * 4 + 16);   // two shadow queue sets
     b += tiles * 8;                              // look-back words of the shade tiles
     return b;
@@ -304,7 +304,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
     // Default capacity 2^25 paths: a 1920x1080 frame of 16 spp is one wave, so each kernel
     // launches once per segment and drains its tail once (measured: 23% more rays/s than
     // 2^22-path waves); buffers are sized to the largest wave actually planned (about
-    // 310 B per path).  At most 2^28 paths, so packed shadow-ray ids fit in 32 bits.
+    // 300 B per path).  At most 2^28 paths, so packed shadow-ray ids fit in 32 bits.
     const Knobs& kn = opt.knobs;
     uint32_t cap = kn.wave_paths ? std::min(kn.wave_paths, kMaxWavePaths) : kDefaultWavePaths;
     cap = std::max(cap, max_npix);

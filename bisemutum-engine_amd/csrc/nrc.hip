@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void k_nrc_infer(NrcInferArgs a) {
             const float4 b = a.beta ? a.beta[e] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
             V3 c = v3(b.x * fmaxf(o[r][0], 0.0f), b.y * fmaxf(o[r][1], 0.0f), b.z * fmaxf(o[r][2], 0.0f));
             if (!finite3(c)) c = v3(0.0f, 0.0f, 0.0f);
-            a.ps.acc[path] = make_float4(c.x, c.y, c.z, 0.0f);
+            a.ps.acc[path] = Rgb{c.x, c.y, c.z};
         }
     }
 }

@@ -97,7 +97,8 @@ struct Knobs {
 struct Engine {
     uint32_t wave_cap = 0, wave_slots = 0, wave_sh_mult = 0;
     DevBuf<float> qa[6], qb[6], sq_f[2][6];
-    DevBuf<float4> qa_beta, qb_beta, acc, sq_cp[2];
+    DevBuf<float4> qa_beta, qb_beta, sq_cp[2];
+    DevBuf<Rgb> acc;
     DevBuf<uint32_t> qa_path, qb_path;
     DevBuf<HitRec> hit_rec;
     DevBuf<uint64_t> tile_state;           // look-back words of the shade launch's tiles

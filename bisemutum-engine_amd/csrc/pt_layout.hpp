@@ -15,7 +15,7 @@
 //              (48 B) in sorted leaf order
 //   per wave   SoA ray queues (o.xyz, d.xyz, path id), 16-B hit records (t, leaf, u, v),
 //              throughput and last BSDF pdf (16 B, in queue order), per-kind radiance
-//              accumulators (16 B), shadow queues (SoA o.xyz, d.xyz; 16 B contribution.xyz and
+//              accumulators (12 B), shadow queues (SoA o.xyz, d.xyz; 16 B contribution.xyz and
 //              path<<3|kind)
 // Nodes are read whole by one lane (4 x 16-B loads); rays, hits and path state are
 // read by consecutive lanes at consecutive addresses (coalesced).
@@ -337,12 +337,16 @@ struct ShadowQueue {
     float4* cp;
 };
 __device__ __forceinline__ uint32_t shadow_pk(const float4& cp) { return __float_as_uint(cp.w); }
-// Radiance accumulators [slot][cap] by path, xyz (16 B each: the scattered additions of the
-// shadow kernel and the misses are one load and one store).  A kind's slot does not depend
+// Radiance accumulators [slot][cap] by path, xyz in 12 B: the scattered additions of the
+// shadow kernel and the misses are one load and one store (16-B records: the same times,
+// 4 B per path and slot more).  A kind's slot does not depend
 // on the job's number of lights, so the shadow kernel needs no job to find it.
 constexpr uint32_t kSlotMiss = 0u, kSlotSky = 1u, kSlotLights = 2u;   // light l: kSlotLights + l; rect lights after them
+struct Rgb {
+    float x, y, z;
+};
 struct PathState {
-    float4* acc;
+    Rgb* acc;
     uint32_t cap;
 };
 

@@ -136,7 +136,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         beta = v3(1.0f, 1.0f, 1.0f);
         pdf_prev = 0.0f;
         for (uint32_t k = 0; k < nslots; ++k) {
-            a.ps.acc[k * cap + path] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            a.ps.acc[k * cap + path] = Rgb{0.0f, 0.0f, 0.0f};
         }
     } else {
         o = v3(a.qin.ox[i], a.qin.oy[i], a.qin.oz[i]);
@@ -153,7 +153,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
         float w = 1.0f;
         if (!primary && J.sky_nee) w = power_heuristic(pdf_prev, sky_pdf(J.sky, d));
         V3 c = (beta * ls) * w;
-        a.ps.acc[path] = make_float4(c.x, c.y, c.z, 0.0f);
+        a.ps.acc[path] = Rgb{c.x, c.y, c.z};
         if (want_depth) J.depth_out[pixel] = 0.0f;
     } else {
         const float t = hit.t, hu = hit.u, hv = hit.v;
@@ -187,7 +187,7 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             J.cache_rec[key.q] = r;
             beta = v3(1.0f, 1.0f, 1.0f);
             for (uint32_t k = 0; k < nslots; ++k) {
-                a.ps.acc[k * cap + path] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                a.ps.acc[k * cap + path] = Rgb{0.0f, 0.0f, 0.0f};
             }
         }
         Frame fr = make_frame(N);
@@ -203,9 +203,9 @@ __device__ __forceinline__ void shade_entry(const ShadeArgs& a, const JobRec& J,
             V3 c = (le * f) * beta;
             if (!any_pos(c)) continue;
             if (L.sm_index < 0) {
-                float4* acc = a.ps.acc + (kSlotLights + l) * cap + path;
-                const float4 s = *acc;
-                *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
+                Rgb* acc = a.ps.acc + (kSlotLights + l) * cap + path;
+                const Rgb s = *acc;
+                *acc = Rgb{s.x + c.x, s.y + c.y, s.z + c.z};
                 continue;
             }
             out.c[l] = c;
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         const bool fresh = primary || (at_cache && (J.flags & kJobTrain));
         const bool lit = leaf != kLeafMiss && !ends;
         if (!lit && !primary) return;
-        float4* acc = a.ps.acc + (size_t)(kSlotLights + J.num_lights) * a.ps.cap + path;
+        Rgb* acc = a.ps.acc + (size_t)(kSlotLights + J.num_lights) * a.ps.cap + path;
         V3 sum = v3(0.0f, 0.0f, 0.0f);
         if (lit) {
             V3 o, d, beta = v3(1.0f, 1.0f, 1.0f);
@@ -430,7 +430,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 d = v3(a.qin.dx[i], a.qin.dy[i], a.qin.dz[i]);
             }
             if (!fresh) {
-                const float4 b = a.qin.beta[i], s = *acc;
+                const float4 b = a.qin.beta[i];
+                const Rgb s = *acc;
                 beta = v3(b.x, b.y, b.z);
                 sum = v3(s.x, s.y, s.z);
             }
@@ -453,7 +454,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 sum = sum + c * beta;
             }
         }
-        *acc = make_float4(sum.x, sum.y, sum.z, 0.0f);
+        *acc = Rgb{sum.x, sum.y, sum.z};
     });
 }
 
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(256) void k_resolve(ResolveArgs a) {
     for (uint32_t s = 0; s < samples; ++s) {
         const size_t p = (size_t)pbase + (size_t)s * npix + q;
         auto slot = [&](uint32_t k) {
-            const float4 v = a.ps.acc[k * cap + p];
+            const Rgb v = a.ps.acc[k * cap + p];
             return v3(v.x, v.y, v.z);
         };
         V3 r = slot(kSlotMiss);

@@ -586,9 +586,9 @@ __device__ __forceinline__ bool apply_shadow(const ShadowArgs& a, uint32_t i, bo
         c = c * keep;
     }
     const uint32_t slot = kind == kKindSky ? kSlotSky : kSlotLights + kind;
-    float4* acc = a.ps.acc + (size_t)slot * a.ps.cap + path;
-    const float4 s = *acc;
-    *acc = make_float4(s.x + c.x, s.y + c.y, s.z + c.z, 0.0f);
+    Rgb* acc = a.ps.acc + (size_t)slot * a.ps.cap + path;
+    const Rgb s = *acc;
+    *acc = Rgb{s.x + c.x, s.y + c.y, s.z + c.z};
     return kind == kKindSky;
 }
 

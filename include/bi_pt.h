@@ -206,7 +206,7 @@ typedef struct bi_pt_settings {
     uint32_t spp;             /* samples per pixel rendered by this call */
     uint32_t seed;            /* PCG32 streams keyed by (seed, pixel, sample, bounce) */
     uint32_t flags;
-    uint32_t wave_paths;      /* paths in flight per wave; 0 = 2^25 (about 310 B of queues per path), at most 2^28 */
+    uint32_t wave_paths;      /* paths in flight per wave; 0 = 2^25 (about 300 B of queues per path), at most 2^28 */
     uint32_t stack_lds;       /* traversal stack entries kept in LDS (0 = automatic, <= 32) */
     uint32_t refill_lanes;    /* idle lanes before a wavefront fetches new rays (0 = automatic, <= 64) */
     uint32_t work_parts;      /* ray-queue parts with their own fetch counter (0 = automatic, <= 32) */
