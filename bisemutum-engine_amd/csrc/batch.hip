@@ -63,6 +63,7 @@ bi_pt_status bi_pt_batch_create(const bi_pt_device_desc* desc, bi_pt_batch** out
     if (!b) return BI_PT_ERROR_OUT_OF_MEMORY;
     b->device = desc ? desc->device : 0;
     b->budget = desc ? desc->hbm_budget_bytes : 0;
+    b->give_back = [](Owner* o) { return engine_give_back(o, static_cast<bi_pt_batch*>(o)->eng); };
     int ndev = 0;
     hipError_t e = hipGetDeviceCount(&ndev);
     if (e != hipSuccess || ndev == 0 || b->device < 0 || b->device >= ndev) {

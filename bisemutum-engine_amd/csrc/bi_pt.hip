@@ -235,6 +235,7 @@ bi_pt_status bi_pt_create(const bi_pt_device_desc* desc, bi_pt_ctx** out_ctx) {
     if (!ctx) return BI_PT_ERROR_OUT_OF_MEMORY;
     ctx->device = desc ? desc->device : 0;
     ctx->budget = desc ? desc->hbm_budget_bytes : 0;
+    ctx->give_back = [](Owner* o) { return engine_give_back(o, static_cast<bi_pt_ctx*>(o)->eng); };
     int ndev = 0;
     hipError_t e = hipGetDeviceCount(&ndev);
     if (e != hipSuccess || ndev == 0 || ctx->device < 0 || ctx->device >= ndev) {

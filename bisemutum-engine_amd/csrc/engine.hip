@@ -147,26 +147,70 @@ bi_pt_status validate_job(Owner* own, const bi_pt_camera* c, const bi_pt_setting
     return BI_PT_OK;
 }
 
-uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult) {
+uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult, uint32_t shadow_sets) {
     const uint64_t c = cap, tiles = (cap + 255u) / 256u + 1u;
     uint64_t b = 0;
     b += 12 * c * 4 + 2 * c * 4;                 // queues A and B: 6 floats + path id each
     b += c * sizeof(HitRec);                     // hit records
     b += 2 * c * 16;                             // throughput and pdf of queues A and B
     b += (uint64_t)slots * c * sizeof(Rgb);      // radiance accumulators
-    b += 2 * (uint64_t)sh_mult * c * (6 * 4 + 16);   // two shadow queue sets
+    b += shadow_sets * (uint64_t)sh_mult * c * kShadowRayBytes;
     b += tiles * 8;                              // look-back words of the shade tiles
     return b;
 }
 
+// The second shadow queue set only lets a segment's shadow rays trace beside the next
+// segment's closest hits: it is given back where the budget or the card needs its memory (per
+// path 40 B for each of its shadow rays, more than the throughput records added to the
+// path, so a budget that held a wave without those still does).
+bool engine_give_back(Owner* own, Engine& eng) {
+    if (eng.shadow_sets < 2) return false;
+    for (auto& f : eng.sq_f[1]) dfree(own, f);
+    dfree(own, eng.sq_cp[1]);
+    eng.shadow_sets = 1;
+    ++eng.wave_version;
+    return true;
+}
+
 namespace {
 
+bi_pt_status alloc_shadow_set(Owner* own, Engine& eng, int t, size_t shcap) {
+    for (auto& f : eng.sq_f[t]) BI_TRY(dalloc(own, f, shcap));
+    return dalloc(own, eng.sq_cp[t], shcap);
+}
+
+// The second shadow set, if it is wanted and there is room for it.
+void second_shadow_set(Owner* own, Engine& eng) {
+    if (eng.shadow_sets == 2 || eng.max_shadow_sets < 2) return;
+    const uint64_t rays = (uint64_t)eng.wave_cap * eng.wave_sh_mult;
+    if (eng.second_set_failed == rays) return;   // the card had no room for it
+    if (own->budget && own->allocated + rays * kShadowRayBytes > own->budget) return;
+    const std::string err = own->err;
+    auto* const give_back = own->give_back;
+    own->give_back = nullptr;   // not in exchange for itself
+    const bi_pt_status st = alloc_shadow_set(own, eng, 1, rays);
+    own->give_back = give_back;
+    eng.shadow_sets = 2;
+    ++eng.wave_version;
+    if (st == BI_PT_OK) return;
+    (void)engine_give_back(own, eng);
+    (void)hipGetLastError();
+    own->err = err;
+    eng.second_set_failed = rays;
+}
+
 bi_pt_status ensure_wave_buffers(Owner* own, Engine& eng, uint32_t cap, uint32_t slots, uint32_t sh_mult) {
-    if (cap <= eng.wave_cap && slots <= eng.wave_slots && sh_mult <= eng.wave_sh_mult) return BI_PT_OK;
+    if (cap <= eng.wave_cap && slots <= eng.wave_slots && sh_mult <= eng.wave_sh_mult) {
+        second_shadow_set(own, eng);
+        return BI_PT_OK;
+    }
     cap = std::max(cap, eng.wave_cap);
     slots = std::max(slots, eng.wave_slots);
     sh_mult = std::max(sh_mult, eng.wave_sh_mult);
     eng.wave_cap = 0;   // a failure below leaves no complete set: the next call starts over
+    (void)engine_give_back(own, eng);
+    eng.second_set_failed = 0;
+    ++eng.wave_version;
     for (int k = 0; k < 6; ++k) {
         BI_TRY(dalloc(own, eng.qa[k], cap));
         BI_TRY(dalloc(own, eng.qb[k], cap));
@@ -177,15 +221,13 @@ bi_pt_status ensure_wave_buffers(Owner* own, Engine& eng, uint32_t cap, uint32_t
     BI_TRY(dalloc(own, eng.qa_beta, cap));
     BI_TRY(dalloc(own, eng.qb_beta, cap));
     BI_TRY(dalloc(own, eng.acc, (size_t)slots * cap));
-    const size_t shcap = (size_t)cap * sh_mult;
-    for (int t = 0; t < 2; ++t) {
-        for (int k = 0; k < 6; ++k) BI_TRY(dalloc(own, eng.sq_f[t][k], shcap));
-        BI_TRY(dalloc(own, eng.sq_cp[t], shcap));
-    }
+    BI_TRY(alloc_shadow_set(own, eng, 0, (size_t)cap * sh_mult));
     BI_TRY(dalloc(own, eng.tile_state, (cap + 255u) / 256u + 1u));
+    eng.shadow_sets = 1;
     eng.wave_cap = cap;
     eng.wave_slots = slots;
     eng.wave_sh_mult = sh_mult;
+    second_shadow_set(own, eng);
     return BI_PT_OK;
 }
 
@@ -581,7 +623,7 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
     std::vector<uint64_t> key;
     if (graph) {
         key = {n, cap, lds_stack, refill, parts, block, (uint64_t)(uintptr_t)eng.plan.p, eng.wave_cap, eng.wave_slots,
-               eng.wave_sh_mult, plan_bytes, (uint64_t)any_hit, (uint64_t)any_point, (uint64_t)any_keep};
+               eng.wave_sh_mult, eng.wave_version, plan_bytes, (uint64_t)any_hit, (uint64_t)any_point, (uint64_t)any_keep};
         for (uint32_t j = 0; j < n; ++j) {
             const Prep& p = prep[j];
             key.insert(key.end(), {(uint64_t)(uintptr_t)p.ctx, (uint64_t)(uintptr_t)p.scene,
@@ -620,9 +662,10 @@ bi_pt_status render_jobs(Owner* own, Engine& eng, const JobIn* jobs, uint32_t n,
             sqs[t] = ShadowQueue{eng.sq_f[t][0].p, eng.sq_f[t][1].p, eng.sq_f[t][2].p, eng.sq_f[t][3].p, eng.sq_f[t][4].p,
                                  eng.sq_f[t][5].p, eng.sq_cp[t].p};
         // shadow launches overlap the next segment's closest hit, except when timing kernel
-        // classes, recording queues, or training the cache (whose reset of a training path's
-        // accumulators at the cache segment must follow the earlier shadow additions)
-        const bool overlap = !timing && !record && !any_train;
+        // classes, recording queues, training the cache (whose reset of a training path's
+        // accumulators at the cache segment must follow the earlier shadow additions), or
+        // without memory for the second set of shadow queues
+        const bool overlap = !timing && !record && !any_train && eng.shadow_sets == 2;
 
         if (record) { eng.rec_ext.clear(); eng.rec_sh.clear(); }
 

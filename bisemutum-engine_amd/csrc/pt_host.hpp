@@ -28,6 +28,8 @@ struct Owner {
     uint64_t budget = 0;      // 0 = unlimited
     uint64_t allocated = 0;
     std::string err;
+    // frees what the owner holds for speed alone; false if there was nothing (null: never any)
+    bool (*give_back)(Owner*) = nullptr;
 };
 
 inline bi_pt_status fail(Owner* o, bi_pt_status st, const std::string& msg) {
@@ -49,12 +51,14 @@ inline bi_pt_status fail(Owner* o, bi_pt_status st, const std::string& msg) {
     } while (0)
 
 // Room for n elements; the contents are lost where the buffer grows.  A growth that the budget
-// refuses leaves the buffer as it was.
+// refuses leaves the buffer as it was.  Memory held for speed alone gives way.
 template <class T>
 bi_pt_status dalloc(Owner* o, DevBuf<T>& b, size_t n) {
     if (b.p && b.n >= n) return BI_PT_OK;
     const size_t bytes = n * sizeof(T), held = b.p ? b.n * sizeof(T) : 0;
-    if (n && o->budget && o->allocated - held + bytes > o->budget)
+    auto refused = [&] { return n && o->budget && o->allocated - held + bytes > o->budget; };
+    if (refused() && o->give_back) (void)o->give_back(o);
+    if (refused())
         return fail(o, BI_PT_ERROR_OUT_OF_MEMORY,
                     "HBM budget exceeded: need " + std::to_string(bytes) + " B more, budget " +
                         std::to_string(o->budget) + " B, in use " + std::to_string(o->allocated - held) + " B");
@@ -67,6 +71,7 @@ bi_pt_status dalloc(Owner* o, DevBuf<T>& b, size_t n) {
     if (n == 0) return BI_PT_OK;
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess && o->give_back && o->give_back(o)) e = hipMalloc(&p, bytes);
     if (e != hipSuccess) return fail(o, BI_PT_ERROR_OUT_OF_MEMORY, std::string("hipMalloc: ") + hipGetErrorString(e));
     b.p = static_cast<T*>(p);
     b.n = n;
@@ -96,6 +101,10 @@ struct Knobs {
 // Queues and per-wave buffers, sized for the largest wave rendered so far.
 struct Engine {
     uint32_t wave_cap = 0, wave_slots = 0, wave_sh_mult = 0;
+    uint32_t shadow_sets = 0;              // shadow queue sets held: two, or one where memory is short
+    uint32_t max_shadow_sets = 2;
+    uint64_t second_set_failed = 0;        // shadow rays for which the card had no room for the second set
+    uint64_t wave_version = 0;             // changes with every allocation of the above
     DevBuf<float> qa[6], qb[6], sq_f[2][6];
     DevBuf<float4> qa_beta, qb_beta, sq_cp[2];
     DevBuf<Rgb> acc;
@@ -132,7 +141,9 @@ struct Engine {
 bi_pt_status engine_init(Owner* own, Engine& eng);
 // Device bytes of the wave buffers for waves of `cap` paths, `slots` radiance kinds and
 // `sh_mult` shadow rays per path (what ensure_wave_buffers allocates).
-uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult);
+uint64_t engine_bytes(uint32_t cap, uint32_t slots, uint32_t sh_mult, uint32_t shadow_sets);
+// Frees the second set of shadow queues, if it is held (Owner::give_back of contexts and batches).
+bool engine_give_back(Owner* own, Engine& eng);
 void engine_free(Owner* own, Engine& eng);
 // Statistics and the error flags raised since the last check (synchronises the device;
 // clears the flags it reports).

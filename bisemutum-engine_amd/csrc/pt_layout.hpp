@@ -336,6 +336,7 @@ struct ShadowQueue {
     float *ox, *oy, *oz, *dx, *dy, *dz;
     float4* cp;
 };
+constexpr uint32_t kShadowRayBytes = 6 * sizeof(float) + sizeof(float4);
 __device__ __forceinline__ uint32_t shadow_pk(const float4& cp) { return __float_as_uint(cp.w); }
 // Radiance accumulators [slot][cap] by path, xyz in 12 B: the scattered additions of the
 // shadow kernel and the misses are one load and one store (16-B records: the same times,

@@ -56,7 +56,8 @@ struct bi_pt_server : bipt::Owner {
     uint64_t rounds = 0;
 
     double now() const { return std::chrono::duration<double>(Clock::now() - t0).count(); }
-    uint64_t reserve = 0;          // wave buffers at full capacity for the resident scenes
+    uint64_t reserve = 0;          // wave buffers at full capacity for the resident scenes,
+    uint32_t slots = 0, sh = 0;    // which need these radiance slots and shadow rays per path
     uint32_t wave_cap = kDefaultWavePaths;   // the wave engine's capacity (what `reserve` covers)
     uint64_t used() const { return scene_bytes + job_bytes + std::max<uint64_t>(reserve, batch->allocated); }
 };
@@ -66,6 +67,27 @@ namespace {
 uint64_t job_cost(const SrvJob& j) {
     const uint64_t npix = (uint64_t)j.cam.width * j.cam.height;
     return npix * 12 + npix * 16;   // running sums + RGBA32F output
+}
+
+// Whether `bytes` more fit the budget beside the wave buffers, which are reserved at full
+// capacity for these slots and shadow rays; where they do not, the second set of shadow queues
+// (for speed alone) is given up for good.
+bool reserve_waves(bi_pt_server* s, uint32_t slots, uint32_t sh, uint64_t bytes) {
+    Engine& eng = s->batch->eng;
+    for (uint32_t sets = eng.max_shadow_sets; sets >= 1; --sets) {
+        const uint64_t need = engine_bytes(s->wave_cap, slots, sh, sets);
+        if (s->budget && need + bytes > s->budget) continue;
+        if (sets < eng.max_shadow_sets) {
+            (void)hipSetDevice(s->device);
+            eng.max_shadow_sets = sets;
+            (void)engine_give_back(s->batch, eng);
+        }
+        s->slots = slots;
+        s->sh = sh;
+        s->reserve = need;
+        return true;
+    }
+    return false;
 }
 
 void release(bi_pt_server* s, SrvJob& j) {
@@ -143,15 +165,10 @@ bi_pt_status bi_pt_server_add_scene(bi_pt_server* s, bi_pt_ctx* scene, uint32_t*
         for (const LightRec& L : c->lights) m += L.sm_index >= 0 ? 1u : 0u;
         return m;
     };
-    uint32_t slots = (uint32_t)scene->lights.size() + 2u, sh = shadow_mult(scene);
-    for (const bi_pt_ctx* c : s->scenes) {
-        slots = std::max<uint32_t>(slots, (uint32_t)c->lights.size() + 2u);
-        sh = std::max(sh, shadow_mult(c));
-    }
-    const uint64_t reserve = std::max(engine_bytes(s->wave_cap, slots, sh), s->reserve);
-    if (s->budget && s->scene_bytes + scene->allocated + reserve + s->job_bytes > s->budget)
+    const uint32_t slots = (uint32_t)scene->lights.size() + 2u + (scene->rects_host.empty() ? 0u : 1u);
+    if (!reserve_waves(s, std::max(slots, s->slots), std::max(shadow_mult(scene), s->sh),
+                       s->scene_bytes + scene->allocated + s->job_bytes))
         return fail(s, BI_PT_ERROR_OUT_OF_MEMORY, "scene does not fit the HBM budget");
-    s->reserve = reserve;
     s->scene_bytes += scene->allocated;
     s->scenes.push_back(scene);
     *scene_id = (uint32_t)(s->scenes.size() - 1);
@@ -173,7 +190,7 @@ bi_pt_status bi_pt_server_submit(bi_pt_server* s, const bi_pt_request* r, uint64
     j.st.flags &= ~(uint32_t)(BI_PT_FLAG_RECORD_QUEUES | BI_PT_FLAG_TIMING);
     j.st.flags |= BI_PT_FLAG_REUSE_BVH;
     j.t_submit = r->arrival_s >= 0.0 ? r->arrival_s : s->now();
-    if (s->budget && s->scene_bytes + s->reserve + job_cost(j) > s->budget)
+    if (!reserve_waves(s, s->slots, s->sh, s->scene_bytes + job_cost(j)))
         return fail(s, BI_PT_ERROR_OUT_OF_MEMORY, "job can never fit the HBM budget");
     const uint64_t id = s->next_id++;
     s->jobs.emplace(id, j);

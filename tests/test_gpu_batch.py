@@ -186,3 +186,62 @@ def test_batch_mixed_shadow_casting_lights_match_oracle(oracle_lib):
         t.close()
     b.close()
     assert all(ok), ok
+
+
+PATH_BYTES, PATH_BYTES_BEFORE = 300, 284   # queues of a path (one shadowed light, sky), with two sets of shadow queues;
+                                           # and before the throughput was held by both ray queues
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_budget_without_room_for_the_second_shadow_set(oracle_lib, graph):
+    """A budget that held the queues before the throughput was stored in both ray queues still
+    holds them: shadow rays then do without their second set of queues.  Solo and batched, also
+    replayed from a graph; the images are the oracle's."""
+    import torch
+    print(f"case: plane 512x512 4 spp under a budget of {PATH_BYTES_BEFORE} B per path, graph {graph}", flush=True)
+    sc, cam = plane_scene(), plane_camera(512, 512)
+    paths, npix = 512 * 512 * 4, 512 * 512
+    budget = paths * PATH_BYTES_BEFORE + npix * 12 + (2 << 20)
+    assert budget < paths * PATH_BYTES
+    want = oracle_lib.OracleScene(sc).render32(cam, 4, 31, spp=4)["sums"]
+    if not graph:
+        t = bi_pt.PathTracer(hbm_budget_bytes=budget)
+        t.set_scene(sc)
+        for _ in range(2):
+            t.render(cam, spp=4, max_bounces=4, seed=31)
+            assert np.array_equal(t.sums(npix).view(np.uint32), want.view(np.uint32))
+        t.stats()
+        t.close()
+    t = bi_pt.PathTracer()
+    t.set_scene(sc)
+    b = bi_pt.Batch(hbm_budget_bytes=budget)
+    b.set_tuning(use_graph=graph)
+    stream = torch.cuda.Stream()
+    for _ in range(3):
+        b.render([bi_pt.Job(t, cam, spp=4, max_bounces=4, seed=31)], stream=stream.cuda_stream)
+        stream.synchronize()
+        assert np.array_equal(t.sums(npix).view(np.uint32), want.view(np.uint32))
+        torch.cuda.synchronize()
+    b.stats()
+    b.close()
+    t.close()
+
+
+def test_second_shadow_set_gives_way_to_a_scene(oracle_lib, c0_scene):
+    """The second set of shadow queues, held since an earlier render, makes room for a larger scene."""
+    print("case: plane 512x512 4 spp, then c0, under one budget", flush=True)
+    sc, cam = plane_scene(), plane_camera(512, 512)
+    paths, npix = 512 * 512 * 4, 512 * 512
+    t = bi_pt.PathTracer(hbm_budget_bytes=paths * PATH_BYTES + npix * 12 + (2 << 20))
+    t.set_scene(sc)
+    t.render(cam, spp=4, max_bounces=4, seed=31)
+    want = oracle_lib.OracleScene(sc).render32(cam, 4, 31, spp=4)["sums"]
+    assert np.array_equal(t.sums(npix).view(np.uint32), want.view(np.uint32))
+    t.set_scene(c0_scene)   # about 8 MB with its build buffers
+    cam = scenes.camera_c0(64, 48)
+    for _ in range(2):
+        t.render(cam, spp=2, max_bounces=5, seed=3)
+        want = oracle_lib.OracleScene(c0_scene).render32(cam, 5, 3, spp=2)["sums"]
+        assert np.array_equal(t.sums(64 * 48).view(np.uint32), want.view(np.uint32))
+    t.stats()
+    t.close()

@@ -248,3 +248,37 @@ def test_server_with_textured_rect_lights_matches_oracle(c0_scene, oracle_lib):
     srv.close()
     for t in owners:
         t.close()
+
+
+def test_server_budget_without_room_for_the_second_shadow_set(c0_scene):
+    """A server budget that held the resident scene, the queues of 284 B per path (before the
+    throughput was stored in both ray queues) and a job still takes them: the reserve does
+    without the second set of shadow queues."""
+    print("case: server, c0, a budget of 284 B per path", flush=True)
+    owner = bi_pt.PathTracer()
+    owner.set_scene(c0_scene)
+    cam, cap = scenes.camera_c0(256, 256), 1 << 17
+    per_job = 256 * 256 * 28
+    probe = bi_pt.Server(spp_per_round=1, wave_paths=cap)
+    probe.add_scene(owner)
+    scene_bytes = probe.stats()["hbm_used"] - cap * 300 - (cap // 256 + 1) * 8
+    probe.close()
+    assert scene_bytes > 0
+    budget = scene_bytes + cap * 284 + (cap // 256 + 1) * 8 + per_job
+    srv = bi_pt.Server(hbm_budget_bytes=budget, spp_per_round=1, wave_paths=cap)
+    sid = srv.add_scene(owner)
+    ids = [srv.submit(sid, cam, spp=2, max_bounces=4, seed=7 + k) for k in range(3)]
+    for _ in range(100):
+        active = srv.step()
+        assert srv.stats()["hbm_used"] <= budget
+        for k, jid in enumerate(ids):
+            if jid is not None and srv.poll(jid)["state"] == 2:
+                got = srv.take_result(jid, 256 * 256)
+                want = solo_image(c0_scene, cam, spp=2, max_bounces=4, seed=7 + k)
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+                ids[k] = None
+        if active == 0:
+            break
+    assert ids == [None] * 3
+    srv.close()
+    owner.close()
