@@ -29,7 +29,7 @@ STATUS = {0: "OK", 1: "INVALID_ARGUMENT", 2: "OUT_OF_MEMORY", 3: "HIP", 4: "NO_S
 # every entry point declared in include/bi_pt.h
 EXPORTS = ["bi_pt_create", "bi_pt_destroy", "bi_pt_last_error", "bi_pt_set_scene", "bi_pt_update_transforms",
            "bi_pt_set_lights", "bi_pt_set_point_lights", "bi_pt_set_rect_lights", "bi_pt_set_rect_light_textures", "bi_pt_rect_texture_mips", "bi_pt_set_ltc_luts", "bi_pt_set_sky", "bi_pt_set_sky_cube", "bi_pt_render", "bi_pt_render_gbuffer", "bi_pt_drawables_layout", "bi_pt_set_scene_drawables", "bi_pt_reset_accumulation", "bi_pt_get_stats",
-           "bi_pt_debug_get_bvh", "bi_pt_debug_get_bvh4", "bi_pt_debug_num_tris", "bi_pt_debug_built_rounds", "bi_pt_debug_queue", "bi_pt_debug_get_sums",
+           "bi_pt_debug_get_bvh", "bi_pt_debug_get_bvh4", "bi_pt_debug_get_trav_nodes", "bi_pt_debug_num_tris", "bi_pt_debug_built_rounds", "bi_pt_debug_queue", "bi_pt_debug_get_sums",
            "bi_pt_debug_trace", "bi_pt_trace_closest", "bi_pt_trace_occlusion", "bi_pt_batch_create", "bi_pt_batch_destroy", "bi_pt_batch_last_error",
            "bi_pt_batch_set_tuning", "bi_pt_batch_get_tuning", "bi_pt_render_batch", "bi_pt_batch_get_stats",
            "bi_pt_batch_autotune", "bi_pt_create_view", "bi_pt_server_create", "bi_pt_server_destroy",
@@ -43,6 +43,8 @@ EXPORTS = ["bi_pt_create", "bi_pt_destroy", "bi_pt_last_error", "bi_pt_set_scene
 NOALLOC_MAX_RAYS = 1 << 18
 NRC_PARAMS = 17408
 NRC_FREEZE = 1
+TRAV_NODE_DTYPE = np.dtype([("base", np.float32, 3), ("scale", np.float32, 3), ("plane", np.uint8, (6, 4)),
+                            ("child", np.int32, 4)])
 
 
 class PtError(RuntimeError):
@@ -245,6 +247,7 @@ def lib():
         L.bi_pt_debug_num_tris.argtypes = [vp]
         L.bi_pt_debug_num_tris.restype = u32
         L.bi_pt_debug_built_rounds.argtypes = [vp]
+        L.bi_pt_debug_get_trav_nodes.argtypes = [vp, vp]
         L.bi_pt_debug_built_rounds.restype = u32
         L.bi_pt_debug_queue.argtypes = [vp, u32, u32, u32, u32p, u32, u32p]
         L.bi_pt_debug_get_sums.argtypes = [vp, f32p]
@@ -578,6 +581,12 @@ class PathTracer:
         box4 = np.zeros((ni, 24), np.float32)
         self._check(lib().bi_pt_debug_get_bvh4(self.h, _p(child4, C.c_int32), _p(box4)))
         return child4, box4
+
+    def trav_nodes(self):
+        """The traversal nodes of the LBVH that stands now (TRAV_NODE_DTYPE)."""
+        out = np.zeros(max(self.num_tris() - 1, 1), TRAV_NODE_DTYPE)
+        self._check(lib().bi_pt_debug_get_trav_nodes(self.h, C.c_void_p(out.ctypes.data)))
+        return out
 
     def queue(self, wave, bounce, kind):
         cnt = C.c_uint32()

@@ -1066,18 +1066,32 @@ bi_pt_status bi_pt_debug_get_bvh4(bi_pt_ctx* ctx, int32_t* child4, float* box4) 
     const uint32_t n = ctx->num_tris;
     if (n == 0) return BI_PT_OK;
     const size_t ni = n > 1 ? n - 1 : 1;
-    // the children of the traversal's nodes with their exact boxes, made from the BVH2
-    DevBuf<Bvh4Node> exact;
-    BI_TRY(dalloc(ctx, exact, ni));
-    launch_collapse_exact(ctx->nodes.p, n, exact.p, nullptr);
-    std::vector<Bvh4Node> nodes(ni);
-    const hipError_t e = hipMemcpy(nodes.data(), exact.p, ni * sizeof(Bvh4Node), hipMemcpyDeviceToHost);
-    dfree(ctx, exact);
-    BI_HIP_TRY(ctx, e);
+    // links as the traversal reads them; boxes exact, from the BVH2 (collapsed here again)
+    std::vector<BvhNode> nodes(ni);
+    std::vector<TravNode> trav(ni);
+    BI_HIP_TRY(ctx, hipMemcpy(nodes.data(), ctx->nodes.p, ni * sizeof(BvhNode), hipMemcpyDeviceToHost));
+    BI_HIP_TRY(ctx, hipMemcpy(trav.data(), ctx->nodes4.p, ni * sizeof(TravNode), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < ni; ++i) {
-        if (child4) std::memcpy(&child4[4 * i], nodes[i].child, 16);
-        if (box4) std::memcpy(&box4[24 * i], nodes[i].lox, 96);
+        if (child4) std::memcpy(&child4[4 * i], trav[i].child, 16);
+        if (!box4) continue;
+        int32_t id[4];
+        float box[4][6];
+        const int cnt = trav_children(nodes.data(), (int)i, id, box);
+        for (int k = 0; k < 4; ++k)
+            for (int a = 0; a < 6; ++a) box4[24 * i + 4 * a + k] = k < cnt ? box[k][a] : INFINITY;
     }
+    return BI_PT_OK;
+}
+
+bi_pt_status bi_pt_debug_get_trav_nodes(bi_pt_ctx* ctx, void* nodes64) {
+    if (ctx && ctx->scene_src) ctx = ctx->scene_src;   // a view is inspected through its scene
+    if (!ctx || !nodes64) return BI_PT_ERROR_INVALID_ARGUMENT;
+    if (!ctx->bvh_built) return fail(ctx, BI_PT_ERROR_UNSUPPORTED, "no LBVH stands");
+    BI_HIP_TRY(ctx, hipSetDevice(ctx->device));
+    BI_HIP_TRY(ctx, hipDeviceSynchronize());
+    const uint32_t n = ctx->num_tris;
+    if (n == 0) return BI_PT_OK;
+    BI_HIP_TRY(ctx, hipMemcpy(nodes64, ctx->nodes4.p, (n > 1 ? n - 1 : 1) * sizeof(TravNode), hipMemcpyDeviceToHost));
     return BI_PT_OK;
 }
 

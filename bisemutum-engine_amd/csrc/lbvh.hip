@@ -602,18 +602,6 @@ __global__ __launch_bounds__(kRefitBlock) void k_leaves(const uint32_t* __restri
     }
 }
 
-// BVH4 collapse.  Every internal BVH2 node k is turned into a BVH4 node stored at
-// index k, independently of the others: starting from k's two children, the internal
-// child with the largest box surface (ties: the lower slot) is replaced in its slot by
-// its first child and its second child is appended, until four slots are filled or
-// only leaves are left.  Traversal starts at node 0 and follows internal links, which
-// are BVH2 node indices and so name the BVH4 node built from that node; nodes not
-// reached that way are never read.  Runs after the refit: every box is final.
-__device__ __forceinline__ float half_area(const float* b) {
-    const float dx = b[3] - b[0], dy = b[4] - b[1], dz = b[5] - b[2];
-    return (dx * dy + dy * dz) + dz * dx;
-}
-
 // ---------------------------------------------------------------- treelet restructuring
 // Rounds of treelet restructuring (Karras & Aila 2013, "Fast Parallel Construction of
 // High-Quality Bounding Volume Hierarchies") lower the tree's surface-area cost after
@@ -1121,65 +1109,22 @@ __global__ __launch_bounds__(64) void k_tl_climb(TreeletArgs a) {
     }
 }
 
-// The children of BVH4 node k: links id and boxes (lo xyz, hi xyz); returns how many.
-__device__ __forceinline__ int collapse4(const BvhNode* __restrict__ nodes, int k, int (&id)[4], float (&box)[4][6]) {
-    int cnt = 2;
-    for (int c = 0; c < 2; ++c) {
-        id[c] = nodes[k].child[c];
-        for (int a = 0; a < 6; ++a) box[c][a] = nodes[k].box[6 * c + a];
-    }
-    while (cnt < 4) {
-        int pick = -1;
-        float best = -1.0f;
-        for (int j = 0; j < cnt; ++j) {
-            if (id[j] < 0) continue;
-            const float ar = half_area(box[j]);
-            if (ar > best) { best = ar; pick = j; }
-        }
-        if (pick < 0) break;
-        const BvhNode& m = nodes[id[pick]];
-        id[cnt] = m.child[1];
-        for (int a = 0; a < 6; ++a) box[cnt][a] = m.box[6 + a];
-        id[pick] = m.child[0];
-        for (int a = 0; a < 6; ++a) box[pick][a] = m.box[a];
-        ++cnt;
-    }
-    return cnt;
-}
-
-// The traversal's nodes.
+// BVH4 collapse.  Every internal BVH2 node k is turned into a BVH4 node stored at
+// index k, independently of the others: starting from k's two children, the internal
+// child with the largest box surface (ties: the lower slot) is replaced in its slot by
+// its first child and its second child is appended, until four slots are filled or
+// only leaves are left.  Traversal starts at node 0 and follows internal links, which
+// are BVH2 node indices and so name the BVH4 node built from that node; nodes not
+// reached that way are never read.  Runs after the refit: every box is final.  (trav_children
+// and trav_pack: pt_trav.hpp.)
 __global__ __launch_bounds__(256) void k_collapse4(const BvhNode* __restrict__ nodes, int ni,
                                                    TravNode* __restrict__ out) {
     const int k = (int)(blockIdx.x * 256u + threadIdx.x);
     if (k >= ni) return;
     int id[4];
     float box[4][6];
-    const int cnt = collapse4(nodes, k, id, box);
+    const int cnt = trav_children(nodes, k, id, box);
     out[k] = trav_pack(box, id, cnt);
-}
-
-// The same nodes with exact boxes (inspection).
-__global__ __launch_bounds__(256) void k_collapse4_exact(const BvhNode* __restrict__ nodes, int ni,
-                                                         Bvh4Node* __restrict__ out) {
-    const int k = (int)(blockIdx.x * 256u + threadIdx.x);
-    if (k >= ni) return;
-    int id[4];
-    float box[4][6];
-    const int cnt = collapse4(nodes, k, id, box);
-    Bvh4Node r;
-    const float inf = __builtin_inff();
-    for (int j = 0; j < 4; ++j) {
-        const bool used = j < cnt;
-        r.lox[j] = used ? box[j][0] : inf;
-        r.loy[j] = used ? box[j][1] : inf;
-        r.loz[j] = used ? box[j][2] : inf;
-        r.hix[j] = used ? box[j][3] : inf;
-        r.hiy[j] = used ? box[j][4] : inf;
-        r.hiz[j] = used ? box[j][5] : inf;
-        r.child[j] = used ? id[j] : 0;
-        r.pad[j] = 0;
-    }
-    out[k] = r;
 }
 
 }  // namespace
@@ -1227,11 +1172,6 @@ void launch_build_lbvh(const BuildArgs& a, hipStream_t s) {
         }
     }
     hipLaunchKernelGGL(k_collapse4, dim3((ni + 255) / 256), dim3(256), 0, s, a.nodes, ni, a.nodes4);
-}
-
-void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s) {
-    const int ni = n > 1 ? (int)n - 1 : 1;
-    hipLaunchKernelGGL(k_collapse4_exact, dim3((ni + 255) / 256), dim3(256), 0, s, nodes, ni, out);
 }
 
 uint32_t treelet_start_cap(uint32_t n) { return n / 6u + 1u; }

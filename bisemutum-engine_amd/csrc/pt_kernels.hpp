@@ -58,8 +58,6 @@ struct BuildArgs {
     uint32_t* tl_starts; // 1 + treelet_start_cap(num_tris) entries
 };
 void launch_build_lbvh(const BuildArgs& a, hipStream_t s);
-// BVH4 nodes with exact boxes of a built BVH2 (inspection): n triangles, max(n - 1, 1) nodes.
-void launch_collapse_exact(const BvhNode* nodes, uint32_t n, Bvh4Node* out, hipStream_t s);
 uint32_t bounds_words();
 uint32_t sort_words(uint32_t n);
 uint32_t treelet_start_cap(uint32_t n);

@@ -46,17 +46,6 @@ struct alignas(16) BvhNode {
 };
 static_assert(sizeof(BvhNode) == 64, "node record is 64 bytes");
 
-// BVH4 node with exact boxes (inspection; the traversal reads the TravNode made from the
-// same children): child k's box is (lox[k], loy[k], loz[k]) - (hix[k], hiy[k], hiz[k]);
-// child k is internal (BVH4 node index >= 0) or leaf j (stored as ~j).  An empty slot
-// has the box (+inf,+inf,+inf)-(+inf,+inf,+inf), which every slab test rejects.
-struct alignas(128) Bvh4Node {
-    float lox[4], loy[4], loz[4], hix[4], hiy[4], hiz[4];
-    int32_t child[4];
-    int32_t pad[4];
-};
-static_assert(sizeof(Bvh4Node) == 128, "BVH4 node record is 128 bytes");
-
 struct alignas(64) LeafGeo {
     float v[16];       // v0.xyz, e1.xyz, e2.xyz; v[9]: flag bits (kLeafNonOpaque); box lo.xyz, hi.xyz
 };

@@ -95,6 +95,37 @@ PT_HD TravNode trav_pack(const float (*box)[6], const int32_t* id, int n) {
     return r;
 }
 
+// The children of the traversal node made at node k of a BVH2 (whose nodes hold two child
+// links and boxes, lo xyz and hi xyz): k's children, of which the internal one with the largest
+// surface is replaced by its own two until there are four or only leaves.  Returns how many;
+// id: links, box: exact boxes.
+template <class Node>
+PT_HD int trav_children(const Node* nodes, int k, int32_t (&id)[4], float (&box)[4][6]) {
+    int cnt = 2;
+    for (int c = 0; c < 2; ++c) {
+        id[c] = nodes[k].child[c];
+        for (int a = 0; a < 6; ++a) box[c][a] = nodes[k].box[6 * c + a];
+    }
+    while (cnt < 4) {
+        int pick = -1;
+        float best = -1.0f;
+        for (int j = 0; j < cnt; ++j) {
+            if (id[j] < 0) continue;
+            const float dx = box[j][3] - box[j][0], dy = box[j][4] - box[j][1], dz = box[j][5] - box[j][2];
+            const float half = (dx * dy + dy * dz) + dz * dx;
+            if (half > best) { best = half; pick = j; }
+        }
+        if (pick < 0) break;
+        const Node& m = nodes[id[pick]];
+        id[cnt] = m.child[1];
+        for (int a = 0; a < 6; ++a) box[cnt][a] = m.box[6 + a];
+        id[pick] = m.child[0];
+        for (int a = 0; a < 6; ++a) box[pick][a] = m.box[a];
+        ++cnt;
+    }
+    return cnt;
+}
+
 // A ray as the visit test reads it: inverse direction, and per axis -(o inv) -/+ 4u |o inv|
 // (u = 2^-24) for the planes met first and last.
 //

@@ -695,11 +695,16 @@ bi_pt_status bi_pt_trace_occlusion(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays*
  * parents[max(n-1,1)+n] (internal nodes, then leaves; root -1), centroid_bounds[6]. */
 bi_pt_status bi_pt_debug_get_bvh(bi_pt_ctx* ctx, uint32_t* morton, uint32_t* order, int32_t* children,
                                  float* child_bounds, int32_t* parents, float* centroid_bounds);
-/* Copy the BVH4 traversal nodes built from the last LBVH: for each BVH2 internal node
+/* The BVH4 traversal nodes built from the last LBVH: for each BVH2 internal node
  * k (max(n-1,1) of them), child4[4k..4k+3] (internal: node index, leaf j as ~j, empty
- * slot 0) and box4[24k..24k+23] (lo.x[4], lo.y[4], lo.z[4], hi.x[4], hi.y[4], hi.z[4];
- * an empty slot holds +inf). */
+ * slot 0), copied from the nodes that the traversal reads, and box4[24k..24k+23] (lo.x[4],
+ * lo.y[4], lo.z[4], hi.x[4], hi.y[4], hi.z[4]; an empty slot holds +inf), the children's
+ * exact boxes, which those nodes hold as 8-bit planes. */
 bi_pt_status bi_pt_debug_get_bvh4(bi_pt_ctx* ctx, int32_t* child4, float* box4);
+/* The traversal nodes of the LBVH that stands now as they are, 64 B each (max(n-1,1) of them):
+ * per axis the frame's base, then scale (f32 x 3 each); six words of one byte per child (low and
+ * high plane of x, y, z); four child links. */
+bi_pt_status bi_pt_debug_get_trav_nodes(bi_pt_ctx* ctx, void* nodes64);
 uint32_t bi_pt_debug_num_tris(const bi_pt_ctx* ctx);
 /* Treelet rounds of the LBVH that stands now (0xffffffff: none is current). */
 uint32_t bi_pt_debug_built_rounds(const bi_pt_ctx* ctx);

@@ -19,6 +19,7 @@ import pytest
 
 import bi_pt
 import scenes
+from test_gpu_parity import check_trav_nodes
 
 pytestmark = pytest.mark.gpu
 
@@ -104,6 +105,7 @@ def test_batch_c2_trees_equal_oracle(oracle_lib):
         assert t.built_rounds() == r   # the tree that the batch built, not one rebuilt for inspection
         gc, gb = t.bvh4()
         assert np.array_equal(gc, oc) and np.array_equal(gb.view(np.uint32), ob.view(np.uint32)), (k, sc.num_tris, r)
+        check_trav_nodes(t.trav_nodes(), oc, ob)
     print(f"64 trees equal ({sum(1 for r in rounds if r)} restructured)", flush=True)
     b.close()
     for t in ts:

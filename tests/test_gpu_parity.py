@@ -1,12 +1,18 @@
 """GPU parity: the HIP pass (through the C ABI) against the CPU restatement.
 
-Bit-exact: Morton codes, sorted order, BVH topology and refit boxes, closest and
-any-hit traversal results, queue contents per segment, and per-pixel radiance
+Bit-exact: Morton codes, sorted order, BVH topology and refit boxes, the traversal's nodes,
+closest and any-hit traversal results, queue contents per segment, and per-pixel radiance
 sums.  The radiance comparison states its tolerance anyway (relative 1e-6 per
 channel on at least 99.9% of pixels), but the expected and observed result is
 exact equality, because the kernels and the restatement evaluate the same float
 operations in the same order.
 """
+import ctypes
+import functools
+import os
+import subprocess
+import tempfile
+
 import numpy as np
 import pytest
 
@@ -45,6 +51,37 @@ def compare_bvh4(gpu, ora):
     oc, ob = ora.bvh4()
     assert np.array_equal(gc, oc)
     assert np.array_equal(gb.view(np.uint32), ob.view(np.uint32))
+    check_trav_nodes(gpu.trav_nodes(), oc, ob)
+
+
+@functools.lru_cache(maxsize=None)
+def trav_pack_lib():
+    so = os.path.join(tempfile.mkdtemp(prefix="trav_pack"), "trav_pack.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-o", so,
+                    os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_wave", "trav_pack_host.cpp")], check=True)
+    return ctypes.CDLL(so)
+
+
+def check_trav_nodes(nodes, child, box):
+    """The nodes that the traversal reads (64 B: 8-bit planes in a frame), made on the GPU, against
+    the children and their exact boxes: the links, every child's planes around its box and at most
+    two quanta away, and the whole record equal to the packing on the CPU."""
+    n = len(child)
+    assert nodes.dtype.itemsize == 64 and np.array_equal(nodes["child"], child)
+    used = child != 0
+    box = box.reshape(n, 6, 4).astype(np.float64)
+    q = nodes["plane"].astype(np.float64)
+    for a in range(3):
+        base, scale = (nodes[k][:, a, None].astype(np.float64) for k in ("base", "scale"))
+        lo, hi = base + q[:, 2 * a] * scale, base + q[:, 2 * a + 1] * scale
+        # planes on the frame's edge, which need no slack, stand within the base's rounding
+        eps = np.abs(base) * 2.0 ** -23
+        assert np.all((lo <= box[:, a] + eps) & (lo >= box[:, a] - 2.0 * scale - eps), where=used)
+        assert np.all((hi >= box[:, 3 + a] - eps) & (hi <= box[:, 3 + a] + 2.0 * scale + eps), where=used)
+    want = np.zeros(n, nodes.dtype)
+    child, box32 = np.ascontiguousarray(child), np.ascontiguousarray(box.astype(np.float32))
+    trav_pack_lib().trav_pack_nodes(ctypes.c_int64(n), *(ctypes.c_void_p(x.ctypes.data) for x in (child, box32, want)))
+    assert nodes.tobytes() == want.tobytes()
 
 
 def test_bvh_bit_exact_c0(c0_gpu, c0_oracle):
