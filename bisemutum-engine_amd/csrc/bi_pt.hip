@@ -186,7 +186,9 @@ namespace {
 
 // A query's launch: the context's scene and the caller's rays.  It needs no scratch (each
 // wavefront has its own range of rays), so queries of one context on several streams share
-// nothing but the scene.
+// nothing but the scene and its LBVH: they may overlap once it is complete.  (A query that
+// builds the LBVH enqueues the build on its own stream; the caller orders it before queries
+// on others.)
 QueryArgs query_args(bi_pt_ctx* ctx, uint32_t n, const bi_pt_rays* rays, float tmax) {
     QueryArgs a{};
     a.bvh = bvh_view(ctx);

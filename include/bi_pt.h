@@ -661,8 +661,9 @@ bi_pt_status bi_pt_nrc_debug_samples(bi_pt_nrc* nrc, float* records, float* targ
  * Rays: n origins and directions as six device arrays (directions need not be unit
  * length; t is in units of the direction), TMin = 0.001 as in the reference's passes, one
  * TMax for all rays (0.001 < tmax <= 1.7e38).  The context's LBVH is built on `stream` if
- * the scene changed since the last build (order queries after other streams' renders of
- * the same context).  Closest hits are those of the path tracer (independent of the tree
+ * the scene changed since the last build: order a query after other streams' renders of the
+ * same context, and after another stream's query that builds.  Queries of a context whose
+ * LBVH is complete share nothing else and may overlap on several streams.  Closest hits are those of the path tracer (independent of the tree
  * and of traversal order).  Errors of the traversal (stack bound) are reported by
  * bi_pt_get_stats like a render's.  Stream-ordered, no host synchronisation. */
 typedef struct bi_pt_rays {
