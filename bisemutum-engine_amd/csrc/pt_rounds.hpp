@@ -22,20 +22,30 @@ inline uint32_t kept_rounds(uint64_t paths, uint32_t tris, uint32_t configured) 
 }
 
 // Rounds that a call's own paths repay, at most `configured`: for trees that no later call
-// traces.  Round k runs when the call traces at least (2^21 + 32 n) (1 + k (k - 1) / 3) paths
+// traces.  Round k runs when the call traces at least (2^21 + 20 n) (1 + k (k - 1) / 3) paths
 // of the scene's n triangles (paths of fewer than four segments count in proportion): the
 // first round saves most, the third a tenth of it, and each costs the same.  Frame with
-// 0 / 1 / 2 / 3 rounds, build included:
-//   atrium (262k), 8 segments, 2.1 M paths   5.52 /  5.55 /  5.85 /  6.21 ms
-//                              4.1 M         8.88 /  8.40 /  8.62 /  8.91
-//                             16.6 M        28.68 / 25.21 / 24.91 / 25.10
-//                             33.2 M        55.2  / 47.7  / 46.8  / 46.6
-//   rooms of 20k, 6 segments,  1.8 M         3.01 /  3.05 /  3.27 /  3.49
-//                              7.4 M         7.49 /  7.03 /  7.14 /  7.32
-//   250k                       7.4 M         6.86 /  7.08 /  7.64 /  8.11
-//   900k                       8.3 M        11.31 / 13.34 / 14.85 / 16.38
+// 0 / 1 / 2 / 3 rounds, build included, ms:
+//   atrium (262k), 8 segments, 2.1 M paths   4.97 /  4.97 /  5.26 /  5.60
+//                              4.1 M         8.15 /  7.66 /  7.89 /  8.17
+//                              8.3 M        14.55 / 13.16 / 13.21 / 13.43
+//                             16.6 M        27.17 / 23.87 / 23.58 / 23.66
+//                             33.2 M        52.58 / 45.43 / 44.49 / 44.29
+//   rooms of 20k, 6 segments,  1.8 M         2.75 /  2.78 /  2.99 /  3.20
+//                              3.7 M         4.13 /  4.01 /  4.20 /  4.39
+//                              7.4 M         6.88 /  6.42 /  6.57 /  6.73
+//   100k                       3.7 M         3.27 /  3.41 /  3.73 /  4.00
+//                              7.4 M         5.10 /  5.05 /  5.33 /  5.61
+//                             16.6 M         9.56 /  9.09 /  9.31 /  9.60
+//   250k                       7.4 M         6.75 /  6.91 /  7.49 /  7.94
+//                             16.6 M        16.34 / 15.28 / 15.69 / 16.14
+//   900k                       7.4 M         8.23 / 10.47 / 12.27 / 13.72
+//                             16.6 M        16.44 / 17.64 / 19.16 / 20.83
+// A path of the atrium saves about twice what a room's does, so the line lies between: at
+// 32 n the atrium's 8.3 M paths went without (8% slower than three rounds), below 16 n the
+// 900k room's 16.6 M got one (7% slower than none).
 inline uint32_t paid_rounds(uint64_t full_paths, uint32_t tris, uint32_t configured) {
-    const uint64_t first = (1ull << 21) + 32ull * tris;
+    const uint64_t first = (1ull << 21) + 20ull * tris;
     uint32_t k = 0;
     while (k < configured && 3ull * full_paths >= first * (3ull + (uint64_t)k * (k + 1ull))) ++k;
     return k;

@@ -42,7 +42,7 @@ def test_kept_trees(rounds, use):
 def test_trees_of_one_call(rounds):
     cases, want = [], []
     for n in (0, 1, 20504, 262144, 900000, (1 << 29) - 1):
-        first = (1 << 21) + 32 * n
+        first = (1 << 21) + 20 * n
         for k in (1, 2, 3, 4, 16):   # round k runs from first (1 + k (k - 1) / 3) paths on
             need = -(-first * (3 + k * (k - 1)) // 3)
             for paths, r in ((need - 1, k - 1), (need, k)):
@@ -50,6 +50,8 @@ def test_trees_of_one_call(rounds):
                     cases.append((1, 0, 0, paths, paths, n, configured))
                     want.append(min(r, configured))
     assert rounds(cases) == want
+    # the 262k-triangle atrium's frames of 1, 4, 8 and 16 samples at 1080p
+    assert rounds([(1, 0, 0, 2073600 * s, 2073600 * s, 262144, 3) for s in (1, 4, 8, 16)]) == [0, 1, 2, 3]
     # never more rounds than a kept tree of the same call
     kept = rounds([(1, 1, 0) + c[3:] for c in cases])
     assert all(a <= b for a, b in zip(want, kept))
