@@ -4,7 +4,7 @@
 //   scene      mesh pool (float xyz positions/normals, uint32 indices; texture
 //              coordinates and tangents where materials sample textures), instance
 //              records, material table (128 B each), texture records + texel pool + sRGB
-//              table, sky texels (equirect or six cube faces) + importance and guide tables
+//              table, sky texels (equirect or six cube faces) + importance and alias tables
 //   per frame  world triangles (36 B) + normals (36 B) in instance order, Morton keys,
 //              sorted order, BVH2 nodes (64 B: both child boxes + child links; the build
 //              structure), BVH4 traversal nodes (64 B: four child boxes as 8-bit planes in

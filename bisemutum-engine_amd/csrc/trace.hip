@@ -18,13 +18,14 @@
 // nearest hit internal child entered and the other hit internal children pushed
 // (ascending slot order).
 //
-// What bounds it (atrium, 16 spp at 1080p, depth 8, SQ and TCP counters): extension rays
-// issue 1.05 VALU instructions per clock and CU and look up 0.83 cache lines per clock and
-// CU in the vector cache, whose limit is one; with 128-B nodes of FP32 planes it was the
-// lookups alone (seven 16-B loads a node).  Closest hit 24.4 -> 17.5 ms, shadow 16.5 ->
-// 12.9 ms per frame from 64-B nodes (4 loads), near and far planes by the ray's signs and
-// fused multiply-adds, winners' barycentrics kept in LDS instead of a second triangle test,
-// and a step whose masks stay in scalar registers (215 -> 150 VALU instructions).
+// What bounds it (atrium, 16 spp at 1080p, depth 8, SQ and TCP counters): VALU issue first, the
+// vector cache close behind.  Extension rays issue 1.02 VALU instructions per clock and CU and
+// look up 0.88 cache lines per clock and CU in the vector cache, whose limit is about one
+// (shadow rays 0.85 and 0.79); with 128-B nodes of FP32 planes it was the lookups (seven 16-B
+// loads a node).  Closest hit 24.4 -> 17.5 ms, shadow 16.5 -> 12.9 ms per frame from 64-B
+// nodes (4 loads), near and far planes by the ray's signs and fused multiply-adds, winners'
+// barycentrics kept in LDS instead of a second triangle test, and a step whose masks stay in
+// scalar registers; per extension ray 94 -> 78 wavefront VALU instructions.
 #include <algorithm>
 
 #include "pt_kernels.hpp"
@@ -823,7 +824,7 @@ void shadow_lb(const ShadowArgs& a, uint32_t capacity, hipStream_t s) {
     hipLaunchKernelGGL((k_trace_shadow<AH, L, B>), dim3(groups), dim3(B), 0, s, a);
 }
 
-// Block shapes: 128, 256 (default) or 512 threads; LDS stack depths 8, 12, 16 (default), 24, 32.
+// Block shapes: 128, 256 (default) or 512 threads; LDS stack depths 8, 12 (default), 16, 24, 32.
 template <bool P, bool AH, int B>
 void closest_b(const TraceArgs& a, uint32_t capacity, uint32_t lds, hipStream_t s) {
     if (lds <= 8) closest_lb<P, AH, 8, B>(a, capacity, s);
