@@ -15,8 +15,8 @@ struct TreeUse {
 };
 
 // Rounds of a tree that later calls trace too (renders that keep it, ray queries, the
-// server): all configured ones, unless the call itself is so small that the tree is likely
-// a preview's (a round costs ~0.1-0.5 ms).
+// server): all configured ones, unless the call itself is so small that the tree is likely a
+// preview's (a round costs 0.2 ms for 20k triangles, 0.4 to 0.8 ms for 260k, 1.4 to 3 ms for 900k).
 inline uint32_t kept_rounds(uint64_t paths, uint32_t tris, uint32_t configured) {
     return paths >= std::max<uint64_t>(4ull * tris, 1ull << 20) ? configured : 0u;
 }
